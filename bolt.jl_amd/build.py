@@ -17,7 +17,13 @@ LIB = os.path.join(HERE, "libbolt_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["bolt_hip.hip", "host_tables.cpp", "host_api.cpp"]
+# The solver's one loop spans thousands of instructions: constants that machine
+# LICM hoists to its top stay live across it and spill scalar registers.
+SOLVE = ["-mllvm", "-disable-machine-licm"]
+# (object, source, extra flags); the solver is compiled once per scan shape
+SOURCES = [("bolt_hip.o", "bolt_hip.hip", []), ("boltsolve.o", "boltsolve.hip", SOLVE)] + \
+          [(f"solve_sr{sr}.o", "solve.hip", SOLVE + [f"-DSOLVE_SR={sr}"]) for sr in (6, 7, 8)] + \
+          [("host_tables.o", "host_tables.cpp", []), ("host_api.o", "host_api.cpp", [])]
 
 
 def hip_flags():
@@ -31,12 +37,12 @@ def build(verbose=False, nanfill=False):
     """libbolt_hip.so; nanfill=True builds the debug variant
     libbolt_hip_nanfill.so, whose solver starts every k-mode from a workspace
     filled with NaNs (load it with BOLT_HIP_LIB=<path>)."""
-    objs = []
+    objs, jobs = [], []
     tmp = os.path.join(HERE, "_build_nanfill" if nanfill else "_build")
     os.makedirs(tmp, exist_ok=True)
-    for src in SOURCES:
-        obj = os.path.join(tmp, src + ".o")
-        cmd = [HIPCC] + hip_flags() + (["-DBOLT_DEBUG_NANFILL"] if nanfill else []) + \
+    for name, src, extra in SOURCES:
+        obj = os.path.join(tmp, name)
+        cmd = [HIPCC] + hip_flags() + extra + (["-DBOLT_DEBUG_NANFILL"] if nanfill else []) + \
               ["-c", os.path.join(CSRC, src), "-o", obj]
         if src.endswith(".cpp"):
             cmd = [HIPCC, "-x", "c++"] + [f for f in hip_flags() if not f.startswith("--offload-arch")
@@ -45,8 +51,11 @@ def build(verbose=False, nanfill=False):
                   ["-c", os.path.join(CSRC, src), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)
-        subprocess.check_call(cmd)
+        jobs.append((cmd, subprocess.Popen(cmd)))
         objs.append(obj)
+    for cmd, job in jobs:
+        if job.wait():
+            raise subprocess.CalledProcessError(job.returncode, cmd)
     lib = LIB.replace(".so", "_nanfill.so") if nanfill else LIB
     out_tmp = lib + ".tmp"
     cmd = [HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", out_tmp] + objs

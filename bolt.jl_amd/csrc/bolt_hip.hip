@@ -43,2209 +43,7 @@ int set_error(int code, const std::string& msg);
 }
 using bolt::set_error;
 
-#define WAVE 64
-#define NWAVE 4                // wavefronts per k-mode in the solver
-#define NTHR (NWAVE * WAVE)
-#define MAXSEG 64              // independent row segments of the banded solve
-
-// thread coordinates in the workgroup that owns one k-mode
-struct Thr {
-    int tid, nt, lane, wv;
-};
-__device__ inline Thr thr_self() {
-    Thr t;
-    t.tid = threadIdx.x;
-    t.nt = blockDim.x;
-    t.lane = t.tid & (WAVE - 1);
-    t.wv = t.tid / WAVE;
-    return t;
-}
-
-// ---------------------------------------------------------------- device data
-struct CosmoDev {
-    double h, Or, Ob, Oc, A, ns, Yp, Nnu, mnu;
-    double H0, eta0, rho_crit, Onu;  // Onu = 7*(2/3)*N_ν/8*(4/11)^(4/3)*Ω_r
-    double x0, x1, dx, idx;  // idx = 1/dx
-    int nx, nq;
-    const double* coef;    // [16][nx+2]
-    const double* qv;      // [nq] q_i
-    const double* df0;     // [nq] dlnf0dlnq(q_i)
-    const double* base;    // [nq] 4π q_i² f0(q_i)/dxdq(q_i) w_i
-    const double* thbase;  // [nq] 4π q_i³ f0(q_i)/dxdq(q_i) w_i
-    double Pprim_A, Pprim_n;
-    double Om_nu_nr;       // massive-ν Ω used by plin (spectra.jl:182-187)
-};
-
-struct CfgDev {
-    int ng, nn, nm, nq, n;
-    double reltol, abstol;
-    int max_steps;
-    int flags;  // bolt_hier_cfg.flags: BOLT_CFG_FP32_SOLVE and the refinement count
-};
-
-struct ModeDesc {
-    double k;
-    int cosmo, cfg, out;
-    int pad;
-};
-
-// geometry of the chain-ordered state
-struct Geo {
-    int ng, nn, nm, nq, n;
-    int cB, cC, cM, cD, cE, nch;
-};
-
-__device__ __host__ inline Geo make_geo(const CfgDev& c) {
-    Geo g;
-    g.ng = c.ng; g.nn = c.nn; g.nm = c.nm; g.nq = c.nq; g.n = c.n;
-    g.cB = g.ng + 3;                 // chain A: δb, vb, Θ0..Θℓᵧ
-    g.cC = g.cB + g.ng + 1;          // chain B: Θᵖ0..Θᵖℓᵧ
-    g.cM = g.cC + g.nn + 1;          // chain C: 𝒩0..𝒩ℓ_ν
-    g.cD = g.cM + g.nq * (g.nm + 1); // chains M_i: ℳ0,i..ℳℓ_mν,i
-    g.cE = g.cD + 2;                 // chain D: δ, v ; chain E: Φ
-    g.nch = 3 + g.nq + 2;
-    return g;
-}
-
-// chain-order index -> Bolt's state index (perturbations.jl:114-125)
-__device__ __host__ inline int chain_to_state(const Geo& g, int c) {
-    int iN = 2 * (g.ng + 1), iM = iN + g.nn + 1, iPhi = iM + (g.nm + 1) * g.nq;
-    if (c < g.cB) {
-        if (c == 0) return iPhi + 3;  // δ_b
-        if (c == 1) return iPhi + 4;  // v_b
-        return c - 2;                 // Θℓ
-    }
-    if (c < g.cC) return g.ng + 1 + (c - g.cB);
-    if (c < g.cM) return iN + (c - g.cC);
-    if (c < g.cD) {
-        int t = c - g.cM, qi = t / (g.nm + 1), l = t % (g.nm + 1);
-        return iM + l * g.nq + qi;
-    }
-    if (c == g.cD) return iPhi + 1;  // δ
-    if (c == g.cD + 1) return iPhi + 2;  // v
-    return iPhi;                          // Φ
-}
-
-__device__ inline void chain_range(const Geo& g, int ch, int& c0, int& m) {
-    if (ch == 0) { c0 = 0; m = g.ng + 3; }
-    else if (ch == 1) { c0 = g.cB; m = g.ng + 1; }
-    else if (ch == 2) { c0 = g.cC; m = g.nn + 1; }
-    else if (ch < 3 + g.nq) { c0 = g.cM + (ch - 3) * (g.nm + 1); m = g.nm + 1; }
-    else if (ch == 3 + g.nq) { c0 = g.cD; m = 2; }
-    else { c0 = g.cE; m = 1; }
-}
-
-__device__ inline double node_x(const CosmoDev& C, int j) { return (C.x0 * (C.nx - 1 - j) + C.x1 * j) / (C.nx - 1); }
-
-// uniform cubic B-spline (src/util.jl:11-13)
-__device__ inline double spl(const CosmoDev& C, int tab, double x, int deriv = 0) {
-    double t = (x - C.x0) * C.idx;
-    int i = (int)floor(t);
-    i = i < 0 ? 0 : (i > C.nx - 2 ? C.nx - 2 : i);
-    double s = t - i, r = 1.0 - s;
-    const double* q = C.coef + (size_t)tab * (C.nx + 2) + i;
-    constexpr double sixth = 1.0 / 6.0, two3 = 2.0 / 3.0;
-    if (deriv == 0)
-        return (r * r * r) * sixth * q[0] + (two3 - s * s + 0.5 * s * s * s) * q[1] +
-               (two3 - r * r + 0.5 * r * r * r) * q[2] + (s * s * s) * sixth * q[3];
-    if (deriv == 1)
-        return (-0.5 * r * r * q[0] + (-2.0 * s + 1.5 * s * s) * q[1] + (2.0 * r - 1.5 * r * r) * q[2] +
-                0.5 * s * s * q[3]) * C.idx;
-    return (r * q[0] + (-2.0 + 3.0 * s) * q[1] + (-2.0 + 3.0 * r) * q[2] + s * q[3]) * (C.idx * C.idx);
-}
-
-// ------------------------------------------------------------ reductions
-// 64-bit DPP move within a row of 16 lanes; lanes whose source is outside the
-// row read 0
-template <int CTRL>
-__device__ inline double dpp64(double v) {
-    int lo = __double2loint(v), hi = __double2hiint(v);
-    lo = __builtin_amdgcn_update_dpp(0, lo, CTRL, 0xF, 0xF, true);
-    hi = __builtin_amdgcn_update_dpp(0, hi, CTRL, 0xF, 0xF, true);
-    return __hiloint2double(hi, lo);
-}
-__device__ inline double readlane64(double v, int l) {
-    int lo = __builtin_amdgcn_readlane(__double2loint(v), l);
-    int hi = __builtin_amdgcn_readlane(__double2hiint(v), l);
-    return __hiloint2double(hi, lo);
-}
-// 32-bit counterparts, and an overload set the scans are written against, so
-// that one scan serves FP64 and FP32 substitutions
-template <int CTRL>
-__device__ inline float dpp32(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
-}
-__device__ inline float readlane32(float v, int l) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l)); }
-template <int CTRL> __device__ inline double dppz(double v) { return dpp64<CTRL>(v); }
-template <int CTRL> __device__ inline float dppz(float v) { return dpp32<CTRL>(v); }
-__device__ inline double rdlane(double v, int l) { return readlane64(v, l); }
-__device__ inline float rdlane(float v, int l) { return readlane32(v, l); }
-__device__ inline double fmaT(double a, double b, double c) { return __builtin_fma(a, b, c); }
-__device__ inline float fmaT(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
-
-// Σ over the wavefront, the same value (same rounding) in every lane: an
-// inclusive scan inside each row of 16 (row_shr 1, 2, 4, 8), then the four row
-// totals added in a fixed order.
-__device__ inline double wave_sum(double v) {
-    v += dpp64<0x111>(v);
-    v += dpp64<0x112>(v);
-    v += dpp64<0x114>(v);
-    v += dpp64<0x118>(v);
-    return ((readlane64(v, 15) + readlane64(v, 31)) + readlane64(v, 47)) + readlane64(v, 63);
-}
-// max over the wavefront of non-negative values, the same in every lane
-__device__ inline double wave_max(double v) {
-    v = fmax(v, dpp64<0x111>(v));
-    v = fmax(v, dpp64<0x112>(v));
-    v = fmax(v, dpp64<0x114>(v));
-    v = fmax(v, dpp64<0x118>(v));
-    return fmax(fmax(readlane64(v, 15), readlane64(v, 31)), fmax(readlane64(v, 47), readlane64(v, 63)));
-}
-// N sums at once over values held by lanes 0..15 only (other lanes' values are
-// ignored): interleaved scans inside row 0, the totals read from lane 15; the
-// same value (same rounding) in every lane
-template <int N>
-__device__ inline void row0_sums(double (&a)[N]) {
-#pragma unroll
-    for (int i = 0; i < N; ++i) a[i] += dpp64<0x111>(a[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) a[i] += dpp64<0x112>(a[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) a[i] += dpp64<0x114>(a[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) a[i] += dpp64<0x118>(a[i]);
-#pragma unroll
-    for (int i = 0; i < N; ++i) a[i] = readlane64(a[i], 15);
-}
-
-// 1/d from v_rcp_f64 refined twice (pivots here are O(1) to O(1e12): no
-// denormal or overflow range is involved).  With e = 1 - d·r₀,
-// r₁ = r₀(1 + e) has error e² and r₂ = r₁(1 + e²) error e⁴; e² is formed
-// beside r₁, so the dependent chain is rcp, fma, fma, fma.
-__device__ inline double rcp(double d) {
-    const double r = __builtin_amdgcn_rcp(d);
-    const double e = fma(-d, r, 1.0);
-    const double r1 = fma(r, e, r);
-    const double e2 = e * e;
-    return fma(r1, e2, r1);
-}
-
-// 1/d refined once (relative error e² ≈ 2e-15 from v_rcp_f64's e ≈ 5e-8): the
-// pivots of the banded LU, where the pivot recurrence is the critical path
-__device__ inline double rcp_piv(double d) {
-    const double r = __builtin_amdgcn_rcp(d);
-    return fma(r, fma(-d, r, 1.0), r);
-}
-// FP32 factors: v_rcp_f32 is within one ulp
-__device__ inline float rcp_piv(float d) { return __builtin_amdgcn_rcpf(d); }
-
-// largest hierarchy cut-off accepted (row descriptors pack ℓ in 11 bits)
-#define LTAB 512
-
-// x-dependent coefficients of hierarchy! (perturbations.jl:163-172), with the
-// divisions by per-mode and per-x constants taken once here: three reciprocals
-// per evaluation point instead of one division per use
-struct XC {
-    double x, a, Hc, eta, tp, tpp, csb2, kH, R, c12, gg, k23, iHeta;
-    double fs2;                         // Ψ:  c12 / (4 ρ_crit)        (multiplies Σ σ)
-    double fp0, fp1, fp2, fp3, fp4;     // Φ′: gg Ω_c/a, gg Ω_b/a, gg 4Ω_r/a², gg 4Ω_ν/a², gg/(ρ_crit a²)
-    bool rsa;
-};
-
-__device__ inline XC make_xc(const CosmoDev& C, double k, double x) {
-    XC X;
-    X.x = x;
-    X.a = exp(x);
-    X.Hc = spl(C, BOLT_T_HC, x);
-    X.eta = spl(C, BOLT_T_ETA, x);
-    X.tp = spl(C, BOLT_T_TAU_P, x);
-    X.tpp = spl(C, BOLT_T_TAU_PP, x);
-    X.csb2 = spl(C, BOLT_T_CSB2, x);
-    // a, ℋ, η are O(1e-9)..O(1e4): the refined reciprocal is within an ulp or two
-    const double ia = rcp(X.a), ia2 = ia * ia, iHc = rcp(X.Hc), iHc2 = iHc * iHc, ik2 = 1.0 / (k * k);
-    const double H02 = C.H0 * C.H0, irho = 1.0 / C.rho_crit;
-    X.kH = k * iHc;
-    X.R = (4.0 * C.Or / (3.0 * C.Ob)) * ia;
-    X.c12 = (12.0 * H02) * ik2 * ia2;
-    X.gg = (0.5 * H02) * iHc2;
-    X.k23 = (k * k / 3.0) * iHc2;
-    X.iHeta = iHc * rcp(X.eta);
-    X.fs2 = X.c12 * (0.25 * irho);
-    X.fp0 = X.gg * C.Oc * ia;
-    X.fp1 = X.gg * C.Ob * ia;
-    X.fp2 = X.gg * (4.0 * C.Or) * ia2;
-    X.fp3 = X.gg * (4.0 * C.Onu) * ia2;
-    X.fp4 = X.gg * irho * ia2;
-    X.rsa = (k * X.eta > 240.0) && (-X.tp * X.Hc / X.eta > 100.0);  // perturbations.jl:216
-    return X;
-}
-
-// q-quantities at one x: (q/ϵ, ϵ/q·dlnf₀/dlnq, 4πq²f₀w·q²/ϵ, 4πq²f₀w·ϵ) per bin
-struct QSet {
-    const double* qe;
-    const double* eqdf;
-    const double* sw;
-    const double* rw;
-};
-
-// The x-dependent scalars every row coefficient is built from, one table per
-// x point: kH = k/ℋ, τ′, 1/(ℋη), τ′R, kH·c_s², 1, the RSA factor of the
-// photon/ν rows (0 when RSA is on), then kH·q_i/ε_i and
-// kH·(ε_i/q_i)·dlnf₀/dlnq (nq each)
-enum { K_KH = 0, K_TP, K_IHETA, K_TPR, K_KHCS, K_ONE, K_RSA, K_Q0 };
-
-// the LU of W = I - hγL at one stage point: l1 <- multipliers, d <- 1/pivot,
-// u1 <- upper entries; the second band lives only in the first block of the
-// first segment (rows 0..CB-1), kept in l2c/u2c
-template <class T>
-struct BandsT {
-    T* l1;
-    T* d;
-    T* u1;
-    T* l2c;
-    T* u2c;
-};
-using Bands = BandsT<double>;
-
-#define CB 8      // rows per block of the banded sweeps
-// rows per lane of the substitution scans (64·SR rows per pass): a template
-// parameter of the solver, SR_MIN..SR_MAX, picked per hierarchy size by the
-// autotuner (SR_DEFAULT until tuned).  Lane strides of 5 or 7 doubles spread a
-// wavefront's 8-byte LDS accesses over all banks, 6 over half of them; 8 covers
-// n = 473 in one pass.
-#define SR_MIN 5
-#define SR_MAX 8
-// the shapes the solver launches and the autotuner scans.  Five rows per lane
-// (two scan passes at n = 323) is not launched: in the build that added the
-// tangent-linear solve its results left the oracle's trajectory (3499 against
-// 2040 accepted steps on the massive-ν cosmology, varying from run to run),
-// while the debug build that fills each mode's workspace with NaN first gave
-// the oracle's; the cause was not found.  Six and seven rows also take two
-// passes at n = 473 and match the oracle.
-#define SR_RUN_MIN 6
-#define SR_DEFAULT 6
-#define NXC 24    // doubles per stored XC
-
-// LDS workspace of one k-mode.  Vectors of n doubles: u, f, u_{n+1}, f_{n+1}, ψ,
-// w, Z₀..Z₅, the border columns c_S, c_P, c_Π, the row recipes (six
-// coefficient vectors), and the LU of W at the five implicit stage points (3
-// vectors each).  Then the q arrays (mode constants, the current x, the five
-// stage points), the compact second bands, the five stage points' coefficients,
-// the six scalar tables (five stage points and the current x), cross-wavefront
-// partial sums, and the integer tables (row descriptors, recipe kinds,
-// segments).  Every pointer is base + offset arithmetic.
-struct WS {
-    double* b;
-    int n, nq;
-    __host__ __device__ double* u() const { return b; }
-    __host__ __device__ double* f() const { return b + n; }
-    __host__ __device__ double* un() const { return b + 2 * n; }
-    __host__ __device__ double* fn() const { return b + 3 * n; }
-    __host__ __device__ double* arg() const { return b + 4 * n; }
-    __host__ __device__ double* w() const { return b + 5 * n; }
-    __host__ __device__ double* Z(int j) const { return b + (6 + j) * n; }
-    __host__ __device__ double* cS() const { return b + 12 * n; }
-    __host__ __device__ double* cP() const { return b + 13 * n; }
-    __host__ __device__ double* cPi() const { return b + 14 * n; }
-    __host__ __device__ double* rcp_(int j) const { return b + (15 + j) * n; }  // recipe vector j (RC_*)
-    __host__ __device__ Bands bands(int s) const {
-        Bands B;
-        B.l1 = b + (21 + 3 * s) * n; B.d = b + (22 + 3 * s) * n; B.u1 = b + (23 + 3 * s) * n;
-        B.l2c = b + 36 * n + 27 * nq + 2 * CB * s;
-        B.u2c = B.l2c + CB;
-        return B;
-    }
-    // FP32 solve mode: the five stage points' factors as floats in the first
-    // half of the bands' region (second bands in the first half of their
-    // double slots), and a copy of the stage right-hand side after them
-    __host__ __device__ BandsT<float> bandsF(int s) const {
-        BandsT<float> B;
-        float* f = (float*)(b + 21 * n);
-        B.l1 = f + 3 * s * n; B.d = f + (3 * s + 1) * n; B.u1 = f + (3 * s + 2) * n;
-        B.l2c = (float*)(b + 36 * n + 27 * nq + 2 * CB * s);
-        B.u2c = B.l2c + CB;
-        return B;
-    }
-    __host__ __device__ double* rvec() const { return b + 21 * n + (15 * n + 1) / 2; }
-    template <class T> __host__ __device__ BandsT<T> bandsT(int s) const;
-    __host__ __device__ double* q() const { return b + 36 * n; }
-    __host__ __device__ double* df0() const { return b + 36 * n + nq; }
-    __host__ __device__ double* base() const { return b + 36 * n + 2 * nq; }
-    __host__ __device__ double* qe() const { return b + 36 * n + 3 * nq; }
-    __host__ __device__ double* eqdf() const { return b + 36 * n + 4 * nq; }
-    __host__ __device__ double* sw() const { return b + 36 * n + 5 * nq; }
-    __host__ __device__ double* rw() const { return b + 36 * n + 6 * nq; }
-    __host__ __device__ double* qst_base(int s) const { return b + 36 * n + (7 + 4 * s) * nq; }  // qe, eqdf, sw, rw
-    __host__ __device__ QSet qcur() const { QSet Q; Q.qe = qe(); Q.eqdf = eqdf(); Q.sw = sw(); Q.rw = rw(); return Q; }
-    __host__ __device__ QSet qst(int s) const {
-        const double* p = qst_base(s);
-        QSet Q; Q.qe = p; Q.eqdf = p + nq; Q.sw = p + 2 * nq; Q.rw = p + 3 * nq;
-        return Q;
-    }
-    __host__ __device__ double* xcs(int s) const { return b + 36 * n + 27 * nq + 10 * CB + NXC * s; }
-    // scalar table of stage point s (s < 5) or of the current x (s = 5)
-    __host__ __device__ double* ktab(int s) const { return b + 36 * n + 27 * nq + 10 * CB + 5 * NXC + (K_Q0 + 2 * nq) * s; }
-    __host__ __device__ double* kcur() const { return ktab(5); }
-    // [24]: border functionals 0..11, the refinement's 12..14, the dump slot 15,
-    // the refinement's per-wavefront convergence maxima 16..19 (20..23 spare)
-    __host__ __device__ double* red() const { return ktab(6); }
-    __host__ __device__ double* dump() const { return red() + 15; }  // store slot nobody reads
-    __host__ __device__ int* desc() const { return (int*)(red() + 24); }
-    __host__ __device__ int* kinds() const { return desc() + n; }
-    __host__ __device__ int* seg() const { return desc() + 2 * n; }          // [MAXSEG][2]: c0, m
-    __host__ __device__ int* misc() const { return seg() + 2 * MAXSEG; }     // nseg
-};
-
-template <> __host__ __device__ inline BandsT<double> WS::bandsT<double>(int s) const { return bands(s); }
-template <> __host__ __device__ inline BandsT<float> WS::bandsT<float>(int s) const { return bandsF(s); }
-
-__host__ __device__ inline void ws_bind(WS& W, double* lds, int n, int nq) {
-    W.b = lds;
-    W.n = n;
-    W.nq = nq;
-}
-__host__ __device__ inline size_t ws_bytes(int n, int nq) {
-    return sizeof(double) * ((size_t)36 * n + 27 * nq + 10 * CB + 5 * NXC + 6 * (K_Q0 + 2 * nq) + 24) +
-           sizeof(int) * (size_t)(2 * n + 2 * MAXSEG + 4) + sizeof(double) * WAVE * SR_MAX;  // scan read padding
-}
-
-__device__ inline void store_xc(double* p, const XC& X) {
-    p[0] = X.x; p[1] = X.a; p[2] = X.Hc; p[3] = X.eta; p[4] = X.tp; p[5] = X.tpp; p[6] = X.csb2; p[7] = X.kH;
-    p[8] = X.R; p[9] = X.c12; p[10] = X.gg; p[11] = X.k23; p[12] = X.iHeta; p[13] = X.fs2; p[14] = X.fp0;
-    p[15] = X.fp1; p[16] = X.fp2; p[17] = X.fp3; p[18] = X.fp4; p[19] = X.rsa ? 1.0 : 0.0;
-}
-__device__ inline XC load_xc(const double* p) {
-    XC X;
-    X.x = p[0]; X.a = p[1]; X.Hc = p[2]; X.eta = p[3]; X.tp = p[4]; X.tpp = p[5]; X.csb2 = p[6]; X.kH = p[7];
-    X.R = p[8]; X.c12 = p[9]; X.gg = p[10]; X.k23 = p[11]; X.iHeta = p[12]; X.fs2 = p[13]; X.fp0 = p[14];
-    X.fp1 = p[15]; X.fp2 = p[16]; X.fp3 = p[17]; X.fp4 = p[18]; X.rsa = p[19] != 0.0;
-    return X;
-}
-
-// row types of the chain-ordered state
-enum {
-    R_DB = 0, R_VB, R_T0, R_T1, R_TL, R_TN, R_P0, R_PL, R_PN, R_N0, R_N1, R_NL, R_NN,
-    R_M0, R_M1, R_ML, R_MN, R_DEL, R_V, R_PHI
-};
-__device__ __host__ inline int pack_desc(int type, int l, int qi) { return type | (l << 5) | (qi << 16); }
-
-__device__ __host__ inline int row_desc(const Geo& G, int c) {
-    if (c < G.cB) {
-        if (c == 0) return pack_desc(R_DB, 0, 0);
-        if (c == 1) return pack_desc(R_VB, 0, 0);
-        int l = c - 2;
-        return pack_desc(l == 0 ? R_T0 : l == 1 ? R_T1 : l < G.ng ? R_TL : R_TN, l, 0);
-    }
-    if (c < G.cC) {
-        int l = c - G.cB;
-        return pack_desc(l == 0 ? R_P0 : l < G.ng ? R_PL : R_PN, l, 0);
-    }
-    if (c < G.cM) {
-        int l = c - G.cC;
-        return pack_desc(l == 0 ? R_N0 : l == 1 ? R_N1 : l < G.nn ? R_NL : R_NN, l, 0);
-    }
-    if (c < G.cD) {
-        int t = c - G.cM, qi = t / (G.nm + 1), l = t % (G.nm + 1);
-        return pack_desc(l == 0 ? R_M0 : l == 1 ? R_M1 : l < G.nm ? R_ML : R_MN, l, qi);
-    }
-    if (c == G.cD) return pack_desc(R_DEL, 0, 0);
-    if (c == G.cD + 1) return pack_desc(R_V, 0, 0);
-    return pack_desc(R_PHI, 0, 0);
-}
-
-// Row recipes (perturbations.jl:196-265).  Every coefficient of row c is a
-// row constant times one table scalar: l1 = al·K[kl], u1 = au·K[ku],
-// d = dc + dt·τ′ + di/(ℋη) + dr·τ′R, c_S = cs·K[kcs], c_P = cp, c_Π = cpi·τ′,
-// all times K[km] (the RSA factor on photon/ν rows, 1 elsewhere).  dt, dc, dr
-// follow from the row index (d_coef); al, au, di, cs, cp, cpi are stored.  The
-// second band is v_b's u2 = 3τ′R (row 1) and Θ₁'s l2 = τ′/3 (row 3).
-enum { RC_AL = 0, RC_AU, RC_DI, RC_CS, RC_CP, RC_CPI, RC_N };
-
-// the diagonal of L at row c: dt = 1 on the photon rows from Θ₁ on (Θ₀ has no
-// τ′ term), dc = -1 on v_b (row 1) and v, dr = 1 on v_b
-__device__ inline double d_coef(const Geo& G, const double* K, int c, double di) {
-    const double dc = (c == 1 || c == G.cD + 1) ? -1.0 : 0.0;
-    const double dtp = (c >= 3 && c < G.cC) ? K[K_TP] : 0.0;
-    const double drp = c == 1 ? K[K_TPR] : 0.0;
-    return dc + dtp + di * K[K_IHETA] + drp;
-}
-
-__device__ inline void row_recipe(const CosmoDev& C, const Geo& G, const WS& W, int c) {
-    const int dsc = W.desc()[c];
-    const int type = dsc & 31, l = (dsc >> 5) & 2047, qi = dsc >> 16;
-    const double third = 1.0 / 3.0;
-    const bool photon = type >= R_T0 && type <= R_PN;
-    const bool photon_nu = type >= R_T0 && type <= R_NN;
-    const bool massive = type >= R_M0 && type <= R_MN;
-    const int kq = massive ? K_Q0 + qi : K_KH;
-    double r[RC_N] = {0, 0, 0, 0, 0, 0};
-    int kl = K_KH, ku = K_KH, kcs = K_KH;
-    if (type == R_TL || type == R_PL || type == R_NL || type == R_ML) {
-        // interior of a hierarchy: ℓ/(2ℓ+1) and (ℓ+1)/(2ℓ+1) couplings
-        kl = ku = kq;
-        r[RC_AL] = (double)l / (double)(2 * l + 1);
-        r[RC_AU] = -((double)(l + 1) / (double)(2 * l + 1));
-        r[RC_CPI] = (photon && l == 2) ? -0.1 : 0.0;
-    } else if (type == R_TN || type == R_PN || type == R_NN || type == R_MN) {
-        // truncation rows
-        kl = kq;
-        r[RC_AL] = 1.0;
-        r[RC_DI] = -(double)((type == R_NN ? G.nn : type == R_MN ? G.nm : G.ng) + 1);
-    } else {
-        switch (type) {
-            case R_DB: r[RC_AU] = 1.0; r[RC_CP] = -3.0; break;
-            case R_VB: kl = K_KHCS; r[RC_AL] = -1.0; r[RC_CS] = -1.0; break;
-            case R_T0: case R_N0: r[RC_AU] = -1.0; r[RC_CP] = -1.0; break;
-            case R_T1: r[RC_AL] = third; r[RC_AU] = -2.0 * third; r[RC_CS] = third; break;
-            case R_P0: r[RC_AU] = -1.0; r[RC_CPI] = -0.5; break;
-            case R_N1: r[RC_AL] = third; r[RC_AU] = -2.0 * third; r[RC_CS] = third; break;
-            case R_M0: ku = kq; r[RC_AU] = -1.0; r[RC_CP] = C.df0[qi]; break;
-            case R_M1:
-                kl = ku = kq; kcs = K_Q0 + G.nq + qi;
-                r[RC_AL] = third; r[RC_AU] = -2.0 * third; r[RC_CS] = -third;
-                break;
-            case R_DEL: r[RC_AU] = 1.0; r[RC_CP] = -3.0; break;
-            case R_V: r[RC_CS] = -1.0; break;
-            default: r[RC_CP] = 1.0; break;  // R_PHI
-        }
-    }
-#pragma unroll
-    for (int j = 0; j < RC_N; ++j) W.rcp_(j)[c] = r[j];
-    W.kinds()[c] = kl | (ku << 8) | (kcs << 16) | ((photon_nu ? K_RSA : K_ONE) << 24);
-}
-
-// per-mode row tables (caller syncs): descriptors and recipes of every row,
-// and the segments of the banded LU: consecutive chains packed greedily up to
-// the longest chain's length.  Chains never couple to each other (the first
-// row of a chain has l1 = l2 = 0, the last u1 = u2 = 0), so the LU of a
-// segment is that of its chains and one lane can sweep a whole segment.
-__device__ inline void setup_rows(const CosmoDev& C, const Geo& G, const WS& W, const Thr& T) {
-    for (int c = T.tid; c < G.n; c += T.nt) {
-        W.desc()[c] = row_desc(G, c);
-        row_recipe(C, G, W, c);
-    }
-    if (T.tid == 0) {
-        int lmax = 0;
-        for (int ch = 0; ch < G.nch; ++ch) {
-            int c0, m;
-            chain_range(G, ch, c0, m);
-            lmax = m > lmax ? m : lmax;
-        }
-        int ns = 0, cur0 = 0, curm = 0;
-        for (int ch = 0; ch < G.nch; ++ch) {
-            int c0, m;
-            chain_range(G, ch, c0, m);
-            if (curm > 0 && curm + m > lmax) {
-                W.seg()[2 * ns] = cur0; W.seg()[2 * ns + 1] = curm; ++ns;
-                curm = 0;
-            }
-            if (curm == 0) cur0 = c0;
-            curm += m;
-        }
-        W.seg()[2 * ns] = cur0; W.seg()[2 * ns + 1] = curm; ++ns;
-        W.misc()[0] = ns;
-    }
-}
-
-// per-x q-quantities of bin i at scale factor a (perturbations.jl:203-213,
-// 127-145) into the arrays at p (qe, eqdf, sw, rw, nq apart), and their
-// entries of the scalar table K (kH = k/ℋ at the same x)
-__device__ inline void qfill_one(const CosmoDev& C, const WS& W, double a, double kH, double* p, double* K, int i) {
-    double q = W.q()[i];
-    double am = a * C.mnu;
-    double eps = sqrt(q * q + am * am);
-    double ie = 1.0 / eps;
-    const double qe = q * ie, eqdf = eps / q * W.df0()[i];
-    p[i] = qe;
-    p[W.nq + i] = eqdf;
-    p[2 * W.nq + i] = W.base()[i] * (q * q * ie);
-    p[3 * W.nq + i] = W.base()[i] * eps;
-    K[K_Q0 + i] = kH * qe;
-    K[K_Q0 + W.nq + i] = kH * eqdf;
-}
-
-// the x-only entries of a scalar table
-__device__ inline void ktab_head(double* K, const XC& X) {
-    K[K_KH] = X.kH;
-    K[K_TP] = X.tp;
-    K[K_IHETA] = X.iHeta;
-    K[K_TPR] = X.tp * X.R;
-    K[K_KHCS] = X.kH * X.csb2;
-    K[K_ONE] = 1.0;
-    K[K_RSA] = X.rsa ? 0.0 : 1.0;
-}
-
-// the current-x set and scalar table (every thread holds the same X); caller
-// syncs
-__device__ inline void qfill(const CosmoDev& C, const Geo& G, const XC& X, const WS& W, const Thr& T) {
-    if (T.tid < G.nq) qfill_one(C, W, X.a, X.kH, W.qe(), W.kcur(), T.tid);
-    if (T.tid == T.nt - 1) ktab_head(W.kcur(), X);
-}
-
-// One row of du = L u + c_S Ψ + c_P Φ′ + c_Π Π (perturbations.jl:196-265)
-// from its recipe and the scalar table K of the x point
-__device__ inline double row_eval(const Geo& G, const WS& W, const double* K, const double* v, int c, int n, double S,
-                                  double P, double Pi) {
-    // branch-free: the first row has no l1 and the last no u1, so clamped
-    // neighbours contribute exact zeros
-    const int kd = W.kinds()[c];
-    const int cm = c > 0 ? c - 1 : 0, cp = c + 1 < n ? c + 1 : c;
-    const double d = d_coef(G, K, c, W.rcp_(RC_DI)[c]);
-    double acc = d * v[c];
-    acc += (W.rcp_(RC_AL)[c] * K[kd & 255]) * v[cm];
-    acc += (W.rcp_(RC_AU)[c] * K[(kd >> 8) & 255]) * v[cp];
-    const double e1 = (3.0 * K[K_TPR]) * v[3], e3 = (K[K_TP] * (1.0 / 3.0)) * v[1];
-    acc += c == 1 ? e1 : (c == 3 ? e3 : 0.0);
-    acc += (W.rcp_(RC_CS)[c] * K[(kd >> 16) & 255]) * S + W.rcp_(RC_CP)[c] * P + (W.rcp_(RC_CPI)[c] * K[K_TP]) * Pi;
-    return K[kd >> 24] * acc;
-}
-
-// Ψ, Φ′, Π of chain-ordered vectors (perturbations.jl:184-194, 247)
-struct Fun {
-    double S, P, Pi;
-};
-
-// the fixed rows of a chain-ordered vector the functionals read
-struct FunRows {
-    double e, t2, n2, dl, db, t0, n0, p2, p0;
-};
-__device__ inline FunRows fun_rows(const Geo& G, const double* v) {
-    FunRows r;
-    r.e = v[G.cE]; r.t2 = v[4]; r.n2 = v[G.cC + 2]; r.dl = v[G.cD]; r.db = v[0]; r.t0 = v[2]; r.n0 = v[G.cC];
-    r.p2 = v[G.cB + 2]; r.p0 = v[G.cB];
-    return r;
-}
-
-__device__ inline Fun fun_finish(const CosmoDev& C, const XC& X, const FunRows& v, double s2, double s0) {
-    Fun F;
-    F.S = -v.e - X.c12 * (C.Or * v.t2 + C.Onu * v.n2) - X.fs2 * s2;
-    F.P = F.S - X.k23 * v.e + (X.fp0 * v.dl + X.fp1 * v.db + X.fp2 * v.t0 + X.fp3 * v.n0 + X.fp4 * s0);
-    F.Pi = v.t2 + v.p2 + v.p0;
-    return F;
-}
-
-// the q-bin sums Σ sw_i v[ℳ₂,ᵢ] and Σ rw_i v[ℳ₀,ᵢ] of a vector, folded onto
-// lanes 0..15 (bins i, i+16, i+32 on lane i)
-__device__ inline void qsum_fold(const Geo& G, const QSet& Q, const double* v, int lane, double& s2, double& s0) {
-    s2 = 0.0; s0 = 0.0;
-    for (int i = lane; i < G.nq && lane < 16; i += 16) {
-        const int b = G.cM + i * (G.nm + 1);
-        s2 += Q.sw[i] * v[b + 2];
-        s0 += Q.rw[i] * v[b];
-    }
-}
-
-// every wavefront forms the sums over its own lanes (identical in all of them)
-__device__ inline Fun functionals(const CosmoDev& C, const Geo& G, const XC& X, const QSet& Q, const double* v,
-                                  const Thr& T) {
-    const FunRows r = fun_rows(G, v);
-    double a[2];
-    qsum_fold(G, Q, v, T.lane, a[0], a[1]);
-    row0_sums<2>(a);
-    return fun_finish(C, X, r, a[0], a[1]);
-}
-
-// du = f(v) on all rows (out = scale·du), optionally writing the border
-// columns c_S, c_P, c_Π; K is the scalar table of the same x as X and Q;
-// returns the functionals of v
-__device__ inline Fun rhs_rows(const CosmoDev& C, const Geo& G, const XC& X, const WS& W, const QSet& Q,
-                               const double* K, const double* v, double scale, double* out, bool make_c,
-                               const Thr& T, double* copy = nullptr) {
-    Fun F = functionals(C, G, X, Q, v, T);
-    // two rows per thread, every load before any store, so the two rows'
-    // LDS latencies overlap (a row past n repeats row c0 and is not stored)
-    for (int c0 = T.tid; c0 < G.n; c0 += 2 * T.nt) {
-        const int c1 = c0 + T.nt;
-        const bool in1 = c1 < G.n;
-        const int cc[2] = {c0, in1 ? c1 : c0};
-        double r[2], cs[2], cp[2], cpi[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int c = cc[i];
-            r[i] = scale * row_eval(G, W, K, v, c, G.n, F.S, F.P, F.Pi);
-            if (make_c) {
-                const int kd = W.kinds()[c];
-                const double m = K[kd >> 24];
-                cs[i] = m * (W.rcp_(RC_CS)[c] * K[(kd >> 16) & 255]);
-                cp[i] = m * W.rcp_(RC_CP)[c];
-                cpi[i] = m * (W.rcp_(RC_CPI)[c] * K[K_TP]);
-            }
-        }
-        // past n, cc[1] = c0: the repeat is stored first, row c0's own value last
-#pragma unroll
-        for (int i = 1; i >= 0; --i) {
-            const int c = cc[i];
-            out[c] = r[i];
-            if (copy) copy[c] = r[i];
-            if (make_c) { W.cS()[c] = cs[i]; W.cP()[c] = cp[i]; W.cPi()[c] = cpi[i]; }
-        }
-    }
-    return F;
-}
-
-// ------------------------------------------- tangent-linear (forward mode)
-// The derivative of the whole path along one direction of the cosmological
-// parameters, carried beside the solution the way ForwardDiff.Dual carries it
-// through Bolt's code (runtests.jl:54-80, examples/plot_deriv_cl.jl:100-125).
-// The tables, scalars and q arrays come with a tangent copy (a CosmoDev whose
-// every field is the derivative of the primal's); the pieces below form the
-// tangent of each quantity the solver builds from them.  With f(v) = L(p) v,
-// the tangent of f at (v, v̇) is L v̇ + L̇ v: the primal rows applied to v̇ plus
-// the rows' parameter derivative applied to v.
-
-// value and one directional derivative
-struct D1 {
-    double v, d;
-};
-__device__ inline D1 operator+(D1 a, D1 b) { return {a.v + b.v, a.d + b.d}; }
-__device__ inline D1 operator-(D1 a, D1 b) { return {a.v - b.v, a.d - b.d}; }
-__device__ inline D1 operator-(D1 a) { return {-a.v, -a.d}; }
-__device__ inline D1 operator*(D1 a, D1 b) { return {a.v * b.v, a.d * b.v + a.v * b.d}; }
-__device__ inline D1 operator/(D1 a, D1 b) {
-    const double q = a.v / b.v;
-    return {q, (a.d - q * b.d) / b.v};
-}
-__device__ inline D1 operator+(D1 a, double b) { return {a.v + b, a.d}; }
-__device__ inline D1 operator+(double a, D1 b) { return {a + b.v, b.d}; }
-__device__ inline D1 operator-(D1 a, double b) { return {a.v - b, a.d}; }
-__device__ inline D1 operator-(double a, D1 b) { return {a - b.v, -b.d}; }
-__device__ inline D1 operator*(D1 a, double b) { return {a.v * b, a.d * b}; }
-__device__ inline D1 operator*(double a, D1 b) { return {a * b.v, a * b.d}; }
-__device__ inline D1 operator/(D1 a, double b) { return {a.v / b, a.d / b}; }
-__device__ inline D1 operator/(double a, D1 b) {
-    const double q = a / b.v;
-    return {q, -q * b.d / b.v};
-}
-__device__ inline D1 exp(D1 a) {
-    const double e = exp(a.v);
-    return {e, e * a.d};
-}
-__device__ inline D1 sqrt(D1 a) {
-    const double s = sqrt(a.v);
-    return {s, a.d / (2.0 * s)};
-}
-__device__ inline D1 wave_sum(D1 a) { return {wave_sum(a.v), wave_sum(a.d)}; }
-template <class S> struct is_d1 { static constexpr bool value = false; };
-template <> struct is_d1<D1> { static constexpr bool value = true; };
-
-// derivatives of the XC fields (x and a carry none: the grid is fixed)
-struct XCd {
-    double Hc, eta, tp, tpp, csb2, kH, R, c12, gg, k23, iHeta, fs2, fp0, fp1, fp2, fp3, fp4;
-};
-#define NXCD 17
-
-__device__ inline XCd make_xcd(const CosmoDev& C, const CosmoDev& Cd, const XC& X) {
-    XCd D;
-    const double x = X.x, ia = 1.0 / X.a;
-    D.Hc = spl(Cd, BOLT_T_HC, x);
-    D.eta = spl(Cd, BOLT_T_ETA, x);
-    D.tp = spl(Cd, BOLT_T_TAU_P, x);
-    D.tpp = spl(Cd, BOLT_T_TAU_PP, x);
-    D.csb2 = spl(Cd, BOLT_T_CSB2, x);
-    const double rH = D.Hc / X.Hc, rH0 = Cd.H0 / C.H0, rrho = Cd.rho_crit / C.rho_crit;
-    D.kH = -X.kH * rH;
-    D.R = X.R * (Cd.Or / C.Or - Cd.Ob / C.Ob);
-    D.c12 = X.c12 * (2.0 * rH0);
-    D.gg = X.gg * (2.0 * (rH0 - rH));
-    D.k23 = -2.0 * X.k23 * rH;
-    D.iHeta = -X.iHeta * (rH + D.eta / X.eta);
-    D.fs2 = (D.c12 - X.c12 * rrho) * (0.25 / C.rho_crit);
-    D.fp0 = (D.gg * C.Oc + X.gg * Cd.Oc) * ia;
-    D.fp1 = (D.gg * C.Ob + X.gg * Cd.Ob) * ia;
-    D.fp2 = (D.gg * C.Or + X.gg * Cd.Or) * (4.0 * ia * ia);
-    D.fp3 = (D.gg * C.Onu + X.gg * Cd.Onu) * (4.0 * ia * ia);
-    D.fp4 = (D.gg - X.gg * rrho) / C.rho_crit * (ia * ia);
-    return D;
-}
-__device__ inline void store_xcd(double* p, const XCd& D) {
-    const double v[NXCD] = {D.Hc, D.eta, D.tp, D.tpp, D.csb2, D.kH, D.R, D.c12, D.gg,
-                            D.k23, D.iHeta, D.fs2, D.fp0, D.fp1, D.fp2, D.fp3, D.fp4};
-#pragma unroll
-    for (int i = 0; i < NXCD; ++i) p[i] = v[i];
-}
-__device__ inline XCd load_xcd(const double* p) {
-    XCd D;
-    D.Hc = p[0]; D.eta = p[1]; D.tp = p[2]; D.tpp = p[3]; D.csb2 = p[4]; D.kH = p[5]; D.R = p[6]; D.c12 = p[7];
-    D.gg = p[8]; D.k23 = p[9]; D.iHeta = p[10]; D.fs2 = p[11]; D.fp0 = p[12]; D.fp1 = p[13]; D.fp2 = p[14];
-    D.fp3 = p[15]; D.fp4 = p[16];
-    return D;
-}
-
-// Tangent workspace of one k-mode, after the primal's: ẏ vectors u̇, ḟ, u̇ₙ₊₁,
-// ḟₙ₊₁, the stage argument's tangent, the tangent right-hand side/solution, Ż₀..Ż₅;
-// the q arrays' tangents (mode constants), the current x's and the five stage
-// points' tangent q-sets, their XC tangents and tangent scalar tables.
-struct WTan {
-    double* b;
-    int n, nq;
-    __host__ __device__ double* ud() const { return b; }
-    __host__ __device__ double* fd() const { return b + n; }
-    __host__ __device__ double* und() const { return b + 2 * n; }
-    __host__ __device__ double* fnd() const { return b + 3 * n; }
-    __host__ __device__ double* argd() const { return b + 4 * n; }
-    __host__ __device__ double* wd() const { return b + 5 * n; }
-    __host__ __device__ double* Zd(int j) const { return b + (6 + j) * n; }
-    __host__ __device__ double* qd() const { return b + 12 * n; }
-    __host__ __device__ double* df0d() const { return b + 12 * n + nq; }
-    __host__ __device__ double* based() const { return b + 12 * n + 2 * nq; }
-    // tangent q-set of the current x (s = 5) or of stage point s
-    __host__ __device__ double* qset_base(int s) const { return b + 12 * n + (3 + 4 * s) * nq; }
-    __host__ __device__ QSet qset(int s) const {
-        const double* p = qset_base(s);
-        QSet Q; Q.qe = p; Q.eqdf = p + nq; Q.sw = p + 2 * nq; Q.rw = p + 3 * nq;
-        return Q;
-    }
-    __host__ __device__ double* xcd(int s) const { return b + 12 * n + 27 * nq + NXCD * s; }
-    __host__ __device__ double* ktd(int s) const { return b + 12 * n + 27 * nq + 6 * NXCD + (K_Q0 + 2 * nq) * s; }
-};
-__host__ __device__ inline size_t wtan_doubles(int n, int nq) { return (size_t)12 * n + 39 * nq + 6 * NXCD + 6 * K_Q0; }
-// the tangent workspace starts after the primal's, on a double boundary
-__host__ __device__ inline size_t wtan_offset(int n, int nq) { return (ws_bytes(n, nq) + 7) / 8; }
-
-// the tangent entries of a scalar table
-__device__ inline void ktab_head_dot(double* Kd, const XC& X, const XCd& D) {
-    Kd[K_KH] = D.kH;
-    Kd[K_TP] = D.tp;
-    Kd[K_IHETA] = D.iHeta;
-    Kd[K_TPR] = D.tp * X.R + X.tp * D.R;
-    Kd[K_KHCS] = D.kH * X.csb2 + X.kH * D.csb2;
-    Kd[K_ONE] = 0.0;
-    Kd[K_RSA] = 0.0;
-}
-
-// tangent of qfill_one for bin i: p is the primal q-set qfill_one has just
-// written (same thread), pd its tangent; kH, kHd the primal and tangent k/ℋ.
-// dlnf0/dlnq depends on q/T_ν only, which no parameter moves; its tangent
-// array is carried all the same.
-__device__ inline void qfill_one_dot(const CosmoDev& C, const CosmoDev& Cd, const WS& W, const WTan& Wt, double a,
-                                     double kH, double kHd, const double* p, double* pd, double* Kd, int i) {
-    const int nq = W.nq;
-    const double q = W.q()[i], qd = Wt.qd()[i];
-    const double am = a * C.mnu, amd = a * Cd.mnu;
-    const double eps = sqrt(q * q + am * am), epsd = (q * qd + am * amd) / eps;
-    const double qe = p[i], eqdf = p[nq + i];
-    const double qed = (qd - qe * epsd) / eps;
-    const double df0 = W.df0()[i], df0d = Wt.df0d()[i];
-    const double eqdfd = (epsd / q - eps * qd / (q * q)) * df0 + eps / q * df0d;
-    const double base = W.base()[i], based = Wt.based()[i];
-    const double swd = based * (q * q / eps) + base * (2.0 * q * qd / eps - q * q * epsd / (eps * eps));
-    const double rwd = based * eps + base * epsd;
-    pd[i] = qed;
-    pd[nq + i] = eqdfd;
-    pd[2 * nq + i] = swd;
-    pd[3 * nq + i] = rwd;
-    Kd[K_Q0 + i] = kHd * qe + kH * qed;
-    Kd[K_Q0 + nq + i] = kHd * eqdf + kH * eqdfd;
-}
-
-// the parameter part of Ψ and Φ′ at a fixed vector (Π has none)
-struct FunD {
-    double S, P;
-};
-__device__ inline FunD fun_finish_p(const CosmoDev& C, const CosmoDev& Cd, const XC& X, const XCd& D,
-                                    const FunRows& v, double s2, double s0, double s2d, double s0d) {
-    FunD F;
-    F.S = -D.c12 * (C.Or * v.t2 + C.Onu * v.n2) - X.c12 * (Cd.Or * v.t2 + Cd.Onu * v.n2) - D.fs2 * s2 - X.fs2 * s2d;
-    F.P = F.S - D.k23 * v.e + (D.fp0 * v.dl + D.fp1 * v.db + D.fp2 * v.t0 + D.fp3 * v.n0 + D.fp4 * s0 + X.fp4 * s0d);
-    return F;
-}
-
-// functionals of v̇ (F1, primal coefficients) and of v (F0) with their
-// parameter part (P0): the tangent functionals are F1 + P0 (Π: F1.Pi)
-__device__ inline void functionals_tan(const CosmoDev& C, const CosmoDev& Cd, const Geo& G, const XC& X,
-                                       const XCd& D, const QSet& Q, const QSet& Qd, const double* vd,
-                                       const double* v, const Thr& T, Fun& F1, Fun& F0, FunD& P0) {
-    const FunRows r1 = fun_rows(G, vd), r0 = fun_rows(G, v);
-    double a[6];
-    qsum_fold(G, Q, vd, T.lane, a[0], a[1]);
-    qsum_fold(G, Q, v, T.lane, a[2], a[3]);
-    qsum_fold(G, Qd, v, T.lane, a[4], a[5]);
-    row0_sums<6>(a);
-    F1 = fun_finish(C, X, r1, a[0], a[1]);
-    F0 = fun_finish(C, X, r0, a[2], a[3]);
-    P0 = fun_finish_p(C, Cd, X, D, r0, a[2], a[3], a[4], a[5]);
-}
-
-// the parameter derivative of row c of f at a fixed vector v (F0, P0: v's
-// functionals and their parameter part); the RSA factor carries no tangent
-__device__ inline double row_eval_p(const Geo& G, const WS& W, const double* K, const double* Kd, const double* v,
-                                    int c, int n, const Fun& F0, const FunD& P0) {
-    const int kd = W.kinds()[c];
-    const int cm = c > 0 ? c - 1 : 0, cp = c + 1 < n ? c + 1 : c;
-    const double dd = ((c >= 3 && c < G.cC) ? Kd[K_TP] : 0.0) + W.rcp_(RC_DI)[c] * Kd[K_IHETA] +
-                      (c == 1 ? Kd[K_TPR] : 0.0);
-    double acc = dd * v[c];
-    acc += (W.rcp_(RC_AL)[c] * Kd[kd & 255]) * v[cm];
-    acc += (W.rcp_(RC_AU)[c] * Kd[(kd >> 8) & 255]) * v[cp];
-    const double e1 = (3.0 * Kd[K_TPR]) * v[3], e3 = (Kd[K_TP] * (1.0 / 3.0)) * v[1];
-    acc += c == 1 ? e1 : (c == 3 ? e3 : 0.0);
-    const int kcs = (kd >> 16) & 255;
-    acc += W.rcp_(RC_CS)[c] * (Kd[kcs] * F0.S + K[kcs] * P0.S) + W.rcp_(RC_CP)[c] * P0.P +
-           (W.rcp_(RC_CPI)[c] * Kd[K_TP]) * F0.Pi;
-    return K[kd >> 24] * acc;
-}
-
-// out = scale·(f(v̇) + L̇ v) on all rows; returns the tangent functionals
-__device__ inline Fun rhs_rows_tan(const CosmoDev& C, const CosmoDev& Cd, const Geo& G, const XC& X, const XCd& D,
-                                   const WS& W, const QSet& Q, const QSet& Qd, const double* K, const double* Kd,
-                                   const double* vd, const double* v, double scale, double* out, const Thr& T) {
-    Fun F1, F0;
-    FunD P0;
-    functionals_tan(C, Cd, G, X, D, Q, Qd, vd, v, T, F1, F0, P0);
-    for (int c = T.tid; c < G.n; c += T.nt)
-        out[c] = scale * (row_eval(G, W, K, vd, c, G.n, F1.S, F1.P, F1.Pi) + row_eval_p(G, W, K, Kd, v, c, G.n, F0, P0));
-    Fun Ft;
-    Ft.S = F1.S + P0.S;
-    Ft.P = F1.P + P0.P;
-    Ft.Pi = F1.Pi;
-    return Ft;
-}
-
-// W = I - hγL at the five stage points (their scalar tables stored): each
-// thread takes two rows through all five stages, loads before stores; caller
-// syncs
-template <class P>
-__device__ inline void stage_bands(const Geo& G, const WS& W, double hg, const Thr& T) {
-    for (int c0 = T.tid; c0 < G.n; c0 += 2 * T.nt) {
-        const int c1 = c0 + T.nt;
-        const bool in1 = c1 < G.n;
-        const int cc[2] = {c0, in1 ? c1 : c0};
-        double L[2][5], D[2][5], U[2][5];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int c = cc[i];
-            const int kd = W.kinds()[c];
-            const int kl = kd & 255, ku = (kd >> 8) & 255, km = kd >> 24;
-            const double al = W.rcp_(RC_AL)[c], au = W.rcp_(RC_AU)[c], di = W.rcp_(RC_DI)[c];
-#pragma unroll
-            for (int s = 0; s < 5; ++s) {
-                const double* K = W.ktab(s);
-                const double mh = K[km] * hg;
-                L[i][s] = -mh * (al * K[kl]);
-                D[i][s] = 1.0 - mh * d_coef(G, K, c, di);
-                U[i][s] = -mh * (au * K[ku]);
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < 5; ++s) {
-            const BandsT<P> B = W.bandsT<P>(s);
-#pragma unroll
-            for (int i = 1; i >= 0; --i) {  // past n, the repeat of row c0 first, its own values last
-                const int c = cc[i];
-                B.l1[c] = P(L[i][s]); B.d[c] = P(D[i][s]); B.u1[c] = P(U[i][s]);
-            }
-        }
-        if (c0 < CB) {
-            const int km = W.kinds()[c0] >> 24;
-#pragma unroll
-            for (int s = 0; s < 5; ++s) {
-                const double* K = W.ktab(s);
-                const double mh = K[km] * hg;
-                const BandsT<P> B = W.bandsT<P>(s);
-                B.l2c[c0] = P(c0 == 3 ? -mh * (K[K_TP] * (1.0 / 3.0)) : 0.0);
-                B.u2c[c0] = P(c0 == 1 ? -mh * (3.0 * K[K_TPR]) : 0.0);
-            }
-        }
-    }
-}
-
-// RSA overwrite of u (perturbations.jl:217-227); one lane; caller syncs around.
-// S = D1: also the tangent vd (with D, vd and Phip's derivative); the entries
-// read (Φ, v_b, δ_b) are not among those written.
-template <class S>
-__device__ inline void rsa_mutate_t(const Geo& G, const XC& X, const XCd* D, double k, double* v, double* vd, S Phip) {
-    S Phi, vb, db, Hc, tp, tpp, csb2;
-    if constexpr (is_d1<S>::value) {
-        Phi = {v[G.cE], vd[G.cE]}; vb = {v[1], vd[1]}; db = {v[0], vd[0]};
-        Hc = {X.Hc, D->Hc}; tp = {X.tp, D->tp}; tpp = {X.tpp, D->tpp}; csb2 = {X.csb2, D->csb2};
-    } else {
-        Phi = v[G.cE]; vb = v[1]; db = v[0];
-        Hc = X.Hc; tp = X.tp; tpp = X.tpp; csb2 = X.csb2;
-    }
-    const S r[4] = {Phi - Hc / k * tp * vb,
-                    Hc / k * (-2.0 * Phip + tp * (Phi - csb2 * db) + Hc / k * (tpp - tp) * vb),
-                    Phi, -2.0 * Hc / k * Phip};
-    const int at[4] = {2, 3, G.cC, G.cC + 1};
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        if constexpr (is_d1<S>::value) { v[at[i]] = r[i].v; vd[at[i]] = r[i].d; }
-        else v[at[i]] = r[i];
-    }
-    v[4] = 0.0;
-    v[G.cC + 2] = 0.0;
-    if constexpr (is_d1<S>::value) { vd[4] = 0.0; vd[G.cC + 2] = 0.0; }
-}
-__device__ inline void rsa_mutate(const Geo& G, const XC& X, double k, double* v, double Phip) {
-    rsa_mutate_t<double>(G, X, nullptr, k, v, nullptr, Phip);
-}
-
-// Banded LU (bandwidth 2, no pivoting) of every segment, one lane per segment, in
-// left-looking form: row j is finished from rows j-1, j-2 only, so the carried
-// dependency is the pivot recurrence.  Rows are processed in blocks of CB: a
-// block's inputs are loaded into registers before its sequential sweep.
-// Stored: d <- 1/pivot, l1/l2 <- multipliers, u1 <- updated upper entry (u2 is
-// never modified by the elimination).  Reads past the segment end stay inside
-// the LDS workspace and are never stored back.
-//
-// The second band is nonzero on two rows only, both in the first block of the
-// first segment: u2 on v_b (its Θ₁ coupling) and l2 on Θ₁ (its v_b coupling).
-// Every later block is therefore tridiagonal, and there u1 is left unchanged
-// (u1 -= m1·u2 with u2 = 0), which halves the work of those rows.
-// one tridiagonal factor block of rows jb..jb+CB-1; GUARD: store only rows < m
-template <bool GUARD, class T>
-__device__ inline void factor_tri_block(T* l1, T* d, const T* u1, int jb, int m, T& ip1, T& u1p1, T* dump) {
-    T L1[CB], D[CB], U1[CB];
-#pragma unroll
-    for (int i = 0; i < CB; ++i) { L1[i] = l1[jb + i]; D[i] = d[jb + i]; U1[i] = u1[jb + i]; }
-    // the pivot chain is inv_i = 1/(D_i - (L1_i·U1_{i-1})·inv_{i-1}): the
-    // products and the multipliers L1_i·inv_{i-1} stay off it
-    T P[CB];
-#pragma unroll
-    for (int i = 0; i < CB; ++i) {
-        P[i] = L1[i] * u1p1;
-        u1p1 = U1[i];
-    }
-#pragma unroll
-    for (int i = 0; i < CB; ++i) {
-        const T m1 = L1[i] * ip1;
-        const T inv = rcp_piv(fmaT(-P[i], ip1, D[i]));
-        L1[i] = m1; D[i] = inv;
-        ip1 = inv;
-    }
-#pragma unroll
-    for (int i = 0; i < CB; ++i) {
-        const bool in = !GUARD || jb + i < m;
-        *(in ? l1 + jb + i : dump) = L1[i];
-        *(in ? d + jb + i : dump) = D[i];
-    }
-}
-
-// (stores past the segment's end go to the never-read slot dump); T = float
-// factors the FP32 solve mode's bands
-template <class T>
-__device__ inline void chain_factor_seg(const BandsT<T>& Bd, int c0, int m, T* dump) {
-    T* l1 = Bd.l1 + c0; T* d = Bd.d + c0; T* u1 = Bd.u1 + c0;
-    const bool first = c0 == 0;  // the only segment with a second band
-    T ip1 = 0, ip2 = 0, u1p1 = 0, u1p2 = 0, u2p1 = 0, u2p2 = 0;
-    {   // rows 0..FB-1: the full bandwidth-2 recurrence (the second band sits in
-        // rows 1 and 3 of the first segment; from row 4 on L is tridiagonal and
-        // row 3's upper entry is unchanged)
-        constexpr int FB = 4;
-        T L2[FB], L1[FB], D[FB], U1[FB], U2[FB];
-#pragma unroll
-        for (int i = 0; i < FB; ++i) {
-            const T l2 = Bd.l2c[i], u2 = Bd.u2c[i];
-            L2[i] = first ? l2 : T(0); U2[i] = first ? u2 : T(0);
-            L1[i] = l1[i]; D[i] = d[i]; U1[i] = u1[i];
-        }
-#pragma unroll
-        for (int i = 0; i < FB; ++i) {
-            T m2 = L2[i] * ip2;
-            T m1 = (L1[i] - m2 * u1p2) * ip1;
-            T dd = (D[i] - m2 * u2p2) - m1 * u1p1;
-            T uu = U1[i] - m1 * u2p1;
-            T inv = rcp_piv(dd);
-            L2[i] = m2; L1[i] = m1; D[i] = inv; U1[i] = uu;
-            ip2 = ip1; ip1 = inv;
-            u1p2 = u1p1; u1p1 = uu;
-            u2p2 = u2p1; u2p1 = U2[i];
-        }
-#pragma unroll
-        for (int i = 0; i < FB; ++i) {
-            const bool in = i < m;
-            *(first && in ? Bd.l2c + i : dump) = L2[i];
-            *(in ? l1 + i : dump) = L1[i];
-            *(in ? d + i : dump) = D[i];
-            *(in ? u1 + i : dump) = U1[i];
-        }
-    }
-    // tridiagonal blocks of CB rows: full ones unguarded (lanes with shorter
-    // segments leave the loop early), then the partial tail
-    int jb = 4;
-    for (; jb + CB <= m; jb += CB) factor_tri_block<false>(l1, d, u1, jb, m, ip1, u1p1, dump);
-    if (jb < m) factor_tri_block<true>(l1, d, u1, jb, m, ip1, u1p1, dump);
-}
-
-// the LU of all five stage points, one (stage, segment) unit per lane of
-// one wavefront
-template <class T>
-__device__ inline void chain_factor_all(const Geo& G, const WS& W, int lane) {
-    const int nseg = W.misc()[0];
-    for (int u = lane; u < 5 * nseg; u += WAVE) {
-        const int st = u / nseg, sg = u - st * nseg;
-        chain_factor_seg<T>(W.bandsT<T>(st), W.seg()[2 * sg], W.seg()[2 * sg + 1], (T*)W.dump());
-    }
-}
-
-// Makes LDS stores of any lane of this wavefront visible to later LDS loads of
-// any other lane of the same wavefront.  The hardware completes one
-// wavefront's LDS operations in issue order, so what is needed is that the
-// compiler keep them in program order across this point: a wavefront-scope
-// fence (no instruction is emitted for it) and a wave barrier, neither of which
-// LDS accesses may cross.
-__device__ inline void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// ---- substitution by wavefront scans
-// With every chain's first row at l1 = 0 and last row at u1 = 0, the forward
-// and back substitutions over all n rows are each one first-order affine
-// recurrence, y_j = b_j - l1_j·y_{j-1} and x_j = d_j·y_j - d_j·u1_j·x_{j+1}
-// (the chain boundaries cut it by themselves).  A wavefront takes 64·SR rows
-// at a time, SR consecutive rows per lane: each lane composes the maps
-// f_j(t) = a_j·t + b_j of its rows in registers, an inclusive scan across the
-// lanes composes the lane maps (Hillis-Steele in rows of 16 with row_shr 1, 2,
-// 4, 8, then row_bcast 15 and 31 across rows), and each lane takes its
-// incoming value from the previous lane (wave_shr 1).  The two second-band
-// entries (l2 on row 3, u2 on row 1) are added as exact corrections in the
-// lane holding rows 0..3.
-
-// 64-bit DPP move; lanes whose source is invalid or whose row is masked off
-// keep `old`
-template <int CTRL, int RMASK>
-__device__ inline double dpp64_keep(double v, double old) {
-    int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), CTRL, RMASK, 0xF, false);
-    int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), CTRL, RMASK, 0xF, false);
-    return __hiloint2double(hi, lo);
-}
-template <int CTRL, int RMASK>
-__device__ inline float dpp32_keep(float v, float old) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(old), __float_as_int(v), CTRL, RMASK, 0xF, false));
-}
-template <int CTRL, int RMASK> __device__ inline double dppk(double v, double old) { return dpp64_keep<CTRL, RMASK>(v, old); }
-template <int CTRL, int RMASK> __device__ inline float dppk(float v, float old) { return dpp32_keep<CTRL, RMASK>(v, old); }
-// (a, b) <- (a, b) ∘ (a', b') with (a', b') from the lane CTRL names; missing
-// sources act as the identity map (1, 0)
-template <int CTRL, int RMASK, class T>
-__device__ inline void affine_step(T& a, T& b) {
-    const T ap = dppk<CTRL, RMASK>(a, T(1));
-    const T bp = dppk<CTRL, RMASK>(b, T(0));
-    b = fmaT(a, bp, b);
-    a = a * ap;
-}
-// the same for row_shr steps: a lane without a source keeps (a, b) since its
-// b' = a·0 + b with a zero-filled b'
-template <int CTRL, class T>
-__device__ inline void affine_step_shr(T& a, T& b) {
-    const T ap = dppk<CTRL, 0xF>(a, T(1));
-    const T bp = dppz<CTRL>(b);
-    b = fmaT(a, bp, b);
-    a = a * ap;
-}
-// lane L ends with f_L ∘ f_{L-1} ∘ ... ∘ f_0; every lane of the wavefront
-// must take part
-template <class T>
-__device__ inline void affine_scan(T& a, T& b) {
-    affine_step_shr<0x111>(a, b);
-    affine_step_shr<0x112>(a, b);
-    affine_step_shr<0x114>(a, b);
-    affine_step_shr<0x118>(a, b);
-    affine_step<0x142, 0xA>(a, b);
-    affine_step<0x143, 0xC>(a, b);
-}
-
-static_assert(SR_MIN >= 4, "rows 0..3 must sit in one lane");
-
-// the lane maps of one pass: al/be hold f_i ∘ ... ∘ f_0 of the lane's rows;
-// returns the lane's incoming value and advances carry past the pass
-template <int SR, class T>
-__device__ inline T pass_scan(T (&al)[SR], T (&be)[SR], T& carry) {
-#pragma unroll
-    for (int i = 1; i < SR; ++i) { be[i] = fmaT(al[i], be[i - 1], be[i]); al[i] = al[i] * al[i - 1]; }
-    T A = al[SR - 1], B = be[SR - 1];
-    affine_scan(A, B);
-    const T last = fmaT(A, carry, B);
-    const T tin = dppk<0x138, 0xF>(last, carry);  // wave_shr 1; lane 0 keeps carry
-    carry = rdlane(last, WAVE - 1);
-    return tin;
-}
-
-// forward + back substitution of one right-hand side over all n rows by one
-// wavefront (all 64 lanes, uniform control flow).  Branch-free: loads past n
-// stay inside the workspace (it ends with one pass of padding), and stores
-// from lanes whose rows lie past n go to the never-read slot `dump`.  In the
-// forward pass rows past n come after every real row, and the scan carries
-// values only toward later rows, so they need no masking; in the backward
-// pass they come first and are masked to the identity map.
-template <int SR, class T>
-__device__ inline void wave_subst(const BandsT<T>& Bd, int n, double* bv, double* dump, int lane) {
-    // T = float: the FP32 solve mode; the vector stays FP64 in LDS and is
-    // rounded on load, the substitution runs in FP32
-    constexpr int span = WAVE * SR;
-    T carry = T(0);
-    for (int p0 = 0; p0 < n; p0 += span) {
-        T al[SR], be[SR];
-        const int j0 = p0 + SR * lane;
-#pragma unroll
-        for (int i = 0; i < SR; ++i) {
-            al[i] = -Bd.l1[j0 + i];
-            be[i] = T(bv[j0 + i]);
-        }
-        // row 3 (Θ₁) also takes -l2·y_1 with y_1 = b_1 - l1_1·b_0
-        const T corr = Bd.l2c[3] * fmaT(al[1], be[0], be[1]);
-        be[3] -= (p0 == 0 && lane == 0) ? corr : T(0);
-        const T tin = pass_scan(al, be, carry);
-#pragma unroll
-        for (int i = 0; i < SR; ++i) {
-            double* dst = j0 + i < n ? bv + j0 + i : dump;
-            *dst = double(fmaT(al[i], tin, be[i]));
-        }
-    }
-    // backward: pass p covers rows p·span .. p·span + span - 1, lane order
-    // running down the rows; it reads rows other lanes stored above
-    wave_lds_sync();
-    carry = T(0);
-    for (int p = (n - 1) / span; p >= 0; --p) {
-        T al[SR], be[SR];
-        const int jt = p * span + span - 1 - SR * lane;  // the lane's highest row
-#pragma unroll
-        for (int i = 0; i < SR; ++i) {
-            const bool in = jt - i < n;
-            const T dj = Bd.d[jt - i], uj = Bd.u1[jt - i], yj = T(bv[jt - i]);
-            al[i] = in ? -dj * uj : T(0);
-            be[i] = in ? dj * yj : T(0);
-        }
-        // rows 1 and 0 (the last lane of pass 0): row 1 (v_b) also takes
-        // -u2·x_3, row 0 then follows from row 1
-        const bool low = p == 0 && lane == WAVE - 1;
-        const T y0 = T(bv[0]), y1 = T(bv[1]), u2 = Bd.u2c[1], u11 = Bd.u1[1], d1 = Bd.d[1], u10 = Bd.u1[0],
-                d0 = Bd.d[0];
-        const T tin = pass_scan(al, be, carry);
-        T x[SR];
-#pragma unroll
-        for (int i = 0; i < SR; ++i) x[i] = fmaT(al[i], tin, be[i]);
-        const T x1 = ((y1 - u2 * x[SR - 4]) - u11 * x[SR - 3]) * d1;
-        const T x0 = (y0 - u10 * x1) * d0;
-        x[SR - 2] = low ? x1 : x[SR - 2];
-        x[SR - 1] = low ? x0 : x[SR - 1];
-#pragma unroll
-        for (int i = 0; i < SR; ++i) {
-            double* dst = jt - i < n ? bv + jt - i : dump;
-            *dst = double(x[i]);
-        }
-    }
-    // the caller's next reads of bv (the border functionals) come from other lanes
-    wave_lds_sync();
-}
-
-// the four right-hand sides w, c_S, c_P, c_Π after chain_factor: wavefront r
-// takes right-hand side r
-template <int SR, class P>
-__device__ inline void chain_solve4(const Geo& G, const WS& W, int st, const Thr& T) {
-    const BandsT<P> Bd = W.bandsT<P>(st);
-    for (int r = T.wv; r < 4; r += T.nt / WAVE) {
-        double* bv = r == 0 ? W.w() : r == 1 ? W.cS() : r == 2 ? W.cP() : W.cPi();
-        wave_subst<SR>(Bd, G.n, bv, W.dump(), T.lane);
-    }
-}
-
-// one right-hand side with the stored factors, by the first wavefront
-template <int SR, class P>
-__device__ inline void chain_solve1(const Geo& G, const WS& W, int st, double* bvec, const Thr& T) {
-    if (T.wv != 0) return;
-    wave_subst<SR>(W.bandsT<P>(st), G.n, bvec, W.dump(), T.lane);
-}
-
-// 3x3 capacitance matrix M = I - hγ D Y (D: Ψ, Φ′, Π rows; Y = W_L⁻¹[c_S c_P c_Π])
-struct Cap {
-    double m[3][3];
-};
-
-__device__ inline void swap_rows_if(bool c, double* x, double* y) {
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        double t = x[j];
-        x[j] = c ? y[j] : x[j];
-        y[j] = c ? t : y[j];
-    }
-}
-
-// Gaussian elimination with partial pivoting, fully unrolled (all indices
-// compile-time, so the 3x4 array stays in registers)
-__device__ inline void solve3(const Cap& K, const double* r, double* y) {
-    double a0[4] = {K.m[0][0], K.m[0][1], K.m[0][2], r[0]};
-    double a1[4] = {K.m[1][0], K.m[1][1], K.m[1][2], r[1]};
-    double a2[4] = {K.m[2][0], K.m[2][1], K.m[2][2], r[2]};
-    swap_rows_if(fabs(a1[0]) > fabs(a0[0]), a0, a1);
-    swap_rows_if(fabs(a2[0]) > fabs(a0[0]), a0, a2);
-    const double p0 = rcp(a0[0]);
-    double f1 = a1[0] * p0, f2 = a2[0] * p0;
-#pragma unroll
-    for (int j = 1; j < 4; ++j) { a1[j] -= f1 * a0[j]; a2[j] -= f2 * a0[j]; }
-    swap_rows_if(fabs(a2[1]) > fabs(a1[1]), a1, a2);
-    const double p1 = rcp(a1[1]);
-    double g2 = a2[1] * p1;
-#pragma unroll
-    for (int j = 2; j < 4; ++j) a2[j] -= g2 * a1[j];
-    y[2] = a2[3] * rcp(a2[2]);
-    y[1] = (a1[3] - a1[2] * y[2]) * p1;
-    y[0] = (a0[3] - a0[1] * y[1] - a0[2] * y[2]) * p0;
-}
-
-// After the chain solves (w = W_L⁻¹ r, c_* = W_L⁻¹ c_*): build the capacitance
-// matrix K and y = K⁻¹ D w; the stage value is z = w + hγ (c_S y₀ + c_P y₁ + c_Π y₂).
-// Wavefront r evaluates the functionals of vector r (w, c_S, c_P, c_Π), which
-// it has itself solved, into red[3r..3r+2]; after a barrier every wavefront
-// forms the same K and y.  Needs four wavefronts; red is not written again
-// before the next barrier.
-__device__ inline Cap stage_border(const CosmoDev& C, const Geo& G, const XC& X, const WS& W, const QSet& Q,
-                                   double hg, const Thr& T, double* y) {
-    const int r = T.wv;
-    if (r < 4) {
-        const double* v = r == 0 ? W.w() : r == 1 ? W.cS() : r == 2 ? W.cP() : W.cPi();
-        const Fun F = functionals(C, G, X, Q, v, T);
-        if (T.lane == 0) { W.red()[3 * r] = F.S; W.red()[3 * r + 1] = F.P; W.red()[3 * r + 2] = F.Pi; }
-    }
-    __syncthreads();
-    const double* f = W.red();
-    Cap K;
-    K.m[0][0] = 1.0 - hg * f[3]; K.m[0][1] = -hg * f[6]; K.m[0][2] = -hg * f[9];
-    K.m[1][0] = -hg * f[4]; K.m[1][1] = 1.0 - hg * f[7]; K.m[1][2] = -hg * f[10];
-    K.m[2][0] = -hg * f[5]; K.m[2][1] = -hg * f[8]; K.m[2][2] = 1.0 - hg * f[11];
-    double rr[3] = {f[0], f[1], f[2]};
-    solve3(K, rr, y);
-    return K;
-}
-
-// source_function (perturbations.jl:343-383) from the chain-ordered (mutated)
-// u, the derivative rows du of Θ₁..₃, Θᵖ₀..₃, 𝒩₂, v_b, ℳ₂,ᵢ, and Φ′
-// S = D1: with its derivative, from the tangent tables (Cd), XC tangent (D),
-// the tangent current q-set (Qd), u̇, du̇ and Φ′'s derivative.
-template <class S>
-__device__ S source_fn_t(const CosmoDev& C, const CosmoDev* Cd, const Geo& G, const XC& X, const XCd* D,
-                         const WS& W, const QSet* Qd, double k, const double* u, const double* ud,
-                         const double* du, const double* dud, S Phip, int lane) {
-    constexpr bool DU = is_d1<S>::value;
-    const double x = X.x;
-    auto tab = [&](int t) -> S {
-        if constexpr (DU) return S{spl(C, t, x), spl(*Cd, t, x)};
-        else return spl(C, t, x);
-    };
-    auto U = [&](int i) -> S {
-        if constexpr (DU) return S{u[i], ud[i]};
-        else return u[i];
-    };
-    auto dU = [&](int i) -> S {
-        if constexpr (DU) return S{du[i], dud[i]};
-        else return du[i];
-    };
-    S Hc, tp, tpp, H0, Or, Onu, rho_crit;
-    if constexpr (DU) {
-        Hc = {X.Hc, D->Hc}; tp = {X.tp, D->tp}; tpp = {X.tpp, D->tpp};
-        H0 = {C.H0, Cd->H0}; Or = {C.Or, Cd->Or}; Onu = {C.Onu, Cd->Onu}; rho_crit = {C.rho_crit, Cd->rho_crit};
-    } else {
-        Hc = X.Hc; tp = X.tp; tpp = X.tpp; H0 = C.H0; Or = C.Or; Onu = C.Onu; rho_crit = C.rho_crit;
-    }
-    S Hcp = tab(BOLT_T_HC_P), Hcpp = tab(BOLT_T_HC_PP);
-    S tau = tab(BOLT_T_TAU);
-    S g = tab(BOLT_T_G), gp = tab(BOLT_T_G_P), gpp = tab(BOLT_T_G_PP);
-    const double a = X.a;
-    S H02 = H0 * H0;
-    S s2 = S(), s2p = S();
-    if (lane < G.nq) {
-        int b = G.cM + lane * (G.nm + 1) + 2;
-        S sw;
-        if constexpr (DU) sw = {W.sw()[lane], Qd->sw[lane]};
-        else sw = W.sw()[lane];
-        s2 = sw * U(b);
-        s2p = sw * dU(b);
-    }
-    S sig = wave_sum(s2), sigp = wave_sum(s2p);
-    S T0 = U(2), T1 = U(3), T2 = U(4), T3 = U(5);
-    S P0 = U(G.cB), P1 = U(G.cB + 1), P2 = U(G.cB + 2), P3 = U(G.cB + 3);
-    S dT1 = dU(3), dT2 = dU(4), dT3 = dU(5);
-    S dP0 = dU(G.cB), dP1 = dU(G.cB + 1), dP2 = dU(G.cB + 2), dP3 = dU(G.cB + 3);
-    S N2 = U(G.cC + 2), dN2 = dU(G.cC + 2);
-    S vb = U(1), vbp = dU(1);
-    S pre = 12.0 * H02 / (k * k) / (a * a);
-    S Psi = -U(G.cE) - pre * (Or * T2 + Onu * N2 + sig / rho_crit / 4.0);
-    S Psip = -Phip - pre * (Or * (dT2 - 2.0 * T2) + Onu * (dN2 - 2.0 * N2) + (sigp - 2.0 * sig) / rho_crit / 4.0);
-    S Pi = T2 + P2 + P0;
-    S Pip = dT2 + dP2 + dP0;
-    S term1 = g * (T0 + Psi + Pi / 4.0) + exp(-tau) * (Psip - Phip);
-    S term2 = (-1.0 / k) * (Hcp * g * vb + Hc * gp * vb + Hc * g * vbp);
-    S Pipp = 2.0 * k / (5.0 * Hc) * (-Hcp / Hc * T1 + dT1) + (3.0 / 10.0) * (tpp * Pi + tp * Pip) -
-             3.0 * k / (5.0 * Hc) * (-Hcp / Hc * (T3 + P1 + P3) + (dT3 + dP1 + dP3));
-    S term3 = (3.0 / (4.0 * k * k)) * ((Hcp * Hcp + Hc * Hcpp) * g * Pi + 3.0 * Hc * Hcp * (gp * Pi + g * Pip) +
-                                       Hc * Hc * (gpp * Pi + 2.0 * gp * Pip + g * Pipp));
-    return term1 + term2 + term3;
-}
-__device__ double source_fn(const CosmoDev& C, const Geo& G, const XC& X, const WS& W, double k, const double* u,
-                            const double* du, double Phip, int lane) {
-    return source_fn_t<double>(C, nullptr, G, X, nullptr, W, nullptr, k, u, nullptr, du, nullptr, Phip, lane);
-}
-
-// source_function_P (perturbations.jl:385-404): (3/(4y²)) g̃ Π with
-// y = k(η(x_grid[end]) − η(x)); ±Inf at the last node, where y = 0
-__device__ inline double source_fn_P(const CosmoDev& C, const Geo& G, const XC& X, double k, const double* u) {
-    double g = spl(C, BOLT_T_G, X.x);
-    double y = k * (spl(C, BOLT_T_ETA, node_x(C, C.nx - 1)) - X.eta);
-    double Pi = u[4] + u[G.cB + 2] + u[G.cB];
-    return (3.0 / (4.0 * y * y)) * g * Pi;
-}
-
-// derivative rows the source function reads (one per lane)
-__device__ inline int source_row(const Geo& G, int lane) {
-    if (lane < 3) return 3 + lane;                 // Θ₁, Θ₂, Θ₃
-    if (lane < 7) return G.cB + (lane - 3);        // Θᵖ₀..₃
-    if (lane == 7) return G.cC + 2;                // 𝒩₂
-    if (lane == 8) return 1;                       // v_b
-    if (lane < 9 + G.nq) return G.cM + (lane - 9) * (G.nm + 1) + 2;  // ℳ₂,ᵢ
-    return -1;
-}
-
-// initial_conditions (perturbations.jl:274-338), chain order; thread 0 does the
-// photon/ν recursions, threads 1..nq the ℳ chains.  S = D1: also u̇ (ud) from
-// the tangent tables and q arrays (Cd, Wt).
-template <class S>
-__device__ void initial_conditions_t(const CosmoDev& C, const CosmoDev* Cd, const Geo& G, const WS& W,
-                                     const WTan* Wt, double k, double* u, double* ud, const Thr& T) {
-    constexpr bool DU = is_d1<S>::value;
-    const int lane = T.tid;
-    const double xi = C.x0;
-    auto tab = [&](int t) -> S {
-        if constexpr (DU) return S{spl(C, t, xi), spl(*Cd, t, xi)};
-        else return spl(C, t, xi);
-    };
-    auto put = [&](int i, S v) {
-        if constexpr (DU) { u[i] = v.v; ud[i] = v.d; }
-        else u[i] = v;
-    };
-    S Hc = tab(BOLT_T_HC), eta = tab(BOLT_T_ETA), tp = tab(BOLT_T_TAU_P);
-    S Nnu, mnu;
-    if constexpr (DU) { Nnu = {C.Nnu, Cd->Nnu}; mnu = {C.mnu, Cd->mnu}; }
-    else { Nnu = C.Nnu; mnu = C.mnu; }
-    double ai = sqrt(exp(xi) * exp(xi));
-    S fnu = 1.0 / (1.0 + 1.0 / (7.0 * (3.0 / 3.0) * Nnu / 8.0 * pow(4.0 / 11.0, 4.0 / 3.0)));
-    S Phi = (4.0 * fnu + 10.0) / (4.0 * fnu + 15.0) * 1.0;
-    S Cc = -((15.0 + 4.0 * fnu) / (20.0 + 8.0 * fnu)) * Phi;
-    S T0 = -40.0 * Cc / (15.0 + 4.0 * fnu) / 4.0;
-    S T1 = 10.0 * Cc / (15.0 + 4.0 * fnu) * (k * k * eta) / (3.0 * k);
-    S N2 = -(k * k * eta * eta) / 15.0 * 1.0 / (1.0 + 2.0 / 5.0 * fnu) * Phi / 2.0;
-    if (lane == 0) {
-        const int iT = 2, iP = G.cB, iN = G.cC;
-        put(iT, T0);
-        put(iT + 1, T1);
-        S T2 = -8.0 * k / (15.0 * Hc * tp) * T1;
-        put(iT + 2, T2);
-        put(iP, (5.0 / 4.0) * T2);
-        S Pprev = -k / (4.0 * Hc * tp) * T2;
-        put(iP + 1, Pprev);
-        Pprev = (1.0 / 4.0) * T2;
-        put(iP + 2, Pprev);
-        S Tprev = T2;
-        for (int l = 3; l <= G.ng; ++l) {
-            Tprev = -(double)l / (2 * l + 1) * k / (Hc * tp) * Tprev;
-            Pprev = -(double)l / (2 * l + 1) * k / (Hc * tp) * Pprev;
-            put(iT + l, Tprev);
-            put(iP + l, Pprev);
-        }
-        S del = 3.0 / 4.0 * (4.0 * T0);
-        S v = -3.0 * k * T1;
-        put(iN, T0);
-        put(iN + 1, T1);
-        put(iN + 2, N2);
-        S Nprev = N2;
-        for (int l = 3; l <= G.nn; ++l) {
-            Nprev = k / ((2 * l + 1) * Hc) * Nprev;
-            put(iN + l, Nprev);
-        }
-        put(0, del);   // δ_b
-        put(1, v);     // v_b
-        put(G.cD, del);
-        put(G.cD + 1, v);
-        put(G.cE, Phi);
-    } else if (lane <= G.nq) {
-        int i = lane - 1;
-        S q, df0;
-        if constexpr (DU) { q = {W.q()[i], Wt->qd()[i]}; df0 = {W.df0()[i], Wt->df0d()[i]}; }
-        else { q = W.q()[i]; df0 = W.df0()[i]; }
-        S eps = sqrt(q * q + (ai * mnu) * (ai * mnu));
-        const int iM = G.cM + i * (G.nm + 1);
-        put(iM, -T0 * df0);
-        put(iM + 1, -eps / q * T1 * df0);
-        S Mprev = -N2 * df0;
-        put(iM + 2, Mprev);
-        for (int l = 3; l <= G.nm; ++l) {
-            Mprev = q / eps * k / ((2 * l + 1) * Hc) * Mprev;
-            put(iM + l, Mprev);
-        }
-    }
-}
-__device__ void initial_conditions(const CosmoDev& C, const Geo& G, const WS& W, double k, double* u,
-                                   const Thr& T) {
-    initial_conditions_t<double>(C, nullptr, G, W, nullptr, k, u, nullptr, T);
-}
-
-// ------------------------------------------------------------- KenCarp4 data
-__constant__ double KC_C[6] = {0.0, 0.5, 83.0 / 250.0, 31.0 / 50.0, 17.0 / 20.0, 1.0};
-#define KC_G 0.25
-// KenCarp4's A (rows = stages) and embedded weights b̂ (compile-time indices)
-struct KCT {
-    static constexpr double A[6][6] = {
-        {0, 0, 0, 0, 0, 0},
-        {0.25, 0, 0, 0, 0, 0},
-        {8611.0 / 62500.0, -1743.0 / 31250.0, 0, 0, 0, 0},
-        {5012029.0 / 34652500.0, -654441.0 / 2922500.0, 174375.0 / 388108.0, 0, 0, 0},
-        {15267082809.0 / 155376265600.0, -71443401.0 / 120774400.0, 730878875.0 / 902184768.0,
-         2285395.0 / 8070912.0, 0, 0},
-        {82889.0 / 524892.0, 0.0, 15625.0 / 83664.0, 69875.0 / 102672.0, -2260.0 / 8211.0, 0}};
-    static constexpr double BH[6] = {4586570599.0 / 29645900160.0, 0.0, 178811875.0 / 945068544.0,
-                                     814220225.0 / 1159782912.0, -3700637.0 / 11593932.0, 61727.0 / 225920.0};
-};
-
-// One pass after stage S's border solve: Z_S = w + hγ(c_S y₀ + c_P y₁ + c_Π y₂),
-// then the next stage's argument u + Σ_j a_{S+1,j} Z_j, or after the last stage
-// u_{n+1} (stiffly accurate) and the embedded error (into ψ, which no
-// wavefront reads any more; w still is).  The tableau is compile-time; two
-// rows per thread, every load before any store (past n, cc[1] repeats row c0
-// and is stored first).  Caller syncs.
-template <int S, bool ZDONE = false>
-__device__ inline void stage_combine(const Geo& G, const WS& W, double hg, const double* y, const Thr& T) {
-    // ZDONE: Z_S is already in place (the FP32 solve mode's refined stage value)
-    for (int c0 = T.tid; c0 < G.n; c0 += 2 * T.nt) {
-        const int c1 = c0 + T.nt;
-        const int cc[2] = {c0, c1 < G.n ? c1 : c0};
-        double z[2], a[2], e[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int c = cc[i];
-            if constexpr (ZDONE) z[i] = W.Z(S)[c];
-            else z[i] = W.w()[c] + hg * (W.cS()[c] * y[0] + W.cP()[c] * y[1] + W.cPi()[c] * y[2]);
-            double acc = W.u()[c], err = 0.0;
-#pragma unroll
-            for (int j = 0; j < S; ++j) {
-                const double zj = W.Z(j)[c];
-                if constexpr (S < 5) {
-                    acc += KCT::A[S + 1][j] * zj;
-                } else {
-                    acc += KCT::A[5][j] * zj;
-                    err += (KCT::A[5][j] - KCT::BH[j]) * zj;
-                }
-            }
-            if constexpr (S < 5) {
-                a[i] = acc + KCT::A[S + 1][S] * z[i];
-            } else {
-                a[i] = acc + KC_G * z[i];
-                e[i] = err + (KC_G - KCT::BH[5]) * z[i];
-            }
-        }
-#pragma unroll
-        for (int i = 1; i >= 0; --i) {
-            const int c = cc[i];
-            if constexpr (!ZDONE) W.Z(S)[c] = z[i];
-            if constexpr (S < 5) {
-                W.arg()[c] = a[i];
-            } else {
-                W.un()[c] = a[i];
-                W.arg()[c] = e[i];
-            }
-        }
-    }
-}
-
-// ---------------------------------------------------------------- kernels
-struct SolveArgs {
-    const CosmoDev* cosmos;
-    const CfgDev* cfgs;
-    const ModeDesc* modes;
-    int nmodes;
-    int* work_counter;
-    int out_mode;          // 0: save states at x_save; else bit 1: temperature source, bit 2: polarization
-                           // source, at every x node
-    const double* x_save;  // [nsave] sorted
-    int nsave;
-    double* out;           // mode 0: [out][nsave][n_state]; source modes: temperature [out][nx]
-    double* out2;          // polarization source [out][nx]
-    int* status;           // [out]
-    long long* counters;   // [out][4]: accepted, rejected, rhs evals, solves
-    int n_state_stride;    // n of the output layout (mode 0)
-    int lds_doubles;       // dynamic LDS of the launch, in doubles
-    // the tangent-linear solve: the cosmologies' tangent copies and the
-    // outputs' derivatives (same layout as out)
-    const CosmoDev* cosmos_dot = nullptr;
-    double* out_dot = nullptr;
-    // serving from a work queue the host fills while the launch runs: modes,
-    // cosmologies and configurations live in pinned host memory; published
-    // counts the modes written so far; a mode's ModeDesc pad is its output mode
-    // and out its output's offset from `out` in doubles; status and counters are
-    // indexed by the mode's queue position and done[position] receives `epoch`
-    // when the mode's outputs are in memory.  A workgroup leaves once closed is
-    // set, once drain equals the launch's epoch, or after idle_limit polls
-    // without work; the first to leave stores the epoch to leave (device
-    // memory), after which no workgroup of the launch claims another mode.
-    int serve = 0;
-    int epoch = 0;
-    int idle_limit = 0;
-    int poll_sleeps = 4;  // s_sleep 127 (~3.4 µs each) between polls
-    const int* published = nullptr;
-    const int* closed = nullptr;
-    const int* drain = nullptr;
-    int* leave = nullptr;
-    int* done = nullptr;
-};
-
-// the next published mode of a serving launch (queue position), or INT_MAX
-// once the queue is closed, the host drains this launch, no mode has arrived
-// for idle_limit polls, or another workgroup of the launch has left for one of
-// these reasons (the launch ends as a whole: a few workgroups left behind
-// never take a new request's modes on their own); one thread per workgroup.
-// Positions are claimed by compare-and-swap, so no position is taken before
-// the host has published it.  A poll reads host memory: poll_sleeps sleeps
-// between polls keep that traffic small.  The polls are relaxed loads: an acquire at system
-// scope invalidates the L2, which the workgroups still solving would pay for
-// at every poll of every idle workgroup; the caller's one acquire fence after
-// a claim orders what the host wrote before publishing.
-__device__ inline int serve_claim(const SolveArgs& A) {
-    for (int idle = 0;; ++idle) {
-        if (__hip_atomic_load(A.leave, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == A.epoch) return INT_MAX;
-        const bool stop = __hip_atomic_load(A.closed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) ||
-                          __hip_atomic_load(A.drain, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == A.epoch;
-        if (!stop) {
-            const int p = __hip_atomic_load(A.published, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            int c = __hip_atomic_load(A.work_counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            while (c < p) {
-                if (__hip_atomic_compare_exchange_strong(A.work_counter, &c, c + 1, __ATOMIC_RELAXED,
-                                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-                    return c;
-            }
-        }
-        if (stop || idle >= A.idle_limit) {
-            __hip_atomic_store(A.leave, A.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return INT_MAX;
-        }
-        for (int s = 0; s < A.poll_sleeps; ++s) __builtin_amdgcn_s_sleep(127);
-    }
-}
-
-
-// Σ over the workgroup, the same value in every thread: wavefront sums, then
-// the wavefront totals in a fixed order
-__device__ inline double block_sum(double v, const WS& W, const Thr& T) {
-    double s = wave_sum(v);
-    if (T.nt == WAVE) return s;
-    if (T.lane == 0) W.red()[T.wv] = s;
-    __syncthreads();
-    double tot = 0.0;
-    for (int w = 0; w < T.nt / WAVE; ++w) tot += W.red()[w];
-    __syncthreads();
-    return tot;
-}
-
-__device__ inline double wrms(const Geo& G, const WS& W, const double* e, const double* ua, const double* ub,
-                              double rt, double at, const Thr& T) {
-    double s = 0.0;
-    for (int c = T.tid; c < G.n; c += T.nt) {
-        double sc = at + rt * fmax(fabs(ua[c]), fabs(ub[c]));
-        double r = e[c] / sc;
-        s += r * r;
-    }
-    s = block_sum(s, W, T);
-    return sqrt(s / G.n);
-}
-
-
-// output at the node/save point xv from the interval (xa, ua, fa) .. (xb, ub, fb)
-__device__ inline void emit(const CosmoDev& C, const Geo& G, const WS& W, const SolveArgs& A, int out,
-                                  double k, double xa, const double* ua, const double* fa, double xb,
-                                  const double* ub, const double* fb, double xv, int idx, const Thr& T,
-                                  int om, double* obase) {
-    // om: the output mode (A.out_mode, or the mode's own when serving); obase:
-    // a serving mode's output, or nullptr for the launch's own layout
-    double h = xb - xa;
-    if (h == 0.0) {
-        for (int c = T.tid; c < G.n; c += T.nt) W.arg()[c] = ua[c];
-    } else {
-        double th = (xv - xa) / h;
-        for (int c = T.tid; c < G.n; c += T.nt) {
-            double v;
-            if (th == 1.0) v = ub[c];
-            else {
-                double dd = ub[c] - ua[c];
-                v = (1.0 - th) * ua[c] + th * ub[c] +
-                    th * (th - 1.0) * ((1.0 - 2.0 * th) * dd + (th - 1.0) * h * fa[c] + th * h * fb[c]);
-            }
-            W.arg()[c] = v;
-        }
-    }
-    if (om == 0) {
-        double* dst = obase ? obase + (size_t)idx * G.n : A.out + ((size_t)out * A.nsave + idx) * A.n_state_stride;
-        for (int c = T.tid; c < G.n; c += T.nt) dst[chain_to_state(G, c)] = W.arg()[c];
-        return;
-    }
-    // sources at a grid node: hierarchy!(du, u) (mutating u, spectra.jl:16, 36)
-    // on the rows source_function reads, then source_function and/or
-    // source_function_P
-    const bool want_t = (om & 1) != 0, want_p = (om & 2) != 0;
-    XC X = make_xc(C, k, xv);
-    qfill(C, G, X, W, T);
-    __syncthreads();
-    Fun F = functionals(C, G, X, W.qcur(), W.arg(), T);
-    if (want_t && T.wv == 0) {
-        int c = source_row(G, T.lane);
-        if (c >= 0) {
-            W.w()[c] = row_eval(G, W, W.kcur(), W.arg(), c, G.n, F.S, F.P, F.Pi);
-        }
-    }
-    __syncthreads();
-    if (X.rsa && T.tid == 0) rsa_mutate(G, X, k, W.arg(), F.P);
-    __syncthreads();
-    if (want_t && T.wv == 0) {
-        double s = source_fn(C, G, X, W, k, W.arg(), W.w(), F.P, T.lane);
-        if (T.lane == 0) (obase ? obase + idx : A.out + (size_t)out * C.nx + idx)[0] = s;
-    }
-    if (want_p && T.tid == T.nt - 1) A.out2[(size_t)out * C.nx + idx] = source_fn_P(C, G, X, k, W.arg());
-    __syncthreads();
-}
-
-// emit with the tangent: the Hermite interpolant of (u̇, ḟ) beside that of
-// (u, f); saved states or the temperature source and their derivatives
-__device__ inline void emit_tan(const CosmoDev& C, const CosmoDev& Cd, const Geo& G, const WS& W, const WTan& Wt,
-                                const SolveArgs& A, int out, double k, double xa, const double* ua,
-                                const double* fa, const double* uda, const double* fda, double xb, const double* ub,
-                                const double* fb, const double* udb, const double* fdb, double xv, int idx,
-                                const Thr& T) {
-    const double h = xb - xa;
-    const double th = h == 0.0 ? 0.0 : (xv - xa) / h;
-    for (int c = T.tid; c < G.n; c += T.nt) {
-        double v, vd;
-        if (h == 0.0) {
-            v = ua[c]; vd = uda[c];
-        } else if (th == 1.0) {
-            v = ub[c]; vd = udb[c];
-        } else {
-            const double dd = ub[c] - ua[c], ddd = udb[c] - uda[c];
-            v = (1.0 - th) * ua[c] + th * ub[c] +
-                th * (th - 1.0) * ((1.0 - 2.0 * th) * dd + (th - 1.0) * h * fa[c] + th * h * fb[c]);
-            vd = (1.0 - th) * uda[c] + th * udb[c] +
-                 th * (th - 1.0) * ((1.0 - 2.0 * th) * ddd + (th - 1.0) * h * fda[c] + th * h * fdb[c]);
-        }
-        W.arg()[c] = v;
-        Wt.argd()[c] = vd;
-    }
-    if (A.out_mode == 0) {
-        const size_t o = ((size_t)out * A.nsave + idx) * A.n_state_stride;
-        for (int c = T.tid; c < G.n; c += T.nt) {
-            A.out[o + chain_to_state(G, c)] = W.arg()[c];
-            A.out_dot[o + chain_to_state(G, c)] = Wt.argd()[c];
-        }
-        return;
-    }
-    const XC X = make_xc(C, k, xv);
-    qfill(C, G, X, W, T);
-    const XCd D = make_xcd(C, Cd, X);
-    if (T.tid < G.nq) qfill_one_dot(C, Cd, W, Wt, X.a, X.kH, D.kH, W.qe(), Wt.qset_base(5), Wt.ktd(5), T.tid);
-    if (T.tid == T.nt - 1) ktab_head_dot(Wt.ktd(5), X, D);
-    __syncthreads();
-    Fun F1, F0;
-    FunD P0;
-    functionals_tan(C, Cd, G, X, D, W.qcur(), Wt.qset(5), Wt.argd(), W.arg(), T, F1, F0, P0);
-    if (T.wv == 0) {
-        const int c = source_row(G, T.lane);
-        if (c >= 0) {
-            W.w()[c] = row_eval(G, W, W.kcur(), W.arg(), c, G.n, F0.S, F0.P, F0.Pi);
-            Wt.wd()[c] = row_eval(G, W, W.kcur(), Wt.argd(), c, G.n, F1.S, F1.P, F1.Pi) +
-                         row_eval_p(G, W, W.kcur(), Wt.ktd(5), W.arg(), c, G.n, F0, P0);
-        }
-    }
-    __syncthreads();
-    const D1 Phip = {F0.P, F1.P + P0.P};
-    if (X.rsa && T.tid == 0) rsa_mutate_t<D1>(G, X, &D, k, W.arg(), Wt.argd(), Phip);
-    __syncthreads();
-    if (T.wv == 0) {
-        const QSet Qd = Wt.qset(5);
-        const D1 sv = source_fn_t<D1>(C, &Cd, G, X, &D, W, &Qd, k, W.arg(), Wt.argd(), W.w(), Wt.wd(), Phip, T.lane);
-        if (T.lane == 0) {
-            A.out[(size_t)out * C.nx + idx] = sv.v;
-            A.out_dot[(size_t)out * C.nx + idx] = sv.d;
-        }
-    }
-    __syncthreads();
-}
-
-// the tangent of stage S after its solve (w̃ = W⁻¹ r̃ banded, y = K⁻¹ D w̃):
-// Ż_S = w̃ + hγ(c_S y₀ + c_P y₁ + c_Π y₂), then the next stage's argument
-// tangent, or after the last stage u̇ₙ₊₁.  Caller syncs.
-template <int S>
-__device__ inline void stage_combine_tan(const Geo& G, const WS& W, const WTan& Wt, double hg, const double* y,
-                                         const Thr& T) {
-    for (int c = T.tid; c < G.n; c += T.nt) {
-        const double z = Wt.wd()[c] + hg * (W.cS()[c] * y[0] + W.cP()[c] * y[1] + W.cPi()[c] * y[2]);
-        Wt.Zd(S)[c] = z;
-        double acc = Wt.ud()[c];
-        if constexpr (S < 5) {
-#pragma unroll
-            for (int j = 0; j < S; ++j) acc += KCT::A[S + 1][j] * Wt.Zd(j)[c];
-            Wt.argd()[c] = acc + KCT::A[S + 1][S] * z;
-        } else {
-#pragma unroll
-            for (int j = 0; j < 5; ++j) acc += KCT::A[5][j] * Wt.Zd(j)[c];
-            Wt.und()[c] = acc + KC_G * z;
-        }
-    }
-}
-
-// one workgroup of NWAVE wavefronts per k-mode
-template <int SR, bool F32, bool TAN = false>
-__global__ void __launch_bounds__(NTHR) k_boltsolve(SolveArgs A) {
-    // F32: the FP32 solve mode -- factors and substitutions in FP32, each stage
-    // value refined against the FP64 residual of its stage equation.
-    // TAN: the tangent-linear solve -- u̇ along the primal's steps, each stage's
-    // tangent (I − hγL)Ż = h(L ȧrg + L̇(arg + γZ)) solved with the primal's
-    // factors and border; outputs and their derivatives
-    static_assert(!(F32 && TAN), "the tangent solve runs in FP64");
-    using P = typename std::conditional<F32, float, double>::type;
-    extern __shared__ double lds[];
-    __shared__ int s_mode;
-    const Thr T = thr_self();
-    for (;;) {
-        if (T.tid == 0) {
-            if (A.serve) {
-                const int c = serve_claim(A);
-                // what the host wrote before publishing (tables, descriptors) is
-                // read fresh after this: system-scope acquire
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
-                s_mode = c;
-            } else {
-                s_mode = atomicAdd(A.work_counter, 1);
-            }
-        }
-        __syncthreads();
-        const int mi = s_mode;
-        if (mi >= A.nmodes) return;
-#ifdef BOLT_DEBUG_NANFILL
-        // debug build: each mode starts from a workspace full of NaNs, so a read
-        // of anything this mode has not written itself shows as a wrong value
-        for (int i = T.tid; i < A.lds_doubles; i += T.nt) lds[i] = __builtin_nan("");
-        __syncthreads();
-#endif
-        ModeDesc md = A.modes[mi];
-        const CosmoDev C = A.cosmos[md.cosmo];
-        const CfgDev cf = A.cfgs[md.cfg];
-        Geo G = make_geo(cf);
-        WS W;
-        ws_bind(W, lds, G.n, G.nq);
-        const double k = md.k;
-        WTan Wt;
-        const CosmoDev* Cdp = nullptr;
-        if constexpr (TAN) {
-            Wt.b = lds + wtan_offset(G.n, G.nq);
-            Wt.n = G.n;
-            Wt.nq = G.nq;
-            Cdp = A.cosmos_dot + md.cosmo;
-            if (T.tid < G.nq) {
-                Wt.qd()[T.tid] = Cdp->qv[T.tid]; Wt.df0d()[T.tid] = Cdp->df0[T.tid]; Wt.based()[T.tid] = Cdp->base[T.tid];
-            }
-            for (int c = T.tid; c < G.n; c += T.nt) Wt.ud()[c] = 0.0;
-        }
-        if (T.tid < G.nq) { W.q()[T.tid] = C.qv[T.tid]; W.df0()[T.tid] = C.df0[T.tid]; W.base()[T.tid] = C.base[T.tid]; }
-        for (int c = T.tid; c < G.n; c += T.nt) W.u()[c] = 0.0;
-        setup_rows(C, G, W, T);
-        __syncthreads();
-        if constexpr (TAN) initial_conditions_t<D1>(C, Cdp, G, W, &Wt, k, W.u(), Wt.ud(), T);
-        else initial_conditions(C, G, W, k, W.u(), T);
-        __syncthreads();
-        long long nacc = 0, nrej = 0, nrhs = 0, nsol = 0;
-        double x = C.x0, xend = C.x1;
-        const double rt = cf.reltol, at = cf.abstol;
-        const int nref = (cf.flags & BOLT_CFG_REFINE_MASK) ? (cf.flags & BOLT_CFG_REFINE_MASK) >> 4 : 12;
-        int status = BOLT_MODE_OK;
-        int next = 0;  // next output index
-        const int om = A.serve ? md.pad : A.out_mode;
-        double* const obase = A.serve ? A.out + (size_t)(unsigned)md.out : nullptr;
-        const int nout = (om == 0) ? A.nsave : C.nx;
-        // outputs at the starting point take the initial condition as saved
-        while (next < nout) {
-            double xv = (om == 0) ? A.x_save[next] : node_x(C, next);
-            if (!(xv <= x)) break;
-            if constexpr (TAN)
-                emit_tan(C, *Cdp, G, W, Wt, A, md.out, k, x, W.u(), W.u(), Wt.ud(), Wt.ud(), x, W.u(), W.u(), Wt.ud(),
-                         Wt.ud(), xv, next, T);
-            else
-                emit(C, G, W, A, md.out, k, x, W.u(), W.u(), x, W.u(), W.u(), xv, next, T, om, obase);
-            ++next;
-        }
-        // FSAL start: f(u0) (the RSA overwrite, if on, persists in u)
-        {
-            XC X = make_xc(C, k, x);
-            qfill(C, G, X, W, T);
-            XCd D;
-            if constexpr (TAN) {
-                D = make_xcd(C, *Cdp, X);
-                if (T.tid < G.nq) qfill_one_dot(C, *Cdp, W, Wt, X.a, X.kH, D.kH, W.qe(), Wt.qset_base(5), Wt.ktd(5), T.tid);
-                if (T.tid == T.nt - 1) ktab_head_dot(Wt.ktd(5), X, D);
-            }
-            __syncthreads();
-            Fun F = rhs_rows(C, G, X, W, W.qcur(), W.kcur(), W.u(), 1.0, W.f(), false, T);
-            ++nrhs;
-            Fun Fd;
-            if constexpr (TAN) {
-                Fd = rhs_rows_tan(C, *Cdp, G, X, D, W, W.qcur(), Wt.qset(5), W.kcur(), Wt.ktd(5), Wt.ud(), W.u(), 1.0,
-                                  Wt.fd(), T);
-                ++nrhs;
-            }
-            __syncthreads();
-            if constexpr (TAN) {
-                if (X.rsa && T.tid == 0) rsa_mutate_t<D1>(G, X, &D, k, W.u(), Wt.ud(), D1{F.P, Fd.P});
-            } else {
-                if (X.rsa && T.tid == 0) rsa_mutate(G, X, k, W.u(), F.P);
-            }
-            __syncthreads();
-        }
-        // Hairer's starting step (order 4)
-        double h;
-        {
-            double d0 = wrms(G, W, W.u(), W.u(), W.u(), rt, at, T);
-            double d1 = wrms(G, W, W.f(), W.u(), W.u(), rt, at, T);
-            double h0 = (d0 < 1e-5 || d1 < 1e-5) ? 1e-6 : 0.01 * d0 / d1;
-            if (h0 > xend - x) h0 = xend - x;
-            for (int c = T.tid; c < G.n; c += T.nt) W.arg()[c] = W.u()[c] + h0 * W.f()[c];
-            XC X1 = make_xc(C, k, x + h0);
-            qfill(C, G, X1, W, T);
-            __syncthreads();
-            rhs_rows(C, G, X1, W, W.qcur(), W.kcur(), W.arg(), 1.0, W.w(), false, T);
-            ++nrhs;
-            __syncthreads();
-            for (int c = T.tid; c < G.n; c += T.nt) W.w()[c] -= W.f()[c];
-            double d2 = wrms(G, W, W.w(), W.u(), W.u(), rt, at, T) / h0;
-            double dm = fmax(d1, d2);
-            double h1 = (dm <= 1e-15) ? fmax(1e-6, h0 * 1e-3) : pow(0.01 / dm, 1.0 / 5.0);
-            h = fmin(100.0 * h0, h1);
-            if (h > xend - x) h = xend - x;
-        }
-        const int maxsteps = cf.max_steps > 0 ? cf.max_steps : 100000;
-        long long nsteps = 0;
-        bool take = false;  // the last attempt was accepted
-        while (x < xend) {
-            if (++nsteps > maxsteps) { status = BOLT_MODE_MAXSTEPS; break; }
-            bool last = false;
-            if (h >= xend - x) { h = xend - x; last = true; }
-            const double hg = h * KC_G;
-            // Z₀ = h f(u) and the first stage's argument; after an accepted
-            // step this pass also moves u_{n+1}, f_{n+1} into u, f (each thread
-            // copies and reads only its own rows)
-            for (int c = T.tid; c < G.n; c += T.nt) {
-                double uc, fc;
-                if (take) {
-                    uc = W.un()[c]; fc = W.fn()[c];
-                    W.u()[c] = uc; W.f()[c] = fc;
-                } else {
-                    uc = W.u()[c]; fc = W.f()[c];
-                }
-                const double z0 = h * fc;
-                W.Z(0)[c] = z0;
-                W.arg()[c] = uc + KCT::A[1][0] * z0;
-                if constexpr (TAN) {
-                    double udc, fdc;
-                    if (take) {
-                        udc = Wt.und()[c]; fdc = Wt.fnd()[c];
-                        Wt.ud()[c] = udc; Wt.fd()[c] = fdc;
-                    } else {
-                        udc = Wt.ud()[c]; fdc = Wt.fd()[c];
-                    }
-                    const double zd0 = h * fdc;
-                    Wt.Zd(0)[c] = zd0;
-                    Wt.argd()[c] = udc + KCT::A[1][0] * zd0;
-                }
-            }
-            take = false;
-            // the five implicit stage points depend on x and h only: their
-            // coefficients, q-quantities, W bands and LU come first, all stages
-            // at once
-            // lanes 0..4: each stage point's coefficients; wavefronts 1..3 at
-            // the same time: the q-sets, from a = e^x and kH = k/ℋ formed
-            // exactly as make_xc forms them
-            if (T.tid < 5) {
-                const XC Xs = make_xc(C, k, x + KC_C[T.tid + 1] * h);
-                store_xc(W.xcs(T.tid), Xs);
-                ktab_head(W.ktab(T.tid), Xs);
-                if constexpr (TAN) {
-                    const XCd Ds = make_xcd(C, *Cdp, Xs);
-                    store_xcd(Wt.xcd(T.tid), Ds);
-                    ktab_head_dot(Wt.ktd(T.tid), Xs, Ds);
-                }
-            } else if (T.wv > 0) {
-                for (int t = T.tid - WAVE; t < 5 * G.nq; t += T.nt - WAVE) {
-                    const int st = t / G.nq;
-                    const double xs = x + KC_C[st + 1] * h;
-                    const double Hs = spl(C, BOLT_T_HC, xs);
-                    const double kHs = k * rcp(Hs);
-                    const double as = exp(xs);
-                    qfill_one(C, W, as, kHs, W.qst_base(st), W.ktab(st), t - st * G.nq);
-                    if constexpr (TAN) {
-                        const double kHsd = -kHs * (spl(*Cdp, BOLT_T_HC, xs) / Hs);
-                        qfill_one_dot(C, *Cdp, W, Wt, as, kHs, kHsd, W.qst_base(st), Wt.qset_base(st), Wt.ktd(st),
-                                      t - st * G.nq);
-                    }
-                }
-            }
-            __syncthreads();
-            stage_bands<P>(G, W, hg, T);
-            __syncthreads();
-            // the LU of the five stage points on wavefront 0 while the others
-            // form stage 1's right-hand side and border columns (which need
-            // no factor)
-            if (T.wv == 0) {
-                chain_factor_all<P>(G, W, T.lane);
-            } else {
-                Thr Tr = T;
-                Tr.tid -= WAVE;
-                Tr.nt -= WAVE;
-                rhs_rows(C, G, load_xc(W.xcs(0)), W, W.qst(0), W.ktab(0), W.arg(), h, W.w(), true, Tr,
-                         F32 ? W.rvec() : nullptr);
-            }
-            ++nrhs;
-            __syncthreads();
-            Cap K;
-            XC Xs;
-            for (int s = 1; s < 6; ++s) {
-                Xs = load_xc(W.xcs(s - 1));
-                const QSet Qs = W.qst(s - 1);
-                // rhs = h f(ψ) and the border columns (stage 1's are formed above)
-                if (s > 1) {
-                    rhs_rows(C, G, Xs, W, Qs, W.ktab(s - 1), W.arg(), h, W.w(), true, T, F32 ? W.rvec() : nullptr);
-                    ++nrhs;
-                    __syncthreads();
-                }
-                chain_solve4<SR, P>(G, W, s - 1, T);
-                ++nsol;
-                // no barrier: wavefront r's border functionals read only the
-                // vector it has just solved (ordered by wave_lds_sync)
-                double y[3];
-                K = stage_border(C, G, Xs, W, Qs, hg, T, y);
-                if constexpr (F32) {
-                    // Z_s from the FP32 solve, then sweeps of iterative
-                    // refinement: the FP64 residual ρ = r − Z + γ·h·A·Z of the
-                    // stage equation (I − hγA)Z = r, its correction through the
-                    // same FP32 factors and border, Z += δ
-                    for (int c = T.tid; c < G.n; c += T.nt)
-                        W.Z(s)[c] = W.w()[c] + hg * (W.cS()[c] * y[0] + W.cP()[c] * y[1] + W.cPi()[c] * y[2]);
-                    __syncthreads();
-                    for (int it = 0; it < nref; ++it) {
-                        // ρ = r − Z + γ·(h·A·Z)
-                        rhs_rows(C, G, Xs, W, Qs, W.ktab(s - 1), W.Z(s), h, W.w(), false, T);
-                        for (int c = T.tid; c < G.n; c += T.nt)
-                            W.w()[c] = (W.rvec()[c] - W.Z(s)[c]) + KC_G * W.w()[c];
-                        ++nrhs;
-                        __syncthreads();
-                        if (T.wv == 0) {
-                            wave_subst<SR>(W.bandsT<P>(s - 1), G.n, W.w(), W.dump(), T.lane);
-                            const Fun Fc = functionals(C, G, Xs, Qs, W.w(), T);
-                            if (T.lane == 0) { W.red()[12] = Fc.S; W.red()[13] = Fc.P; W.red()[14] = Fc.Pi; }
-                        }
-                        ++nsol;
-                        __syncthreads();
-                        const double rc[3] = {W.red()[12], W.red()[13], W.red()[14]};
-                        double yc[3];
-                        solve3(K, rc, yc);
-                        // excess of each correction over 1e-14 of its own component
-                        double ex = 0.0;
-                        for (int c = T.tid; c < G.n; c += T.nt) {
-                            const double d = W.w()[c] + hg * (W.cS()[c] * yc[0] + W.cP()[c] * yc[1] +
-                                                              W.cPi()[c] * yc[2]);
-                            const double z = W.Z(s)[c] + d;
-                            W.Z(s)[c] = z;
-                            ex = fmax(ex, fabs(d) - 1e-14 * fabs(z));
-                        }
-                        ex = wave_max(ex);
-                        if (T.lane == 0) W.red()[16 + T.wv] = ex;
-                        __syncthreads();
-                        // converged once every correction is below 1e-14 of its component (every
-                        // thread reads the same four maxima, so all leave together; components
-                        // below FP32's range get no correction and count as converged).  A
-                        // stage still unconverged after the last sweep (the FP32 factors' error
-                        // times the stage matrix's condition number near one) is taken as it
-                        // stands: its error enters the step's error estimate
-                        const double* m = W.red();
-                        if (!(fmax(fmax(m[16], m[17]), fmax(m[18], m[19])) > 1e-290)) break;
-                    }
-                    switch (s) {
-                        case 1: stage_combine<1, true>(G, W, hg, y, T); break;
-                        case 2: stage_combine<2, true>(G, W, hg, y, T); break;
-                        case 3: stage_combine<3, true>(G, W, hg, y, T); break;
-                        case 4: stage_combine<4, true>(G, W, hg, y, T); break;
-                        default: stage_combine<5, true>(G, W, hg, y, T); break;
-                    }
-                } else if constexpr (TAN) {
-                    // Z_s, and the stage value arg + γZ_s into w (which nothing reads any more)
-                    for (int c = T.tid; c < G.n; c += T.nt) {
-                        const double z = W.w()[c] + hg * (W.cS()[c] * y[0] + W.cP()[c] * y[1] + W.cPi()[c] * y[2]);
-                        W.Z(s)[c] = z;
-                        W.w()[c] = W.arg()[c] + KC_G * z;
-                    }
-                    __syncthreads();
-                    // r̃ = h(f(ȧrg) + L̇(arg + γZ_s)) at the stage point
-                    rhs_rows_tan(C, *Cdp, G, Xs, load_xcd(Wt.xcd(s - 1)), W, Qs, Wt.qset(s - 1), W.ktab(s - 1),
-                                 Wt.ktd(s - 1), Wt.argd(), W.w(), h, Wt.wd(), T);
-                    ++nrhs;
-                    __syncthreads();
-                    // wavefront 0 solves it with the stage's factors while the others
-                    // form the primal's next argument
-                    if (T.wv == 0) {
-                        wave_subst<SR>(W.bandsT<double>(s - 1), G.n, Wt.wd(), W.dump(), T.lane);
-                        const Fun Fc = functionals(C, G, Xs, Qs, Wt.wd(), T);
-                        if (T.lane == 0) { W.red()[12] = Fc.S; W.red()[13] = Fc.P; W.red()[14] = Fc.Pi; }
-                    } else {
-                        Thr Tr = T;
-                        Tr.tid -= WAVE;
-                        Tr.nt -= WAVE;
-                        switch (s) {
-                            case 1: stage_combine<1, true>(G, W, hg, y, Tr); break;
-                            case 2: stage_combine<2, true>(G, W, hg, y, Tr); break;
-                            case 3: stage_combine<3, true>(G, W, hg, y, Tr); break;
-                            case 4: stage_combine<4, true>(G, W, hg, y, Tr); break;
-                            default: stage_combine<5, true>(G, W, hg, y, Tr); break;
-                        }
-                    }
-                    ++nsol;
-                    __syncthreads();
-                    const double rc[3] = {W.red()[12], W.red()[13], W.red()[14]};
-                    double yt[3];
-                    solve3(K, rc, yt);
-                    switch (s) {
-                        case 1: stage_combine_tan<1>(G, W, Wt, hg, yt, T); break;
-                        case 2: stage_combine_tan<2>(G, W, Wt, hg, yt, T); break;
-                        case 3: stage_combine_tan<3>(G, W, Wt, hg, yt, T); break;
-                        case 4: stage_combine_tan<4>(G, W, Wt, hg, yt, T); break;
-                        default: stage_combine_tan<5>(G, W, Wt, hg, yt, T); break;
-                    }
-                } else {
-                    switch (s) {
-                        case 1: stage_combine<1>(G, W, hg, y, T); break;
-                        case 2: stage_combine<2>(G, W, hg, y, T); break;
-                        case 3: stage_combine<3>(G, W, hg, y, T); break;
-                        case 4: stage_combine<4>(G, W, hg, y, T); break;
-                        default: stage_combine<5>(G, W, hg, y, T); break;
-                    }
-                }
-                __syncthreads();
-            }
-            // Shampine's smoothed estimate: W⁻¹ e with the last stage's W, on
-            // wavefront 0.  Meanwhile the other wavefronts evaluate the FSAL
-            // derivative f(u_{n+1}) at x + h, which is the last stage point
-            // (abscissa 1): its coefficients, q-set and scalar table serve.
-            // It is used only if the step is accepted; a step cut to end on
-            // xend evaluates it at xend after acceptance instead.
-            const bool spec = !last;
-            Fun Fn;
-            if (T.wv == 0) {
-                chain_solve1<SR, P>(G, W, 4, W.arg(), T);
-            } else if (spec) {
-                Thr Tf = T;
-                Tf.tid -= WAVE;
-                Tf.nt -= WAVE;
-                Fn = rhs_rows(C, G, load_xc(W.xcs(4)), W, W.qst(4), W.ktab(4), W.un(), 1.0, W.fn(), false, Tf);
-            }
-            ++nsol;
-            if (spec) ++nrhs;
-            __syncthreads();
-            // the border step of the error solve folded into its norm:
-            // e_c = ψ_c + hγ(c_S y₀ + c_P y₁ + c_Π y₂) is formed and weighted
-            // row by row, never stored
-            double en;
-            {
-                const Fun Fe = functionals(C, G, Xs, W.qst(4), W.arg(), T);
-                double r[3] = {Fe.S, Fe.P, Fe.Pi}, ye[3];
-                solve3(K, r, ye);
-                double ss = 0.0;
-                for (int c = T.tid; c < G.n; c += T.nt) {
-                    const double e = W.arg()[c] + hg * (W.cS()[c] * ye[0] + W.cP()[c] * ye[1] + W.cPi()[c] * ye[2]);
-                    const double sc = at + rt * fmax(fabs(W.u()[c]), fabs(W.un()[c]));
-                    const double q = e / sc;
-                    ss += q * q;
-                }
-                en = sqrt(block_sum(ss, W, T) / G.n);
-            }
-            if (!isfinite(en)) {
-                ++nrej;
-                h *= 0.2;
-                if (h < 1e-14) { status = BOLT_MODE_NONFINITE; break; }
-                continue;
-            }
-            if (en <= 1.0) {
-                double xn = last ? xend : x + h;
-                // FSAL at x_{n+1} (already evaluated unless the step ends on xend)
-                XC Xn;
-                if (spec) {
-                    Xn = load_xc(W.xcs(4));
-                } else {
-                    Xn = make_xc(C, k, xn);
-                    qfill(C, G, Xn, W, T);
-                    __syncthreads();
-                    Fn = rhs_rows(C, G, Xn, W, W.qcur(), W.kcur(), W.un(), 1.0, W.fn(), false, T);
-                    ++nrhs;
-                    __syncthreads();
-                }
-                // Fn is held by wavefronts 1.. in both cases
-                if constexpr (TAN) {
-                    // ḟ(u̇ₙ₊₁) at xₙ₊₁ before the RSA write, from the last stage point's
-                    // tangent tables or the current x's
-                    XCd Dn;
-                    const double *Kn, *Kdn;
-                    QSet Qn, Qdn;
-                    if (spec) {
-                        Dn = load_xcd(Wt.xcd(4));
-                        Kn = W.ktab(4); Kdn = Wt.ktd(4); Qn = W.qst(4); Qdn = Wt.qset(4);
-                    } else {
-                        Dn = make_xcd(C, *Cdp, Xn);
-                        if (T.tid < G.nq)
-                            qfill_one_dot(C, *Cdp, W, Wt, Xn.a, Xn.kH, Dn.kH, W.qe(), Wt.qset_base(5), Wt.ktd(5), T.tid);
-                        if (T.tid == T.nt - 1) ktab_head_dot(Wt.ktd(5), Xn, Dn);
-                        __syncthreads();
-                        Kn = W.kcur(); Kdn = Wt.ktd(5); Qn = W.qcur(); Qdn = Wt.qset(5);
-                    }
-                    const Fun Fnd = rhs_rows_tan(C, *Cdp, G, Xn, Dn, W, Qn, Qdn, Kn, Kdn, Wt.und(), W.un(), 1.0,
-                                                 Wt.fnd(), T);
-                    ++nrhs;
-                    __syncthreads();
-                    if (Xn.rsa && T.wv == 1 && T.lane == 0)
-                        rsa_mutate_t<D1>(G, Xn, &Dn, k, W.un(), Wt.und(), D1{Fn.P, Fnd.P});
-                } else {
-                    if (Xn.rsa && T.wv == 1 && T.lane == 0) rsa_mutate(G, Xn, k, W.un(), Fn.P);
-                }
-                __syncthreads();
-                ++nacc;
-                while (next < nout) {
-                    double xv = (om == 0) ? A.x_save[next] : node_x(C, next);
-                    if (!(xv <= xn)) break;
-                    if constexpr (TAN)
-                        emit_tan(C, *Cdp, G, W, Wt, A, md.out, k, x, W.u(), W.f(), Wt.ud(), Wt.fd(), xn, W.un(), W.fn(),
-                                 Wt.und(), Wt.fnd(), xv, next, T);
-                    else
-                        emit(C, G, W, A, md.out, k, x, W.u(), W.f(), xn, W.un(), W.fn(), xv, next, T, om, obase);
-                    ++next;
-                }
-                take = true;  // u, f <- u_{n+1}, f_{n+1} in the next step's first pass
-                x = xn;
-                double fac = (en == 0.0) ? 10.0 : 0.9 * pow(en, -0.25);
-                fac = fmin(10.0, fmax(0.2, fac));
-                h *= fac;
-            } else {
-                ++nrej;
-                double fac = fmin(1.0, fmax(0.2, 0.9 * pow(en, -0.25)));
-                h *= fac;
-                if (h < 1e-14 * fmax(1.0, fabs(x))) { status = BOLT_MODE_DTMIN; break; }
-            }
-        }
-        if (T.tid == 0) {
-            const int si = A.serve ? mi : md.out;
-            A.status[si] = status;
-            if (A.counters) {
-                long long* cc = A.counters + (size_t)si * 4;
-                cc[0] = nacc; cc[1] = nrej; cc[2] = nrhs; cc[3] = nsol;
-            }
-            if (A.serve) {
-                // the workgroup's outputs (ordered before this thread by the
-                // barrier above) reach memory, then the host's flag is raised
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-                __hip_atomic_store(A.done + mi, A.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
-        }
-        __syncthreads();
-    }
-}
+#include "solve_layout.h"
 
 // hierarchy! parity hook: one wavefront per mode, u/du [n][B]
 __global__ void __launch_bounds__(WAVE) k_rhs(const CosmoDev* cosmos, const CfgDev* cfgs, const ModeDesc* modes,
@@ -3152,6 +950,10 @@ struct bolt_ctx {
     std::mutex server_mu;
 };
 
+// LDS of one workgroup of the solver: the FP64 kernel's own layout is the
+// smaller one except for short states with many momentum bins
+static size_t solve_lds(int n, int nq) { return std::max(ws_bytes(n, nq), wsn_bytes(wsn_layout(n, nq))); }
+
 static int check_cfg(const bolt_hier_cfg* c) {
     if (!c) return set_error(BOLT_E_ARG, "cfg is NULL");
     if (c->ell_g < 3 || c->ell_nu < 2 || c->ell_mnu < 2 || c->nq < 1 || c->nq > 48)
@@ -3251,9 +1053,11 @@ int bolt_ctx_create(int device, bolt_ctx** out) {
         int lds_max = (int)prop.sharedMemPerBlockOptin > 0 ? (int)prop.sharedMemPerBlockOptin
                                                             : (int)prop.sharedMemPerBlock;
         c->lds_max = lds_max - 1024;  // headroom for static __shared__
-        for (const void* f : {(const void*)k_boltsolve<5, false>, (const void*)k_boltsolve<6, false>,
-                              (const void*)k_boltsolve<7, false>, (const void*)k_boltsolve<8, false>,
-                              (const void*)k_boltsolve<SR_DEFAULT, true>, (const void*)k_boltsolve<SR_DEFAULT, false, true>,
+        for (int sr = SR_RUN_MIN; sr <= SR_MAX; ++sr)
+            for (int layout = 0; layout < WSN_LAYOUTS; ++layout)
+                (void)hipFuncSetAttribute(solver_kernel(sr, layout), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                          c->lds_max);
+        for (const void* f : {boltsolve_kernel(false), boltsolve_kernel(true),
                               (const void*)k_rhs, (const void*)k_ics, (const void*)k_rhs_jvp, (const void*)k_ics_jvp})
             (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_max);
         (void)hipGetLastError();  // an unsupported opt-in must not surface at the next launch check
@@ -3303,11 +1107,9 @@ int bolt_ws_layout(int n, int nq, int fp32, int cap, long long* regions, int* nr
                    long long* total_bytes, long long* read_reach) {
     if (n < 1 || nq < 1 || cap < 0 || !regions || !nregions || !dump_off || !total_bytes || !read_reach)
         return set_error(BOLT_E_ARG, "bad workspace layout query");
-    const size_t tot = ws_bytes(n, nq);
+    const size_t tot = fp32 ? ws_bytes(n, nq) : solve_lds(n, nq);
     std::vector<double> mem(tot / sizeof(double) + 1);
-    WS W;
-    ws_bind(W, mem.data(), n, nq);
-    const char* b0 = (const char*)W.b;
+    const char* b0 = (const char*)mem.data();
     int cnt = 0;
     auto add = [&](const void* p, size_t bytes) {
         if (cnt < cap) {
@@ -3317,6 +1119,37 @@ int bolt_ws_layout(int n, int nq, int fp32, int cap, long long* regions, int* nr
         ++cnt;
     };
     const size_t vb = sizeof(double) * (size_t)n, qb = sizeof(double) * (size_t)nq;
+    if (!fp32) {  // k_solve's layout: every read past n stays in its vector's padding
+        auto regions_of = [&](auto N) {
+            using L = decltype(N);
+            N.b = mem.data();
+            N.n = n;
+            N.nq = nq;
+            for (int i = 0; i < L::NV; ++i) add(N.vec(i), sizeof(double) * L::ns);
+            add(N.tail(), sizeof(double) * 10 * CB);
+            for (int st = 0; st < 5; ++st) add(N.xcs(st), sizeof(double) * NXC);
+            add(N.red(), sizeof(double) * 15); add(N.red() + 16, sizeof(double) * 8);
+            for (int st = 0; st < 6; ++st) add(N.ktab(st), sizeof(double) * L::kt);
+            add(N.q(), qb); add(N.df0(), qb); add(N.base(), qb); add(N.qe(), 4 * qb);
+            for (int st = 0; st < 5; ++st) add(N.qst_base(st), 4 * qb);
+            for (int w = 0; w < NWAVE; ++w) add(N.esc(w), sizeof(double) * L::kt + 4 * qb);
+            add(N.kinds(), sizeof(int) * (size_t)n);
+            add(N.seg(), sizeof(int) * 2 * MAXSEG); add(N.misc(), sizeof(int) * 4);
+            add(N.place(), sizeof(unsigned short) * (size_t)n);
+            *dump_off = (const char*)N.dump() - b0;
+            *read_reach = (const char*)N.tail() - b0;
+        };
+        const int layout = wsn_layout(n, nq);
+        if (layout == 0) regions_of(WSN0{});
+        else if (layout == 1) regions_of(WSN1{});
+        else if (layout == 2) regions_of(WSN2{});
+        else regions_of(WSN3{});
+        *nregions = cnt;
+        *total_bytes = (long long)tot;
+        return cnt <= cap ? BOLT_OK : set_error(BOLT_E_ARG, "region buffer too small");
+    }
+    WS W;
+    ws_bind(W, mem.data(), n, nq);
     add(W.u(), vb); add(W.f(), vb); add(W.un(), vb); add(W.fn(), vb); add(W.arg(), vb); add(W.w(), vb);
     for (int j = 0; j < 6; ++j) add(W.Z(j), vb);
     add(W.cS(), vb); add(W.cP(), vb); add(W.cPi(), vb);
@@ -3335,20 +1168,13 @@ int bolt_ws_layout(int n, int nq, int fp32, int cap, long long* regions, int* nr
         const long long r = (const char*)v - b0 + sizeof(float) * std::max<long long>(rows, n + CB);
         reach = std::max(reach, r);
     };
-    for (int st = 0; st < 5; ++st) {
-        if (fp32) {  // the FP32 solve mode's factors, and its copy of the stage right-hand side
-            const BandsT<float> B = W.bandsF(st);
-            add(B.l1, sizeof(float) * n); add(B.d, sizeof(float) * n); add(B.u1, sizeof(float) * n);
-            add(B.l2c, sizeof(float) * CB); add(B.u2c, sizeof(float) * CB);
-            reach_of_f(B.l1); reach_of_f(B.d); reach_of_f(B.u1);
-        } else {
-            const Bands B = W.bands(st);
-            add(B.l1, vb); add(B.d, vb); add(B.u1, vb);
-            add(B.l2c, sizeof(double) * CB); add(B.u2c, sizeof(double) * CB);
-            reach_of(B.l1); reach_of(B.d); reach_of(B.u1);
-        }
+    for (int st = 0; st < 5; ++st) {  // the FP32 factors, and the copy of the stage right-hand side
+        const BandsT<float> B = W.bandsF(st);
+        add(B.l1, sizeof(float) * n); add(B.d, sizeof(float) * n); add(B.u1, sizeof(float) * n);
+        add(B.l2c, sizeof(float) * CB); add(B.u2c, sizeof(float) * CB);
+        reach_of_f(B.l1); reach_of_f(B.d); reach_of_f(B.u1);
     }
-    if (fp32) add(W.rvec(), vb);
+    add(W.rvec(), vb);
     reach_of(W.w()); reach_of(W.cS()); reach_of(W.cP()); reach_of(W.cPi()); reach_of(W.arg());
     add(W.q(), qb); add(W.df0(), qb); add(W.base(), qb);
     add(W.qe(), qb); add(W.eqdf(), qb); add(W.sw(), qb); add(W.rw(), qb);
@@ -3559,18 +1385,16 @@ static std::mutex g_tune_mu;
 static std::map<std::pair<int, int>, int> g_tuned_sr;
 static std::map<std::tuple<int, int, int, int>, int> g_tuned_spw;
 
-// the solver instantiation for a shape: FP64 for every scan row count, the FP32
-// solve mode with SR_DEFAULT rows per lane
-static void launch_solver(int sr, bool f32, int grid, size_t lds, hipStream_t stream, const SolveArgs& A) {
-    if (f32) {
-        hipLaunchKernelGGL((k_boltsolve<SR_DEFAULT, true>), dim3(grid), dim3(NTHR), lds, stream, A);
-        return;
-    }
-    switch (sr) {
-        case 7: hipLaunchKernelGGL((k_boltsolve<7, false>), dim3(grid), dim3(NTHR), lds, stream, A); break;
-        case 8: hipLaunchKernelGGL((k_boltsolve<8, false>), dim3(grid), dim3(NTHR), lds, stream, A); break;
-        default: hipLaunchKernelGGL((k_boltsolve<6, false>), dim3(grid), dim3(NTHR), lds, stream, A); break;
-    }
+// (the FP32 solve mode runs with SR_DEFAULT rows per lane)
+static void launch_solver(int sr, int layout, bool f32, int grid, size_t lds, hipStream_t stream, const SolveArgs& A) {
+    void* args[] = {(void*)&A};
+    (void)hipLaunchKernel(f32 ? boltsolve_kernel(false) : solver_kernel(sr, layout), dim3(grid), dim3(NTHR), args, lds,
+                          stream);
+}
+// resident workgroups of that kernel per CU
+static hipError_t solver_per_cu(int* per_cu, int sr, int layout, bool f32, size_t lds) {
+    const void* f = f32 ? boltsolve_kernel(false) : solver_kernel(sr, layout);
+    return hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, f, NTHR, lds);
 }
 
 // rows per lane of the substitution scans for state length n: the value tuned
@@ -3598,9 +1422,15 @@ static int launch_modes(bolt_ctx* ctx, hipStream_t stream, const SolveBufs* pre,
     const bool tan = cosmos_dot != nullptr;
     std::stable_sort(md.begin(), md.end(), [](const ModeDesc& a, const ModeDesc& b) { return a.k > b.k; });
     size_t lds = 0;
-    for (const CfgDev& c : cfgs)
+    int nmax = 0, layout = 0;
+    for (const CfgDev& c : cfgs) {
+        layout = std::max(layout, wsn_layout(c.n, c.nq));
         lds = std::max(lds, tan ? sizeof(double) * (wtan_offset(c.n, c.nq) + wtan_doubles(c.n, c.nq))
-                                : ws_bytes(c.n, c.nq));
+                                : solve_lds(c.n, c.nq));
+        nmax = std::max(nmax, c.n);
+    }
+    const int sr = force_sr ? force_sr : solver_sr(ctx, nmax);
+    const bool f32 = (cfgs[0].flags & BOLT_CFG_FP32_SOLVE) != 0;
     if ((long long)lds > ctx->lds_max)
         return set_error(BOLT_E_ARG, tan ? "hierarchy too large for one workgroup's LDS with its tangent"
                                          : "hierarchy too large for one workgroup's LDS");
@@ -3651,9 +1481,9 @@ static int launch_modes(bolt_ctx* ctx, hipStream_t stream, const SolveBufs* pre,
     if (persistent) {
         int per_cu = 0;
         if (tan)
-            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_boltsolve<SR_DEFAULT, false, true>, NTHR, lds));
+            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, boltsolve_kernel(true), NTHR, lds));
         else
-            HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_boltsolve<SR_DEFAULT, false>, NTHR, lds));
+            HIPCHK(solver_per_cu(&per_cu, sr, layout, f32, lds));
         if (per_cu < 1) per_cu = 1;
         grid = std::min(B, per_cu * ctx->n_cu);
     }
@@ -3661,17 +1491,16 @@ static int launch_modes(bolt_ctx* ctx, hipStream_t stream, const SolveBufs* pre,
     HIPCHK(hipEventCreate(&e0));
     HIPCHK(hipEventCreate(&e1));
     HIPCHK(hipEventRecord(e0, stream));
-    int nmax = 0;
     for (const CfgDev& c : cfgs) {
-        nmax = std::max(nmax, c.n);
         if ((c.flags & BOLT_CFG_FP32_SOLVE) != (cfgs[0].flags & BOLT_CFG_FP32_SOLVE))
             return set_error(BOLT_E_ARG, "one launch cannot mix FP64 and FP32 solve modes");
     }
-    if (tan)
-        hipLaunchKernelGGL((k_boltsolve<SR_DEFAULT, false, true>), dim3(grid), dim3(NTHR), lds, stream, A);
-    else
-        launch_solver(force_sr ? force_sr : solver_sr(ctx, nmax), (cfgs[0].flags & BOLT_CFG_FP32_SOLVE) != 0, grid,
-                      lds, stream, A);
+    if (tan) {
+        void* args[] = {(void*)&A};
+        HIPCHK(hipLaunchKernel(boltsolve_kernel(true), dim3(grid), dim3(NTHR), args, lds, stream));
+    } else {
+        launch_solver(sr, layout, f32, grid, lds, stream, A);
+    }
     HIPCHK(hipGetLastError());
     HIPCHK(hipEventRecord(e1, stream));
     HIPCHK(hipEventSynchronize(e1));
@@ -4697,7 +2526,7 @@ int bolt_graph_spectrum_create(bolt_ctx* ctx, int cosmo_id, const bolt_hier_cfg*
     for (int i = 0; i < nk; ++i) { md[i].k = kh[i]; md[i].cosmo = 0; md[i].cfg = 0; md[i].out = i; md[i].pad = 0; }
     std::stable_sort(md.begin(), md.end(), [](const ModeDesc& a, const ModeDesc& b) { return a.k > b.k; });
     const CfgDev cd = to_cfgdev(cfg);
-    const size_t lds = ws_bytes(cd.n, cd.nq);
+    const size_t lds = solve_lds(cd.n, cd.nq);
     if ((long long)lds > ctx->lds_max) return set_error(BOLT_E_ARG, "hierarchy too large for one workgroup's LDS");
     // the LOS launch, as cl_core sets it up
     int lmax = 0;
@@ -4740,9 +2569,9 @@ int bolt_graph_spectrum_create(bolt_ctx* ctx, int cosmo_id, const bolt_hier_cfg*
     A.out_mode = 1; A.x_save = nullptr; A.nsave = 0; A.out = d_S; A.out2 = nullptr; A.status = d_status;
     A.counters = (long long*)d_counters; A.n_state_stride = 0; A.lds_doubles = (int)(lds / sizeof(double));
     int per_cu = 0;
-    HIPCHK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_boltsolve<SR_DEFAULT, false>, NTHR, lds));
-    const int sgrid = std::min(nk, std::max(per_cu, 1) * ctx->n_cu);
     const int sr = solver_sr(ctx, cd.n);
+    HIPCHK(solver_per_cu(&per_cu, sr, wsn_layout(cd.n, cd.nq), (cd.flags & BOLT_CFG_FP32_SOLVE) != 0, lds));
+    const int sgrid = std::min(nk, std::max(per_cu, 1) * ctx->n_cu);
     LosArgs L;
     L.cosmo = cs->d_self; L.S = d_S; L.SP = nullptr; L.k_src = d_k; L.nk_src = nk; L.kgrid = d_kgrid; L.nkd = nkd;
     L.lidx = d_lidx; L.lmax = lmax; L.nu = nu; L.etaj = d_eta; L.dxj = d_dx; L.i0 = i0; L.nxi = nxi; L.spin = 0;
@@ -4751,7 +2580,7 @@ int bolt_graph_spectrum_create(bolt_ctx* ctx, int cosmo_id, const bolt_hier_cfg*
     // capture: counter reset, solver, LOS node table, LOS, reduction
     HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(1), 0, ctx->stream, d_ctr);
-    launch_solver(sr, (cd.flags & BOLT_CFG_FP32_SOLVE) != 0, sgrid, lds, ctx->stream, A);
+    launch_solver(sr, wsn_layout(cd.n, cd.nq), (cd.flags & BOLT_CFG_FP32_SOLVE) != 0, sgrid, lds, ctx->stream, A);
     hipLaunchKernelGGL(k_los_prep, dim3((nxi + 255) / 256), dim3(256), 0, ctx->stream, cs->d_self, i0, nxi, d_eta,
                        d_dx);
     launch_los<1>(spw, lgrid, ctx->stream, L);
@@ -5455,7 +3284,7 @@ static void qs_launch_loop(QServer* sv) {
         A.idle_limit = (int)std::max(1000.0, QS_IDLE_US / (3.4 * sv->poll_sleeps + 1.0));
         A.published = sv->ctl; A.closed = sv->ctl + 1; A.drain = sv->ctl + 2; A.leave = sv->d_leave;
         A.done = sv->done;
-        launch_solver(SR_DEFAULT, false, sv->grid, sv->lds, sv->s_solve, A);
+        launch_solver(SR_DEFAULT, WSN_LAYOUTS - 1, false, sv->grid, sv->lds, sv->s_solve, A);
         bool ok = hipGetLastError() == hipSuccess;
         // wait for the launch; drain it once the server has held no request for QS_DRAIN_MS
         double idle_since = -1.0;
@@ -5782,7 +3611,7 @@ int bolt_submit(bolt_ctx* ctx, const bolt_request* req, uint64_t* id) {
     if (ctx->qserver) {
         QServer* sv = ctx->qserver.get();
         const CfgDev cd = to_cfgdev(&req->cfg);
-        if (ws_bytes(cd.n, cd.nq) > (size_t)ctx->lds_max)
+        if (solve_lds(cd.n, cd.nq) > (size_t)ctx->lds_max)
             return set_error(BOLT_E_ARG, "bolt_submit: hierarchy too large for one workgroup's LDS");
         auto q = std::make_shared<QReq>();
         q->rq = *req;
