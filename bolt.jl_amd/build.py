@@ -17,12 +17,13 @@ LIB = os.path.join(HERE, "libbolt_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-# The solver's one loop spans thousands of instructions: constants that machine
-# LICM hoists to its top stay live across it and spill scalar registers.
-SOLVE = ["-mllvm", "-disable-machine-licm"]
+# The solver's, the tables' and the line-of-sight loops span thousands of
+# instructions: constants that machine LICM hoists to their tops stay live across
+# them and spill registers.
+NOLICM = ["-mllvm", "-disable-machine-licm"]
 # (object, source, extra flags); the solver is compiled once per scan shape
-SOURCES = [("bolt_hip.o", "bolt_hip.hip", []), ("boltsolve.o", "boltsolve.hip", SOLVE)] + \
-          [(f"solve_sr{sr}.o", "solve.hip", SOLVE + [f"-DSOLVE_SR={sr}"]) for sr in (6, 7, 8)] + \
+SOURCES = [("bolt_hip.o", "bolt_hip.hip", NOLICM), ("boltsolve.o", "boltsolve.hip", NOLICM)] + \
+          [(f"solve_sr{sr}.o", "solve.hip", NOLICM + [f"-DNOLICM_SR={sr}"]) for sr in (6, 7, 8)] + \
           [("host_tables.o", "host_tables.cpp", []), ("host_api.o", "host_api.cpp", [])]
 
 

@@ -257,9 +257,9 @@ __global__ void k_plin_post(const CosmoDev* cosmos, const CfgDev* cfgs, const Mo
 // turning point ((2ℓ+1)/z > 2) the slot ends once |j_ℓ| < 1e-7 max|j| or once
 // |j_ℓ| grows (there the true j_ℓ decays monotonically, so growth means the
 // recurrence's growing solution has taken over).
-// One block of four wavefronts per dense-k midpoint; lanes own x nodes (slots
-// of 64 consecutive nodes); ℓ runs in chunks reduced across lanes by a
-// butterfly reduce-scatter and across the wavefronts through LDS.
+// One block per dense-k midpoint at a time; lanes own x nodes (slots of 64
+// consecutive nodes); ℓ runs in chunks of 16 reduced across the lanes in registers
+// and, every LOS_SPAN multipoles, across the wavefronts through LDS.
 // NS = 1: one source (C_ℓ^TT, or C_ℓ^EE with the spin factor); NS = 2: the
 // temperature and polarization sources share each j_ℓ and give TT, TE, EE.
 #define LOS_SLOTS 16   // x slots of 64 nodes (up to 1024 nodes after x = -8)
@@ -268,6 +268,7 @@ __global__ void k_plin_post(const CosmoDev* cosmos, const CfgDev* cfgs, const Mo
 // their C_ℓ contributions into a row of its own.  Fixed, so that the
 // summation order, and with it every bit of C_ℓ, does not depend on the device
 #define LOS_GRID 512
+#define LOS_SPAN 128       // multipoles between two exchanges of a block's wavefronts
 #define LOS_SPW_DEFAULT 4  // x slots per wavefront (LOS_SLOTS/SPW wavefronts per block): 1, 2 or 4
 #define LOS_TAU 1e-7
 // lanes with z < LOS_ZS take j_ℓ from its ascending series
@@ -276,6 +277,10 @@ __global__ void k_plin_post(const CosmoDev* cosmos, const CfgDev* cfgs, const Mo
 // z < ℓ), and run until |j_ℓ| < LOS_TAU_SMALL max|j| or ℓ = JSER_L: there the
 // polarization source (∝ 1/z²) makes terms far below the cut above count.
 #define LOS_ZS 2.0
+#define LOS_ZL 32.0  // a wavefront whose live lanes have z >= LOS_ZL takes the short recurrences
+// from this ℓ on no lane with z < LOS_ZL is left: the slowest, z = 32, is cut at
+// ℓ = 52, and the series ends before JSER_L
+#define LOS_LEAN 64
 #define LOS_TAU_SMALL 1e-30
 #define JSER_L 48
 #define JSER_M 14
@@ -351,97 +356,191 @@ __device__ inline double spin_factor(int l) {
     return sqrt((double)((L + 2) * (L + 1) * L * (L - 1)));
 }
 
-// advance one x slot through ℓ = L0+I0 .. L0+CH-1, accumulating j_ℓ s (and j_ℓ sp);
-// NS = 3: accp takes the derivative j_ℓ ṡ + j′_ℓ ż s of the term (sp = ṡ,
-// zs = ż s), with j′_ℓ = j_{ℓ−1} − (ℓ+1)/z j_ℓ from the recurrence's own values
-template <int NS, int CH, int I0>
-__device__ inline void los_slot(double& jp, double& jc, double iz, double s, double sp, double zs, double& M,
-                                bool& al, int L0, double* acc, double* accp, long long& nstep) {
-    double a_jp = jp, a_jc = jc, MM = M;
-    bool live = al;
-    const double base = (double)(2 * L0 - 1);
-#pragma unroll
-    for (int i = I0; i < CH; ++i) {
-        double t = (base + 2.0 * i) * iz;  // (2ℓ-1)/z produces j_ℓ, ℓ = L0+i
-        double jn = t * a_jc - a_jp;
-        a_jp = a_jc;
-        a_jc = jn;
-        // past the turning point j_ℓ decays monotonically: a term below
-        // LOS_TAU·max or a growing one (the recurrence's error has taken over)
-        // ends the slot
-        if (t > 2.0 && (fabs(jn) < LOS_TAU * MM || fabs(jn) > fabs(a_jp))) live = false;
-        MM = fmax(MM, fabs(jn));
-        double v = live ? jn : 0.0;
-        nstep += live ? 1 : 0;
-        acc[i] += v * s;
-        if constexpr (NS == 2) accp[i] += v * sp;
-        if constexpr (NS == 3) {
-            const double vp = live ? a_jp - (double)(L0 + i + 1) * iz * jn : 0.0;
-            accp[i] += v * sp + vp * zs;
-        }
-    }
-    jp = a_jp; jc = a_jc; M = MM; al = live;
+// one lane's state of one x slot: z = k (η₀ − η), j_{ℓ−2}, j_{ℓ−1}, 1/z, the
+// source times Δx and (NS = 2: the second source; NS = 3: its derivative, and
+// zs = ż s with ż = k (dη₀/dp − dη/dp)), the largest |j| so far, z^ℓ of the
+// series.  A lane past its cut, or without a node, has jp = jc = iz = 0: every
+// further j_ℓ is zero.  n: the wavefront's lanes that still count.
+struct LosLane {
+    double jp, jc, iz, s, sp, zs, M, z, zl;
+    int n;
+};
+
+// votes as comparisons of a ballot with zero: known to be the same for the whole
+// wavefront, so that the compiler branches around a path instead of masking it
+__device__ inline bool los_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
+__device__ inline bool los_none(bool p) { return __builtin_amdgcn_ballot_w64(p) == 0; }
+// t = (2ℓ−1)/z, which produces j_ℓ: 2ℓ−1 as the low bits of 2⁵² + 2ℓ−1, a scalar
+// register pair without a conversion; the fma takes 2⁵²/z off again and rounds once,
+// to the same value as the product
+__device__ inline double los_t(const LosLane& q, int l) {
+    return __builtin_fma(__hiloint2double(0x43300000, 2 * l - 1), q.iz, -0x1p52 * q.iz);
+}
+// take the lanes past their cut out
+__device__ inline void los_drop(LosLane& q, bool live) {
+    q.n = __popcll(__builtin_amdgcn_ballot_w64(live));
+    q.jp = live ? q.jp : 0.0;
+    q.jc = live ? q.jc : 0.0;
+    q.iz = live ? q.iz : 0.0;
+}
+// the terms of one ℓ, v = j_ℓ (zero past the cut), vp = j_{ℓ−1} − (ℓ+1)/z j_ℓ = j′_ℓ
+template <int NS>
+__device__ inline void los_add(const LosLane& q, double v, double vp, double& acc, double& accp) {
+    acc += v * q.s;
+    if constexpr (NS == 2) accp += v * q.sp;
+    if constexpr (NS == 3) accp += v * q.sp + vp * q.zs;
 }
 
-// los_slot for a wavefront holding live small-z lanes: those lanes take the
-// series (zl carries z^ℓ), the others the recurrence as in los_slot
-template <int NS, int CH, int I0>
-__device__ inline void los_slot_series(double& jp, double& jc, double iz, double z, double& zl, bool small, double s,
-                                       double sp, double zs, double& M, bool& al, int L0, double* acc, double* accp,
-                                       long long& nstep) {
-    double a_jp = jp, a_jc = jc, MM = M, zz = zl;
-    bool live = al;
-    const double base = (double)(2 * L0 - 1), w = z * z;
+// Advance one x slot through ℓ = L0+I0 .. L0+CH-1, accumulating j_ℓ s (and j_ℓ sp;
+// NS = 3: the derivative j_ℓ ṡ + j′_ℓ ż s of the term).  SERIES: the wavefront holds
+// live lanes with z < LOS_ZS, which take the series (zl carries z^ℓ).
+template <int NS, int CH, int I0, bool SERIES>
+__device__ inline void los_slot(LosLane& q, int L0, double* acc, double* accp, int& nstep) {
+    bool live = q.iz != 0.0;
+    const double w = SERIES ? q.z * q.z : 0.0;
 #pragma unroll
     for (int i = I0; i < CH; ++i) {
-        asm volatile("" ::: "memory");  // keeps this ℓ's series coefficients' loads here
         const int l = L0 + i;
-        double t = (base + 2.0 * i) * iz;
+        const double t = los_t(q, l);
         double jn;
-        if (small) {
-            zz *= z;
-            jn = (live && l < JSER_L) ? jser(l, w, zz) : 0.0;
-            if (!(fabs(jn) >= LOS_TAU_SMALL * MM) || l >= JSER_L) live = false;
+        bool cut;
+        if (SERIES) asm volatile("" ::: "memory");  // keeps this ℓ's series coefficients' loads here
+        if (SERIES && q.z < LOS_ZS) {
+            q.zl *= q.z;
+            jn = (live && l < JSER_L) ? jser(l, w, q.zl) : 0.0;
+            cut = !(fabs(jn) >= LOS_TAU_SMALL * q.M) || l >= JSER_L;
         } else {
-            jn = t * a_jc - a_jp;
-            if (t > 2.0 && (fabs(jn) < LOS_TAU * MM || fabs(jn) > fabs(a_jc))) live = false;
+            // past the turning point j_ℓ decays monotonically: a term below
+            // LOS_TAU·max or a growing one (the recurrence's error has taken over)
+            // ends the slot
+            jn = t * q.jc - q.jp;
+            cut = t > 2.0 && (fabs(jn) < LOS_TAU * q.M || fabs(jn) > fabs(q.jc));
         }
-        a_jp = a_jc;
-        a_jc = jn;
-        MM = fmax(MM, fabs(jn));
-        double v = live ? jn : 0.0;
-        nstep += live ? 1 : 0;
-        acc[i] += v * s;
-        if constexpr (NS == 2) accp[i] += v * sp;
-        if constexpr (NS == 3) {
-            const double vp = live ? a_jp - (double)(l + 1) * iz * jn : 0.0;
-            accp[i] += v * sp + vp * zs;
-        }
+        live = live && !cut;
+        q.jp = q.jc;
+        q.jc = jn;
+        q.M = fmax(q.M, fabs(jn));
+        nstep += __popcll(__builtin_amdgcn_ballot_w64(live));
+        los_add<NS>(q, live ? jn : 0.0, NS == 3 && live ? q.jp - (double)(l + 1) * q.iz * jn : 0.0, acc[i], accp[i]);
     }
-    jp = a_jp; jc = a_jc; M = MM; al = live; zl = zz;
+    los_drop(q, live);
 }
 
-// butterfly reduce-scatter of acc[CH] over the wavefront: lane l returns Σ_lanes acc[l % CH]
-template <int CH>
-__device__ inline double los_reduce(double* acc, int lane) {
+// los_slot for a wavefront whose live lanes all have z >= LOS_ZL, with its chunk's
+// last t above 1.5.  Up to t = 2 no cut can apply: four instructions a step.  From
+// there on a lane is tested in the chunks that begin past its turning point: from
+// z = LOS_ZL up j_ℓ is still above 2e-6 of its maximum CH multipoles on, so no cut
+// falls into the chunk before, and past t = 2 the maximum stays.
+template <int NS, int CH, int I0>
+__device__ inline void los_slot_turn(LosLane& q, int L0, double* acc, double* accp, int& nstep) {
+    if (los_none(los_t(q, L0 + CH - 1) > 2.0)) {
 #pragma unroll
-    for (int w = CH / 2; w >= 1; w >>= 1) {
-        bool up = (lane & w) != 0;
-#pragma unroll
-        for (int i = 0; i < w; ++i) {
-            // the two values pass through an empty asm so that the selects act
-            // on registers: a select between two elements of acc would otherwise
-            // become a lane-dependent index into the whole array
-            double a = acc[i], b = acc[i + w];
-            asm volatile("" : "+v"(a), "+v"(b));
-            const double send = up ? a : b;
-            const double keep = up ? b : a;
-            acc[i] = keep + __shfl_xor(send, w, WAVE);
+        for (int i = I0; i < CH; ++i) {
+            const double jn = los_t(q, L0 + i) * q.jc - q.jp;
+            q.jp = q.jc;
+            q.jc = jn;
+            q.M = fmax(q.M, fabs(jn));
+            los_add<NS>(q, jn, q.jp - (double)(L0 + i + 1) * q.iz * jn, acc[i], accp[i]);
         }
+        nstep += (CH - I0) * q.n;
+        return;
     }
-    double T = acc[0];
+    bool live = q.iz != 0.0;
+    const bool past = los_t(q, L0 + I0) > 2.0;
+    const double thr = past ? LOS_TAU * q.M : 0.0;
 #pragma unroll
-    for (int w = CH; w < WAVE; w <<= 1) T += __shfl_xor(T, w, WAVE);
+    for (int i = I0; i < CH; ++i) {
+        const double jn = los_t(q, L0 + i) * q.jc - q.jp;
+        if (fabs(jn) < thr || (past && fabs(jn) > fabs(q.jc))) live = false;
+        q.jp = q.jc;
+        q.jc = jn;
+        q.M = fmax(q.M, fabs(jn));
+        nstep += __popcll(__builtin_amdgcn_ballot_w64(live));
+        los_add<NS>(q, live ? jn : 0.0, NS == 3 && live ? q.jp - (double)(L0 + i + 1) * q.iz * jn : 0.0, acc[i], accp[i]);
+    }
+    los_drop(q, live);
+}
+
+// SPW lanes' states as separate members: an array would be kept as one register
+// tuple that every update copies
+template <int SPW>
+struct LosLanes {
+    LosLane q;
+    LosLanes<SPW - 1> rest;
+    template <int SL = 0, class F>
+    __device__ __forceinline__ void each(F&& f) {
+        f(q, std::integral_constant<int, SL>{});
+        rest.template each<SL + 1>(f);
+    }
+};
+template <>
+struct LosLanes<0> {
+    template <int SL = 0, class F>
+    __device__ __forceinline__ void each(F&&) {}
+};
+
+// The first N slots of a wavefront through one chunk with t = (2ℓ−1)/z <= 1.5 up to
+// its last ℓ on every lane: neither the cut nor the maximum of |j| falls here.  (At
+// fixed z the largest |j_ℓ| is the last one before the turning point, at ℓ ≈ z −
+// 0.81 z^{1/3}, the Airy maximum; at z = 32 it is 0.048, against 0.037 for all ℓ up
+// to t = 1.5, and the ratio grows with z.)  Three instructions a step, the slots'
+// recurrences side by side and without a branch.
+template <int NS, int CH, int N, int SPW>
+__device__ inline void los_below(LosLanes<SPW>& Q, int L0, double* acc, double* accp, int& nstep) {
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+        Q.each([&](LosLane& q, auto sl) {
+            if constexpr (decltype(sl)::value < N) {
+                const double jn = los_t(q, L0 + i) * q.jc - q.jp;
+                q.jp = q.jc;
+                q.jc = jn;
+                los_add<NS>(q, jn, q.jp - (double)(L0 + i + 1) * q.iz * jn, acc[i], accp[i]);
+            }
+        });
+    Q.each([&](LosLane& q, auto sl) { nstep += decltype(sl)::value < N ? CH * q.n : 0; });
+}
+
+// the two registers' halves traded so that their sum is a on the lanes whose bit
+// 32 (16) is clear and b on the others: v_permlane32_swap, v_permlane16_swap
+__device__ inline double fold32(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane32_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+__device__ inline double fold16(double a, double b) {
+    const auto lo = __builtin_amdgcn_permlane16_swap(__double2loint(a), __double2loint(b), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(__double2hiint(a), __double2hiint(b), false, false);
+    return __hiloint2double(hi[0], lo[0]) + __hiloint2double(hi[1], lo[1]);
+}
+// the same across bit 8 and bit 4 of the lane: DPP moves inside a row of 16, a
+// bank (four lanes) masked off keeping its own value
+template <int CTRL_UP, int BANKS_UP, int CTRL_DN, int BANKS_DN>
+__device__ inline double fold_row(double a, double b) {
+    auto mv = [](double old, double v, auto ctrl, auto banks) {
+        const int lo = __builtin_amdgcn_update_dpp(__double2loint(old), __double2loint(v), decltype(ctrl)::value, 0xF,
+                                                   decltype(banks)::value, false);
+        const int hi = __builtin_amdgcn_update_dpp(__double2hiint(old), __double2hiint(v), decltype(ctrl)::value, 0xF,
+                                                   decltype(banks)::value, false);
+        return __hiloint2double(hi, lo);
+    };
+    const double t = mv(a, b, std::integral_constant<int, CTRL_UP>{}, std::integral_constant<int, BANKS_UP>{});
+    const double u = mv(b, a, std::integral_constant<int, CTRL_DN>{}, std::integral_constant<int, BANKS_DN>{});
+    return t + u;
+}
+// reduce-scatter of acc[16] over the wavefront, in registers: lane l returns
+// Σ_lanes acc[l / 4].  57 VALU instructions; through __shfl_xor (LDS) and selects
+// it was 170 and six LDS round trips a chunk.
+__device__ inline double los_reduce(const double* acc) {
+    double a[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) a[i] = fold32(acc[i], acc[i + 8]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) a[i] = fold16(a[i], a[i + 4]);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) a[i] = fold_row<0x128, 0xC, 0x128, 0x3>(a[i], a[i + 2]);  // row_ror 8
+    double T = fold_row<0x114, 0xA, 0x104, 0x5>(a[0], a[1]);                              // row_shr 4, row_shl 4
+    T += dpp64<0xB1>(T);  // quad_perm 1,0,3,2
+    T += dpp64<0x4E>(T);  // quad_perm 2,3,0,1
     return T;
 }
 
@@ -464,17 +563,31 @@ __device__ __attribute__((noinline)) double los_pw(double A_s, double n_s, doubl
 // T_ℓ(k) = Σ_x j_ℓ(k(η₀−η)) S(x, k) Δx for every requested ℓ, and the
 // C_ℓ contributions T_ℓ² P(k) Δk/k summed over the block's midpoints.
 // A block of LOS_SLOTS/SPW wavefronts; wavefront w owns x slots w, w + W, ...
-// (SPW of them).  C_ℓ of ℓ is accumulated by lane ℓ mod 16 of wavefront 0
-// only (its partial-row entry is read and written by no other thread).
+// (SPW of them).  Each wavefront runs LOS_SPAN multipoles on its own, chunk by
+// chunk, its partial T_ℓ kept in LDS; then the block adds its wavefronts' partials
+// and the row entries (entry ℓ is always read and written by the same thread).
+// What bounds it: FP64 issue.  2500 ℓ x 4999 k x 799 x are 5.7e7 wavefront steps, of
+// three instructions where nothing can be cut (los_below, 70 % of them), four up to
+// the turning point and a dozen past it.  With the cut tested in every step (20
+// instructions) and a reduction through LDS with two barriers every 16 ℓ it was
+// 5.9 ms (9.0e8 VALU instructions); it is 1.77 ms (4.7e8, of which the reductions
+// are a fifth), 56 % of the VALU's issue slots; the rest is the wavefronts' unequal
+// shares between two exchanges (13 slots over 4).  TT, TE and EE of 1499 ℓ x 3000 k:
+// 4.0 -> 1.2 ms.
+// SPW: four slots a wavefront share one reduction and four independent chains; two
+// take 25 % more instructions at twice the wavefronts, the same 1.8 ms for NS = 1
+// and 1.3 times as long for NS = 2, so four is the default.
 template <int NS, int SPW>
-__global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE) k_los(LosArgs A) {
+__global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 && NS == 1) ? 4 : 2) k_los(LosArgs A) {
     constexpr int CH = 16;  // ℓ per chunk (NA·CH accumulators per lane)
     constexpr int NW = LOS_SLOTS / SPW;
     constexpr int NA = NS == 1 ? 1 : 2;                    // accumulator sets
     constexpr int NOUT = NS == 1 ? 1 : (NS == 2 ? 3 : 2);  // partial-row outputs
     const int lane = threadIdx.x & (WAVE - 1);
     const int wv = threadIdx.x / WAVE;
-    __shared__ double part[NW][NA][CH];
+    __shared__ double part[2][NW][NA][LOS_SPAN];  // by turns, so that one barrier a span is enough
+    __shared__ int plive[2][NW];
+    int turn = 0;
     __shared__ double nsum[NW];
     const double eta0 = A.cosmo->eta0;
     const int nx = A.cosmo->nx;
@@ -497,128 +610,160 @@ __global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE) k_los(LosArgs A) {
         const double* Pa = NA == 2 ? A.SP + (size_t)ia * nx + A.i0 : nullptr;
         const double* Pb = NA == 2 ? A.SP + (size_t)(ia + 1) * nx + A.i0 : nullptr;
 
-        double jp[SPW], jc[SPW], iz[SPW], sv[SPW], spv[SPW], mx[SPW], zv[SPW], zl[SPW];
-        double zsv[SPW];  // NS = 3: ż s, with ż = k (dη₀/dp − dη/dp)
-        bool alive[SPW], small[SPW];
-#pragma unroll
-        for (int sl = 0; sl < SPW; ++sl) {
-            const int j = (wv + NW * sl) * WAVE + lane;
+        // the wavefronts' turns at the longest slots (the earliest x) move on with ik,
+        // differently in the two blocks of a CU
+        const int own = (wv + (ik >> 8)) & (NW - 1);
+        LosLanes<SPW> Q;
+        Q.each([&](LosLane& q, auto sl) {
+            const int j = (own + NW * decltype(sl)::value) * WAVE + lane;
+            q.sp = q.zs = 0.0;
             if (j < A.nxi) {
                 const double z = k * (eta0 - A.etaj[j]);
-                const double sx = ((1.0 - tt) * Sa[j] + tt * Sb[j]) * A.dxj[j];
-                const double sp = NA == 2 ? ((1.0 - tt) * Pa[j] + tt * Pb[j]) * A.dxj[j] : 0.0;
-                zsv[sl] = NS == 3 ? k * (A.eta0d - A.etajd[j]) * sx : 0.0;
-                small[sl] = z < LOS_ZS;
+                q.s = ((1.0 - tt) * Sa[j] + tt * Sb[j]) * A.dxj[j];
+                if constexpr (NA == 2) q.sp = ((1.0 - tt) * Pa[j] + tt * Pb[j]) * A.dxj[j];
+                if constexpr (NS == 3) q.zs = k * (A.eta0d - A.etajd[j]) * q.s;
                 const double2 j01 = los_j01(z);
-                const double j0 = j01.x, j1 = j01.y;
-                zv[sl] = z;
-                zl[sl] = z;
-                jp[sl] = j0; jc[sl] = j1;
-                iz[sl] = 1.0 / z;
-                sv[sl] = sx;
-                spv[sl] = sp;
-                mx[sl] = fmax(fabs(j0), fabs(j1));
-                alive[sl] = true;
+                q.z = q.zl = z;
+                q.jp = j01.x;
+                q.jc = j01.y;
+                q.iz = 1.0 / z;
+                q.M = fmax(fabs(q.jp), fabs(q.jc));
             } else {
-                jp[sl] = jc[sl] = iz[sl] = sv[sl] = spv[sl] = mx[sl] = zsv[sl] = 0.0;
-                zv[sl] = zl[sl] = 0.0;
-                alive[sl] = false;
-                small[sl] = false;
+                q.jp = q.jc = q.iz = q.s = q.M = 0.0;
+                q.z = q.zl = LOS_ZS;
             }
-        }
-        long long nstep = 0;
+            q.n = __popcll(__builtin_amdgcn_ballot_w64(j < A.nxi));
+        });
+        int nstep = 0;  // wave-uniform
         const double Pw = los_pw(A.cosmo->Pprim_A, A.cosmo->Pprim_n, k, dk);
         const double Pwd = NS == 3 ? Pw * (A.dlnA + A.dns * log(k / 0.05)) : 0.0;
-        for (int L0 = 0; L0 <= A.lmax; L0 += CH) {
-            double acc[CH], accp[NA == 2 ? CH : 1];
+        // ℓ = L0 .. L0+CH-1 of this wavefront into part[]; form 0: the chunk that begins
+        // with j₀ and j₁, 1: below LOS_LEAN, 2: above
+        auto chunk = [&](int L0, int at, auto form) {
+            constexpr int FORM = decltype(form)::value, I0 = FORM == 0 ? 2 : 0;
+            double acc[CH], accp[CH];  // accp: NA = 2
 #pragma unroll
-            for (int i = 0; i < CH; ++i) acc[i] = 0.0;
-#pragma unroll
-            for (int i = 0; i < (NA == 2 ? CH : 1); ++i) accp[i] = 0.0;
-            bool any_live = false;
-            if (L0 == 0) {
-#pragma unroll
-                for (int sl = 0; sl < SPW; ++sl) {
-                    acc[0] += jp[sl] * sv[sl];
-                    acc[1] += jc[sl] * sv[sl];
-                    if constexpr (NS == 2) { accp[0] += jp[sl] * spv[sl]; accp[1] += jc[sl] * spv[sl]; }
-                    if constexpr (NS == 3) {  // j₀′ = −j₁, j₁′ = j₀ − 2j₁/z
-                        accp[0] += jp[sl] * spv[sl] - jc[sl] * zsv[sl];
-                        accp[1] += jc[sl] * spv[sl] + (jp[sl] - 2.0 * iz[sl] * jc[sl]) * zsv[sl];
+            for (int i = 0; i < CH; ++i) acc[i] = accp[i] = 0.0;
+            int live = 0;
+            Q.each([&](LosLane& q, auto) { live += q.n; });
+            if (live) {
+                int nb = 0;  // leading slots below t = 1.5
+                if constexpr (FORM == 2) {
+                    bool go = true;
+                    Q.each([&](LosLane& q, auto) {
+                        go = go && q.n && los_none(los_t(q, L0 + CH - 1) > 1.5);
+                        nb += go;
+                    });
+                    if (nb == 1) los_below<NS, CH, 1>(Q, L0, acc, accp, nstep);
+                    if constexpr (SPW >= 2)
+                        if (nb == 2) los_below<NS, CH, 2>(Q, L0, acc, accp, nstep);
+                    if constexpr (SPW >= 4) {
+                        if (nb == 3) los_below<NS, CH, 3>(Q, L0, acc, accp, nstep);
+                        if (nb == 4) los_below<NS, CH, 4>(Q, L0, acc, accp, nstep);
                     }
-                    if (__any(alive[sl] && small[sl]))
-                        los_slot_series<NS, CH, 2>(jp[sl], jc[sl], iz[sl], zv[sl], zl[sl], small[sl], sv[sl], spv[sl],
-                                                   zsv[sl], mx[sl], alive[sl], 0, acc, accp, nstep);
-                    else
-                        los_slot<NS, CH, 2>(jp[sl], jc[sl], iz[sl], sv[sl], spv[sl], zsv[sl], mx[sl], alive[sl], 0, acc,
-                                            accp, nstep);
                 }
-                any_live = true;
-            } else {
-#pragma unroll
-                for (int sl = 0; sl < SPW; ++sl) {
-                    if (!__any(alive[sl])) continue;
-                    any_live = true;
-                    if (__any(alive[sl] && small[sl]))
-                        los_slot_series<NS, CH, 0>(jp[sl], jc[sl], iz[sl], zv[sl], zl[sl], small[sl], sv[sl], spv[sl],
-                                                   zsv[sl], mx[sl], alive[sl], L0, acc, accp, nstep);
+                Q.each([&](LosLane& q, auto sl) {
+                    if constexpr (FORM == 0) {
+                        acc[0] += q.jp * q.s;
+                        acc[1] += q.jc * q.s;
+                        if constexpr (NS == 2) { accp[0] += q.jp * q.sp; accp[1] += q.jc * q.sp; }
+                        if constexpr (NS == 3) {  // j₀′ = −j₁, j₁′ = j₀ − 2j₁/z
+                            accp[0] += q.jp * q.sp - q.jc * q.zs;
+                            accp[1] += q.jc * q.sp + (q.jp - 2.0 * q.iz * q.jc) * q.zs;
+                        }
+                    }
+                    if (q.n == 0 || decltype(sl)::value < nb) return;
+                    if (FORM == 2 || los_none(q.iz > 1.0 / LOS_ZL))
+                        los_slot_turn<NS, CH, I0>(q, L0, acc, accp, nstep);
+                    else if (los_any(q.iz != 0.0 && q.z < LOS_ZS))
+                        los_slot<NS, CH, I0, true>(q, L0, acc, accp, nstep);
                     else
-                        los_slot<NS, CH, 0>(jp[sl], jc[sl], iz[sl], sv[sl], spv[sl], zsv[sl], mx[sl], alive[sl], L0, acc,
-                                            accp, nstep);
-                }
+                        los_slot<NS, CH, I0, false>(q, L0, acc, accp, nstep);
+                });
             }
             double Tv = 0.0, Ev = 0.0;
-            if (any_live) {  // wave-uniform
-                Tv = los_reduce<CH>(acc, lane);
-                if constexpr (NA == 2) Ev = los_reduce<CH>(accp, lane);
+            if (live) {
+                Tv = los_reduce(acc);
+                if constexpr (NA == 2) Ev = los_reduce(accp);
             }
-            if (lane < CH) {
-                part[wv][0][lane] = Tv;
-                if (NA == 2) part[wv][NA - 1][lane] = Ev;
+            if ((lane & 3) == 0) {
+                part[turn][own][0][at + (lane >> 2)] = Tv;
+                if (NA == 2) part[turn][own][NA - 1][at + (lane >> 2)] = Ev;
             }
-            const int live_block = __syncthreads_or(any_live ? 1 : 0);
-            if (wv == 0 && lane < CH) {
-                double Tt = part[0][0][lane], Et = NA == 2 ? part[0][NA - 1][lane] : 0.0;
+            return live;
+        };
+        // Thread i < len owns ℓ = span + i.  What it adds to is read before the span's
+        // recurrences: read after them, 20 spans x 10 midpoints waited for it in turn.
+        const int li = threadIdx.x;
+        int u = -1;
+        double r0 = 0.0, r1 = 0.0, r2 = 0.0;
+        auto fetch = [&](int span, int len) {
+            const int l = span + li;
+            u = li < len && l <= A.lmax ? A.lidx[l] : -1;
+            if (u >= 0 && !first) {
+                r0 = row[u];
+                if (NOUT >= 2) r1 = row[A.nu + u];
+                if (NOUT >= 3) r2 = row[2 * A.nu + u];
+            }
+        };
+        // the wavefronts' sums of ℓ = span .. span+len-1 to the block's row; false
+        // when every term was past its cut
+        auto exchange = [&](int span, int len, int live) {
+            if (lane == 0) plive[turn][own] = live;
+            __syncthreads();
+            int live_block = plive[turn][0];
+#pragma unroll
+            for (int w = 1; w < NW; ++w) live_block |= plive[turn][w];
+            if (u >= 0) {
+                const int l = span + li;
+                double Tt = part[turn][0][0][li], Et = NA == 2 ? part[turn][0][NA - 1][li] : 0.0;
 #pragma unroll
                 for (int w = 1; w < NW; ++w) {
-                    Tt += part[w][0][lane];
-                    if (NA == 2) Et += part[w][NA - 1][lane];
+                    Tt += part[turn][w][0][li];
+                    if (NA == 2) Et += part[turn][w][NA - 1][li];
                 }
-                const int l = L0 + lane;
-                const int u = l <= A.lmax ? A.lidx[l] : -1;
-                if (u >= 0) {
-                    if (NS == 1) {
-                        const double v = A.spin ? Tt * spin_factor(l) : Tt;
-                        const double c = v * v * Pw;
-                        row[u] = first ? c : row[u] + c;
-                    } else if (NS == 3) {  // T² P and its derivative 2TṪP + T²Ṗ
-                        const double c0 = Tt * Tt * Pw, c1 = 2.0 * Tt * Et * Pw + Tt * Tt * Pwd;
-                        row[u] = first ? c0 : row[u] + c0;
-                        row[A.nu + u] = first ? c1 : row[A.nu + u] + c1;
-                    } else {
-                        const double ep = Et * spin_factor(l);
-                        const double c0 = Tt * Tt * Pw, c1 = Tt * ep * Pw, c2 = ep * ep * Pw;
-                        row[u] = first ? c0 : row[u] + c0;
-                        row[A.nu + u] = first ? c1 : row[A.nu + u] + c1;
-                        row[2 * A.nu + u] = first ? c2 : row[2 * A.nu + u] + c2;
-                    }
-                }
-                // every term is past its cut: the remaining T_ℓ are zero, so
-                // the block's first midpoint stores zeros for them (same lane
-                // ownership: ℓ ≡ lane mod 16) and later midpoints add nothing
-                if (!live_block && first) {
-                    for (int l2 = L0 + CH + lane; l2 <= A.lmax; l2 += CH) {
-                        const int u2 = A.lidx[l2];
-                        if (u2 < 0) continue;
-                        for (int o = 0; o < NOUT; ++o) row[o * A.nu + u2] = 0.0;
-                    }
+                if (NS == 1) {
+                    const double v = A.spin ? Tt * spin_factor(l) : Tt;
+                    const double c = v * v * Pw;
+                    row[u] = first ? c : r0 + c;
+                } else if (NS == 3) {  // T² P and its derivative 2TṪP + T²Ṗ
+                    const double c0 = Tt * Tt * Pw, c1 = 2.0 * Tt * Et * Pw + Tt * Tt * Pwd;
+                    row[u] = first ? c0 : r0 + c0;
+                    row[A.nu + u] = first ? c1 : r1 + c1;
+                } else {
+                    const double ep = Et * spin_factor(l);
+                    const double c0 = Tt * Tt * Pw, c1 = Tt * ep * Pw, c2 = ep * ep * Pw;
+                    row[u] = first ? c0 : r0 + c0;
+                    row[A.nu + u] = first ? c1 : r1 + c1;
+                    row[2 * A.nu + u] = first ? c2 : r2 + c2;
                 }
             }
-            __syncthreads();
-            if (!live_block) break;
-        }
+            // the remaining T_ℓ are zero, so the block's first midpoint stores
+            // zeros for them (from LOS_LEAN on thread i owns ℓ ≡ LOS_LEAN + i mod
+            // LOS_SPAN) and later midpoints add nothing
+            if (!live_block && first && li < LOS_SPAN)
+                for (int l2 = span + len + li; l2 <= A.lmax; l2 += LOS_SPAN) {
+                    const int u2 = A.lidx[l2];
+                    if (u2 < 0) continue;
+                    for (int o = 0; o < NOUT; ++o) row[o * A.nu + u2] = 0.0;
+                }
+            turn ^= 1;
+            return live_block != 0;
+        };
+        fetch(0, LOS_LEAN);
+        int live = chunk(0, 0, std::integral_constant<int, 0>{});
+        for (int L0 = CH; L0 < LOS_LEAN && L0 <= A.lmax; L0 += CH)
+            live |= chunk(L0, L0, std::integral_constant<int, 1>{});
+        if (exchange(0, LOS_LEAN, live))
+            for (int span = LOS_LEAN; span <= A.lmax; span += LOS_SPAN) {
+                live = 0;
+                fetch(span, LOS_SPAN);
+                for (int L0 = span; L0 < span + LOS_SPAN && L0 <= A.lmax; L0 += CH)
+                    live |= chunk(L0, L0 - span, std::integral_constant<int, 2>{});
+                if (!exchange(span, LOS_SPAN, live)) break;
+            }
         if (A.steps) {
-            const double ns = wave_sum((double)nstep);
+            const double ns = (double)nstep;
             if (lane == 0) nsum[wv] = ns;
             __syncthreads();
             if (threadIdx.x == 0) {
@@ -809,12 +954,12 @@ __global__ void __launch_bounds__(LOS_SLOTS / 2 * WAVE) k_los_spline(LosSplArgs 
                     if constexpr (NS == 2) accp[c] += jv * spv[sl];
                 }
             }
-            const double Tv = los_reduce<CH>(acc, lane);
+            const double Tv = los_reduce(acc);
             double Ev = 0.0;
-            if constexpr (NS == 2) Ev = los_reduce<CH>(accp, lane);
-            if (lane < CH) {
-                part[wv][0][lane] = Tv;
-                if (NS == 2) part[wv][NS - 1][lane] = Ev;
+            if constexpr (NS == 2) Ev = los_reduce(accp);
+            if ((lane & 3) == 0) {
+                part[wv][0][lane >> 2] = Tv;
+                if (NS == 2) part[wv][NS - 1][lane >> 2] = Ev;
             }
             __syncthreads();
             if (wv == 0 && lane < CH && U0 + lane < A.nu) {

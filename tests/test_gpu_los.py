@@ -1,0 +1,57 @@
+"""The line-of-sight sum at the edges of its splits: x nodes per slot of 64 lanes and
+slots per wavefront, chunks of 16 multipoles, the change to the short recurrence at
+ℓ = 64, and the spans of 128 multipoles between two exchanges of a block."""
+import numpy as np
+import pytest
+
+import boltmi
+import cosmo
+import pyoracle
+
+pytestmark = pytest.mark.gpu
+
+
+def setting(nxi):
+    """tables whose x grid has nxi integration nodes after x = -8, with sources: a bump
+    at last scattering, one at reionization and a late smooth part"""
+    n = next(n for n in range(16, 4000)
+             if sum(cosmo.xnode(j, nx=n) > -8.0 for j in range(n)) - 1 == nxi)
+    par = boltmi.CosmoParams()
+    bg = boltmi.Background(par, x_grid=(-20.0, 0.0, n))
+    k = boltmi.quadratic_k(0.1 * bg.H0, 1000 * bg.H0, 30)
+    x = np.asarray(bg.x_grid)
+    S = np.exp(-((x + 7.0) / 0.15)**2) + 0.1 * np.exp(-((x + 2.2) / 0.3)**2) + 0.02 * np.exp(x)
+    S = S * (1.0 + np.cos(60.0 * k / k[-1]))[:, None]
+    P = S / (1.0 + x**2)
+    return par, bg, boltmi.SourceGrid(bg.x_grid, k, S), boltmi.SourceGrid(bg.x_grid, k, P), \
+        boltmi.quadratic_k(0.01 * bg.H0, 1000 * bg.H0, 520)
+
+
+# A term is left out where |j_ℓ| is below 1e-7 of its largest value: up to 2e-7 of C_ℓ
+# where the sum is of the size of its terms, rounded up to the 1e-6 that the other
+# comparisons with the oracle take; 1e-9 of the largest C_ℓ where the terms cancel.
+@pytest.mark.parametrize("spw", ["1", "2", "4"])
+@pytest.mark.parametrize("nxi", [9, 63, 64, 65, 256, 257, 1024])
+def test_x_slots_against_oracle(nxi, spw, monkeypatch):
+    monkeypatch.setenv("BOLT_LOS_SPW", spw)
+    par, bg, T, P, dense = setting(nxi)
+    ctx = boltmi.Context(0)
+    ells = np.array([2, 3, 15, 16, 17, 63, 64, 65, 191, 192, 193, 319, 320, 900, 1500])
+    o = pyoracle.Oracle(par.as_tuple(), bg.tables_dict())
+    got = boltmi.cl_on_grid(ells, T, P, dense, par, bg, ctx=ctx)
+    for g, r in zip(got, o.cl(T.grid, P.grid, T.k_grid, dense, ells, 0, nthreads=8)):
+        np.testing.assert_allclose(g, r, rtol=1e-6, atol=1e-9 * np.max(np.abs(r)))
+    one = boltmi.cltt_on_grid(ells, T, dense, par, bg, ctx=ctx)
+    np.testing.assert_allclose(one, got[0], rtol=1e-13)
+
+
+def test_last_multipole_does_not_matter():
+    """C_ℓ is the same to the last bit whatever the largest ℓ of the call is"""
+    par, bg, T, P, dense = setting(320)
+    full = boltmi.cl_on_grid(np.arange(2, 701), T, P, dense, par, bg)
+    tt = boltmi.cltt_on_grid(np.arange(2, 701), T, dense, par, bg)
+    for lmax in (2, 15, 16, 17, 63, 64, 65, 79, 80, 191, 192, 193, 320, 321):
+        part = boltmi.cl_on_grid(np.arange(2, lmax + 1), T, P, dense, par, bg)
+        for g, r in zip(part, full):
+            np.testing.assert_array_equal(g, r[:lmax - 1])
+        np.testing.assert_array_equal(boltmi.cltt_on_grid(np.arange(2, lmax + 1), T, dense, par, bg), tt[:lmax - 1])
