@@ -23,7 +23,7 @@ ARCH = "gfx950"
 NOLICM = ["-mllvm", "-disable-machine-licm"]
 # (object, source, extra flags); the solver is compiled once per scan shape
 SOURCES = [("bolt_hip.o", "bolt_hip.hip", NOLICM), ("boltsolve.o", "boltsolve.hip", NOLICM)] + \
-          [(f"solve_sr{sr}.o", "solve.hip", NOLICM + [f"-DNOLICM_SR={sr}"]) for sr in (6, 7, 8)] + \
+          [(f"solve_sr{sr}.o", "solve.hip", NOLICM + [f"-DSOLVE_SR={sr}"]) for sr in (6, 7, 8)] + \
           [("host_tables.o", "host_tables.cpp", []), ("host_api.o", "host_api.cpp", [])]
 
 
