@@ -31,6 +31,7 @@
 #include <string>
 #include <thread>
 #include <tuple>
+#include <climits>
 #include <type_traits>
 #include <unordered_map>
 #include <vector>
@@ -780,37 +781,47 @@ __global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 
 // ------------------------------------------- Bolt's spline j_ℓ (bessel_mode 1)
 // bessel_interpolator (spectra.jl:49-58): j_ℓ on the 5001 nodes 0:Δ:z_max
 // (Δ = z_max/5000), interpolated by the natural cubic B-spline of util.jl:11.
-// The table is node-major, tab[(m + 1)·nu + u] for node m and requested ℓ
-// column u, with the spline's padding rows 0 and BES_N + 1, so that a lane
-// reads 16 consecutive columns of one node in one 128-byte line.
+// The spline is linear in its coefficients c_m(ℓ), so the sum over the x nodes
+// (spectra.jl:70-96) is a matrix product:
+//   T_ℓ(k) = Σ_x s_x Σ_p w_p(z_x) c_{i(z_x)+p}(ℓ) = Σ_m W_m(k) c_m(ℓ),
+// W_m(k) the sources times basis weights that fall on coefficient m.  W does not
+// depend on ℓ: k_spline_weights builds it once per k, and k_spline_cl multiplies
+// (FP64 MFMA).  Summed term by term, four gathered coefficients for each (ℓ, k, x),
+// a call was 7.6 ms for 120 ℓ x 4999 k x 799 x and 150 ms for 2499 ℓ, bound by the
+// gathers; it is 0.47 and 2.9 ms.
+// Coefficients are node-major, c[m·nu + u] for requested ℓ column u, with the
+// spline's padding rows 0 and BES_N + 1, then zeros up to BES_LD.
 #define BES_N 5001
+#define BES_LD 5008      // rows of c, columns of W: a multiple of 16
+#define BES_ROWS 6144    // midpoints whose W is kept at once (246 MB per source)
 
-// j_ℓ(z_m) for every requested ℓ at node m (one thread per node): Miller's
-// downward recurrence f_{l-1} = (2l+1)/z f_l - f_{l+1} from f_N = 1e-300,
-// N = max(ℓ_max, z) + 60 + 12·max(ℓ_max, z)^(1/3), rescaled by 1e-250 whenever
-// |f| > 1e250, normalised to the exact j₀ or j₁ (whichever is larger).  A
-// first pass counts the rescalings; the second stores each f_ℓ with the
-// rescalings that follow it applied, then the normalisation.
-__global__ void k_bessel_nodes(double zmax, const int* lidx, int lmax, int nu, double* tab) {
+// a node's table values, up to the factors that are only known at the recurrence's
+// end: j_ℓ = v · scale · 2^(−600·#{q: ℓ > e_q}), zero for ℓ > e[2]
+struct BesNode {
+    double scale;
+    int e[3];
+};
+// j_ℓ(z_m) for every requested ℓ at node m (one thread per node).  From z = ℓ_max up
+// the recurrence runs upward, which is stable for ℓ <= z.  Below, Miller's downward
+// recurrence f_{l-1} = (2l+1)/z f_l - f_{l+1} from f_N = 2^-1000, N = ℓ_max + 60 +
+// 12·ℓ_max^(1/3), rescaled by 2^-600 whenever |f| is found above 2^600, normalised
+// to the exact j₀ or j₁ (whichever is larger).  Each value is stored as it comes: the rescalings that follow it and the normalisation are applied where
+// the prefilter reads it.
+// One wavefront per SIMD at most (79 wavefronts): what counts is the chain.  Downward
+// from N for all nodes and twice (the first pass counted the rescalings) was 10 100
+// steps at z = 4800; it is 1200 up or 1390 down for ℓ_max = 1200, in 59 us.  Against 80-bit arithmetic the upward values are off by 5e-14 of the
+// largest |j_ℓ|, the downward ones from z = 4800 were by 4e-13.
+__global__ void __launch_bounds__(WAVE) k_bessel_nodes(double zmax, const int* ulist, int nu, double* raw, BesNode* node) {
     const int m = blockIdx.x * blockDim.x + threadIdx.x;
     if (m >= BES_N) return;
+    const int lmax = ulist[nu - 1];
     const double z = m * (zmax / (BES_N - 1));
-    double* row = tab + (size_t)(m + 1) * nu;
+    double* row = raw + (size_t)m * nu;
+    BesNode nd = {1.0, {INT_MAX, INT_MAX, INT_MAX}};
     if (z == 0.0) {
-        for (int l = 0; l <= lmax; ++l)
-            if (lidx[l] >= 0) row[lidx[l]] = l == 0 ? 1.0 : 0.0;
+        for (int u = 0; u < nu; ++u) row[u] = ulist[u] == 0 ? 1.0 : 0.0;
+        node[m] = nd;
         return;
-    }
-    const double zm = fmax((double)lmax, z);
-    const int N = (int)(zm + 60.0 + 12.0 * cbrt(zm));
-    const double inv = 1.0 / z;
-    double fp = 0.0, fc = 1e-300;
-    int R = 0;
-    for (int l = N; l >= 1; --l) {
-        const double fm = (2 * l + 1) * inv * fc - fp;
-        fp = fc;
-        fc = fm;
-        if (fabs(fc) > 1e250) { fc *= 1e-250; fp *= 1e-250; ++R; }
     }
     double j0, j1;
     if (z < 1e-3) {
@@ -823,47 +834,137 @@ __global__ void k_bessel_nodes(double zmax, const int* lidx, int lmax, int nu, d
         j0 = sn / z;
         j1 = (sn / z - cs) / z;
     }
-    const double scale = fabs(j0) >= fabs(j1) ? j0 / fc : j1 / fp;
-    fp = 0.0; fc = 1e-300;
-    int r = 0;
-    for (int l = N; l >= 1; --l) {
-        const double fm = (2 * l + 1) * inv * fc - fp;
+    const double inv = 1.0 / z;
+    if (z >= lmax && z >= 1.0) {
+        double fp = j0, fc = j1;  // j_{l-1}, j_l
+        int l = 1;
+        double a = 3.0;  // 2l + 1
+        auto step = [&] {
+            const double fn = a * inv * fc - fp;
+            fp = fc;
+            fc = fn;
+            a += 2.0;
+            ++l;
+        };
+        int next = ulist[0];
+        for (int u = 0; u < nu; ++u) {
+            const int lt = next;
+            next = u + 1 < nu ? ulist[u + 1] : lt;
+            while (l + 4 <= lt) { step(); step(); step(); step(); }
+            while (l < lt) step();
+            row[u] = lt == 0 ? j0 : fc;
+        }
+        node[m] = nd;
+        return;
+    }
+    const double zm = fmax((double)lmax, 1.0);  // z < zm: the same N for the wavefront
+    const int N = (int)(zm + 60.0 + 12.0 * cbrt(zm));
+    double fp = 0.0, fc = 0x1p-1000;
+    int l = N;
+    double a = 2 * N + 1;
+    auto step = [&] {
+        const double fm = a * inv * fc - fp;
         fp = fc;
         fc = fm;
-        if (fabs(fc) > 1e250) { fc *= 1e-250; fp *= 1e-250; ++r; }
-        if (l - 1 <= lmax && lidx[l - 1] >= 0) {
-            double v = fc;
-            for (int q = r; q < R; ++q) v *= 1e-250;
-            row[lidx[l - 1]] = v * scale;
+        a -= 2.0;
+        --l;
+    };
+    auto look = [&] {
+        if (fabs(fc) > 0x1p600) {
+            fc *= 0x1p-600;
+            fp *= 0x1p-600;
+            nd.e[2] = nd.e[1];
+            nd.e[1] = nd.e[0];
+            nd.e[0] = l;  // counts for every ℓ above
         }
+    };
+    // 15 steps grow |f| by at most ((2N+1)/z)^15, less than 2^390 from z = 4e-5 up at
+    // ℓ_max = 1200: |f| is looked at after 8 to 15 of them
+    const bool eight = __all(a * inv < 0x1p26);
+    int next = ulist[nu - 1], since = 0;
+    for (int u = nu - 1; u >= -1; --u) {
+        const int lt = next;
+        next = u > 0 ? ulist[u - 1] : 0;  // the last turn runs on to ℓ = 0
+        if (eight) {
+            for (; l - lt >= 8; since = 0) {
+                step(); step(); step(); step(); step(); step(); step(); step();
+                look();
+            }
+            since += l - lt;
+            while (l > lt) step();
+            if (since >= 8) {
+                look();
+                since = 0;
+            }
+        } else {
+            while (l > lt) { step(); look(); }
+        }
+        if (u >= 0) row[u] = fc;
     }
+    nd.scale = fabs(j0) >= fabs(j1) ? j0 / fc : j1 / fp;
+    node[m] = nd;
 }
 
-// the natural cubic B-spline prefilter of one column (one thread per column),
-// in place: rows 1..BES_N hold the node values; cp is the shared forward
-// elimination factor 1/(4 − cp_{i−1}), cp_0 = 1/4
-__global__ void k_bessel_prefilter(int nu, const double* cp, double* tab) {
-    const int u = blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= nu) return;
-    const int n = BES_N, mm = n - 2;
-    double* c = tab + u;  // c[i·nu] is coefficient i
-    const double c1 = c[(size_t)1 * nu], cn = c[(size_t)n * nu];
-    // d_i = 6 y_{i+1} in row i + 2, i = 0..mm-1
-    double dprev = 0.0;
-    for (int i = 0; i < mm; ++i) {
-        double d = 6.0 * c[(size_t)(i + 2) * nu];
-        if (i == 0) d -= c1;
-        if (i == mm - 1) d -= cn;
-        d = i == 0 ? d / 4.0 : (d - dprev) / (4.0 - cp[i - 1]);
-        c[(size_t)(i + 2) * nu] = d;
-        dprev = d;
+// The natural cubic B-spline prefilter, one lane per column: the tridiagonal solve
+// (off-diagonals 1, diagonal 4) by the factors cp_q = 1/(4 − cp_{q−1}), cp_0 = 1/4,
+// for BES_PC coefficients a block.  Both sweeps forget their start by 0.268 a step:
+// BES_WARM steps ahead leave 4e-28 of it, so that the chunks are independent.  (In one
+// piece, 10 000 steps with a division and a load each, it was 2 ms on two wavefronts
+// for 120 ℓ; it is 32 µs.)
+#define BES_PC 32
+#define BES_WARM 48
+__global__ void __launch_bounds__(WAVE) k_bessel_prefilter(const int* ulist, int nu, const double* raw,
+                                                           const BesNode* node, double* c) {
+    __shared__ double d[BES_PC + BES_WARM + 1][WAVE];
+    __shared__ double cps[BES_PC + 2 * BES_WARM];
+    const int lane = threadIdx.x;
+    const int u0 = blockIdx.x * WAVE + lane, u = u0 < nu ? u0 : nu - 1;
+    const int ell = ulist[u];
+    constexpr int n = BES_N, mm = n - 2;
+    const int q0 = blockIdx.y * BES_PC, q1 = q0 + BES_PC < mm ? q0 + BES_PC : mm;
+    const int qs = q0 > BES_WARM ? q0 - BES_WARM : 0, qe = q1 + BES_WARM < mm ? q1 + BES_WARM : mm;
+    auto y = [&](int m) {
+        const BesNode nd = node[m];
+        double v = raw[(size_t)m * nu + u];
+        if (ell > nd.e[0]) v *= 0x1p-600;
+        if (ell > nd.e[1]) v *= 0x1p-600;
+        return ell > nd.e[2] ? 0.0 : v * nd.scale;
+    };
+    // cp_qs .. cp_{qe-1}; from cp_40 on they are the same to the last bit
+    if (lane == 0) {
+        double cp = 0.25;
+        for (int q = 0; q < (qs < 40 ? qs : 40); ++q) cp = 1.0 / (4.0 - cp);
+        for (int q = qs; q < qe; ++q) {
+            cps[q - qs] = cp;
+            if (q < 40) cp = 1.0 / (4.0 - cp);
+        }
     }
-    for (int i = mm - 2; i >= 0; --i) {
-        const double d = c[(size_t)(i + 2) * nu] - cp[i] * c[(size_t)(i + 3) * nu];
-        c[(size_t)(i + 2) * nu] = d;
+    __syncthreads();
+    const double y0 = y(0), yn = y(n - 1);
+    double dp = 0.0;
+#pragma unroll 16
+    for (int q = qs; q < qe; ++q) {
+        const double r = 6.0 * y(q + 1) - (q == 0 ? y0 : q == mm - 1 ? yn : 0.0);
+        dp = (r - dp) * cps[q - qs];
+        d[q >= q0 ? q - q0 : qe - q0][lane] = dp;  // the steps before q0 into a spare row
     }
-    c[0] = 2.0 * c1 - c[(size_t)2 * nu];
-    c[(size_t)(n + 1) * nu] = 2.0 * cn - c[(size_t)(n - 1) * nu];
+    double xn = 0.0;  // c_{q+3}
+#pragma unroll 16
+    for (int q = qe - 1; q >= q0; --q) {
+        xn = d[q - q0][lane] - cps[q - qs] * xn;
+        if (q < q1 && u0 < nu) c[(size_t)(q + 2) * nu + u] = xn;
+    }
+    const double c2 = xn, cl = d[qe - 1 - q0][lane];  // c_2 of the first chunk, c_{n−1} of the last
+    if (u0 >= nu) return;
+    if (q0 == 0) {
+        c[(size_t)1 * nu + u] = y0;
+        c[u] = 2.0 * y0 - c2;
+    }
+    if (q1 == mm) {
+        c[(size_t)n * nu + u] = yn;
+        c[(size_t)(n + 1) * nu + u] = 2.0 * yn - cl;
+        for (int m = n + 2; m < BES_LD; ++m) c[(size_t)m * nu + u] = 0.0;
+    }
 }
 
 struct LosSplArgs {
@@ -876,115 +977,232 @@ struct LosSplArgs {
     int nkd;
     const int* ulist;   // [nu] the distinct requested ℓ, ascending
     int nu;
-    const double* tab;  // [BES_N + 2][nu]
+    const double* c;    // [BES_LD][nu]
     double izd;         // 1/Δ
     const double* etaj;
     const double* dxj;
     int i0, nxi;
     int spin;
     double* partial;    // [grid][nout][nu]
+    int ik0, rows;      // this launch's midpoints ik0 .. ik0 + rows - 1
+    double* W;          // [NS][tiles·16][BES_LD]
+    double* Pw;         // [tiles·16]
+    double2* kt;        // [tiles·16] k and the weight of the source column ia + 1
+    int* ia;            // [tiles·16]
+    int* ext;           // [tiles] columns of W in use, a multiple of 16
 };
+__device__ inline int spline_node(const LosSplArgs& A, double k, double e) {  // e = η₀ − η
+    const int i = (int)floor(k * e * A.izd);
+    return i < 0 ? 0 : (i > BES_N - 2 ? BES_N - 2 : i);
+}
 
-// T_ℓ(k) with Bolt's spline j_ℓ: every (ℓ, k, x) term, as spectra.jl:70-96
-// evaluates it (no cut); blocks, x slots, partial rows and their lane
-// ownership as in k_los, the ℓ loop over the requested columns in chunks of 16
-template <int NS>
-__global__ void __launch_bounds__(LOS_SLOTS / 2 * WAVE) k_los_spline(LosSplArgs A) {
-    constexpr int CH = 16, SPW = 2, NW = LOS_SLOTS / SPW;
-    constexpr int NOUT = NS == 1 ? 1 : 3;
-    const int lane = threadIdx.x & (WAVE - 1);
-    const int wv = threadIdx.x / WAVE;
-    __shared__ double part[NW][NS][CH];
+// what k_spline_weights needs of each midpoint before it can start, one lane each
+// (read in a chain by every block it was a quarter of that kernel); midpoints beyond
+// `rows` fill up the last tile
+__global__ void __launch_bounds__(256) k_spline_rows(LosSplArgs A) {
+    __shared__ double emax[4];
+    const int tid = threadIdx.x, r = blockIdx.x * 256 + tid, tiles = (A.rows + 15) / 16;
     const double eta0 = A.cosmo->eta0;
-    const int nx = A.cosmo->nx;
-    const int nkm = A.nkd - 1;
-    double* row = A.partial + (size_t)blockIdx.x * NOUT * A.nu;
-    bool first = true;
-    for (int ik = blockIdx.x; ik < nkm; ik += gridDim.x) {
-        const double k = (A.kgrid[ik] + A.kgrid[ik + 1]) / 2.0;
-        const double dk = A.kgrid[ik + 1] - A.kgrid[ik];
-        int lo = 0, hi = A.nk_src - 2;
+    double em = 0.0;
+    for (int j = tid; j < A.nxi; j += 256) em = fmax(em, eta0 - A.etaj[j]);
+    for (int o = WAVE / 2; o; o >>= 1) em = fmax(em, __shfl_xor(em, o));
+    if ((tid & (WAVE - 1)) == 0) emax[tid / WAVE] = em;
+    __syncthreads();
+    em = fmax(fmax(emax[0], emax[1]), fmax(emax[2], emax[3]));
+    const bool in = r < A.rows;
+    double k = 0.0, Pw = 0.0, tt = 0.0;
+    int lo = 0, hi = A.nk_src - 2;
+    if (in) {
+        const double ka = A.kgrid[A.ik0 + r], kb = A.kgrid[A.ik0 + r + 1];
+        k = (ka + kb) / 2.0;
         while (lo < hi) {
-            int mid = (lo + hi + 1) >> 1;
-            if (A.k_src[mid] <= k) lo = mid; else hi = mid - 1;
+            int m = (lo + hi + 1) >> 1;
+            if (A.k_src[m] <= k) lo = m; else hi = m - 1;
         }
-        const int ia = lo;
-        const double tt = (k - A.k_src[ia]) / (A.k_src[ia + 1] - A.k_src[ia]);
-        const double* Sa = A.S + (size_t)ia * nx + A.i0;
-        const double* Sb = A.S + (size_t)(ia + 1) * nx + A.i0;
-        const double* Pa = NS == 2 ? A.SP + (size_t)ia * nx + A.i0 : nullptr;
-        const double* Pb = NS == 2 ? A.SP + (size_t)(ia + 1) * nx + A.i0 : nullptr;
-        double sv[SPW], spv[SPW], w[SPW][4];
-        int base[SPW];
+        tt = (k - A.k_src[lo]) / (A.k_src[lo + 1] - A.k_src[lo]);
+        Pw = los_pw(A.cosmo->Pprim_A, A.cosmo->Pprim_n, k, kb - ka);
+    }
+    double kt = k;  // columns of the tile: up to the largest k of its 16 midpoints
+    for (int o = 8; o; o >>= 1) kt = fmax(kt, __shfl_xor(kt, o));
+    if (r >= tiles * 16) return;
+    A.kt[r] = make_double2(k, tt);
+    A.ia[r] = lo;
+    A.Pw[r] = Pw;
+    if (r % 16 == 0) A.ext[r / 16] = (spline_node(A, kt, em) + 4 + 15) / 16 * 16;
+}
+
+// W of one midpoint per block: W_m = Σ_x s_x w_{m−i(z_x)}(z_x), in the order of the x
+// nodes (a gather over the nodes that reach m: no atomics, so the same bits every
+// time).  z falls with x where η grows: the x nodes that reach m are those between
+// start[m], the first with i <= m, and start[m − 4]; for a table in which η does not
+// grow, every x node is looked at.  4999 k x 799 x: 90 us, bound by the latency of
+// the LDS reads at four blocks to a CU.
+template <int NS>
+__global__ void __launch_bounds__(256) k_spline_weights(LosSplArgs A) {
+    // [NS][4][nxi] weight p times source, [nxi] first node, start[]
+    extern __shared__ double ws[];
+    const int nxi = A.nxi;
+    int* ix = (int*)(ws + (size_t)NS * 4 * nxi);
+    unsigned short* start = (unsigned short*)(ix + nxi);
+    const int r = blockIdx.x, tid = threadIdx.x, tiles = gridDim.x / 16;
+    const bool in = r < A.rows;  // the others' rows of W are zero
+    const double k = A.kt[r].x, tt = A.kt[r].y, eta0 = A.cosmo->eta0;
+    const int nx = A.cosmo->nx, ext = A.ext[r / 16];
+    const double* Sa = A.S + (size_t)A.ia[r] * nx + A.i0;
+    const double* Pa = NS == 2 ? A.SP + (size_t)A.ia[r] * nx + A.i0 : nullptr;
+    for (int j = tid; j < nxi; j += 256) {
+        const double e = eta0 - A.etaj[j];
+        const int i = spline_node(A, k, e);
+        ix[j] = i;
+        const double t = k * e * A.izd, s = t - i, q = 1.0 - s;
+        const double w[4] = {q * q * q / 6.0, 2.0 / 3.0 - s * s + 0.5 * s * s * s, 2.0 / 3.0 - q * q + 0.5 * q * q * q,
+                             s * s * s / 6.0};
+        const double sx = ((1.0 - tt) * Sa[j] + tt * Sa[nx + j]) * A.dxj[j];
+        const double sp = NS == 2 ? ((1.0 - tt) * Pa[j] + tt * Pa[nx + j]) * A.dxj[j] : 0.0;
 #pragma unroll
-        for (int sl = 0; sl < SPW; ++sl) {
-            const int j = (wv + NW * sl) * WAVE + lane;
-            const bool in = j < A.nxi;
-            const int jj = in ? j : 0;
-            const double z = k * (eta0 - A.etaj[jj]);
-            sv[sl] = in ? ((1.0 - tt) * Sa[jj] + tt * Sb[jj]) * A.dxj[jj] : 0.0;
-            spv[sl] = in && NS == 2 ? ((1.0 - tt) * Pa[jj] + tt * Pb[jj]) * A.dxj[jj] : 0.0;
-            // the spline's basis weights at z (orc_bessel_table_eval's form)
-            const double t = z * A.izd;
-            int i = (int)floor(t);
-            i = i < 0 ? 0 : (i > BES_N - 2 ? BES_N - 2 : i);
-            const double s = t - i, r = 1.0 - s;
-            w[sl][0] = r * r * r / 6.0;
-            w[sl][1] = 2.0 / 3.0 - s * s + 0.5 * s * s * s;
-            w[sl][2] = 2.0 / 3.0 - r * r + 0.5 * r * r * r;
-            w[sl][3] = s * s * s / 6.0;
-            base[sl] = i;
+        for (int p = 0; p < 4; ++p) {
+            ws[p * nxi + j] = w[p] * sx;
+            if constexpr (NS == 2) ws[(4 + p) * nxi + j] = w[p] * sp;
         }
-        const double Pw = los_pw(A.cosmo->Pprim_A, A.cosmo->Pprim_n, k, dk);
-        for (int U0 = 0; U0 < A.nu; U0 += CH) {
-            double acc[CH], accp[NS == 2 ? CH : 1];
-#pragma unroll
-            for (int c = 0; c < CH; ++c) acc[c] = 0.0;
-#pragma unroll
-            for (int c = 0; c < (NS == 2 ? CH : 1); ++c) accp[c] = 0.0;
-#pragma unroll
-            for (int sl = 0; sl < SPW; ++sl) {
-                const double* q = A.tab + (size_t)base[sl] * A.nu + U0;
-#pragma unroll
-                for (int c = 0; c < CH; ++c) {
-                    const int cu = U0 + c < A.nu ? c : 0;  // columns past nu repeat column U0 (not stored)
-                    const double jv = w[sl][0] * q[cu] + w[sl][1] * q[A.nu + cu] + w[sl][2] * q[2 * A.nu + cu] +
-                                      w[sl][3] * q[3 * A.nu + cu];
-                    acc[c] += jv * sv[sl];
-                    if constexpr (NS == 2) accp[c] += jv * spv[sl];
-                }
-            }
-            const double Tv = los_reduce(acc);
-            double Ev = 0.0;
-            if constexpr (NS == 2) Ev = los_reduce(accp);
-            if ((lane & 3) == 0) {
-                part[wv][0][lane >> 2] = Tv;
-                if (NS == 2) part[wv][NS - 1][lane >> 2] = Ev;
-            }
-            __syncthreads();
-            if (wv == 0 && lane < CH && U0 + lane < A.nu) {
-                double Tt = part[0][0][lane], Et = NS == 2 ? part[0][NS - 1][lane] : 0.0;
-#pragma unroll
-                for (int w2 = 1; w2 < NW; ++w2) {
-                    Tt += part[w2][0][lane];
-                    if (NS == 2) Et += part[w2][NS - 1][lane];
-                }
-                const int u = U0 + lane, l = A.ulist[u];
-                if (NS == 1) {
-                    const double v = A.spin ? Tt * spin_factor(l) : Tt;
-                    const double c = v * v * Pw;
-                    row[u] = first ? c : row[u] + c;
-                } else {
-                    const double ep = Et * spin_factor(l);
-                    const double c0 = Tt * Tt * Pw, c1 = Tt * ep * Pw, c2 = ep * ep * Pw;
-                    row[u] = first ? c0 : row[u] + c0;
-                    row[A.nu + u] = first ? c1 : row[A.nu + u] + c1;
-                    row[2 * A.nu + u] = first ? c2 : row[2 * A.nu + u] + c2;
-                }
-            }
-            __syncthreads();
+    }
+    __syncthreads();
+    bool grows = true;
+    for (int j = tid; j + 1 < nxi; j += 256) grows = grows && ix[j + 1] <= ix[j];
+    grows = !__syncthreads_or(grows ? 0 : 1);
+    if (grows)  // x node j begins nodes ix[j] .. ix[j−1] − 1; none begins those below the last
+        for (int j = tid; j <= nxi; j += 256) {
+            const int a = j < nxi ? ix[j] : 0, b = j ? ix[j - 1] : ext;
+            for (int m = a; m < b; ++m) start[m] = j;
         }
-        first = false;
+    __syncthreads();
+    // a node has 4·nxi/ext terms on average, but at the early end, where η hardly
+    // grows, up to twenty times as many: that average in lanes share it, every
+    // lanes-th x node each
+    int lg = 0;
+    while (lg < 6 && (ext << lg) < 4 * nxi) ++lg;
+    const int lanes = 1 << lg;
+    double* W = A.W + (size_t)r * BES_LD;
+    for (int m0 = 0; m0 < ext; m0 += 256 >> lg) {
+        const int m = m0 + (tid >> lg);
+        double w0 = 0.0, w1 = 0.0;
+        if (in && m < ext) {
+            const int ja = grows ? start[m] : 0, jb = grows && m >= 4 ? start[m - 4] : nxi;
+            for (int j = ja + (tid & (lanes - 1)); j < jb; j += lanes) {
+                const int p = m - ix[j];
+                if (p < 0 || p > 3) continue;  // only where η does not grow
+                w0 += ws[p * nxi + j];
+                if constexpr (NS == 2) w1 += ws[(4 + p) * nxi + j];
+            }
+        }
+        for (int o = 1; o < lanes; o *= 2) {
+            w0 += __shfl_xor(w0, o);
+            if constexpr (NS == 2) w1 += __shfl_xor(w1, o);
+        }
+        if ((tid & (lanes - 1)) == 0 && m < ext) {
+            W[m] = w0;
+            if constexpr (NS == 2) W[(size_t)tiles * 16 * BES_LD + m] = w1;
+        }
+    }
+}
+static size_t spline_weights_lds(int ns, int nxi) {
+    return (sizeof(double) * 4 * ns + sizeof(int)) * (size_t)nxi + sizeof(unsigned short) * BES_LD;
+}
+
+// T = W c for 16 midpoints x 64 columns a block, each of the four wavefronts over
+// every fourth group of 16 coefficients, then the C_ℓ contributions T_ℓ² P(k) Δk/k
+// summed over the block's midpoints into a partial row.  Four MFMAs (16x16x4) take 16
+// coefficients, lane l the four of its quarter (l / 16) one after the other, so that W
+// comes in two 16-byte loads and c in 128-byte lines, from L2, with no LDS.  The tiles
+// of the largest k, with the most coefficients, come first.
+// What bounds it is the loads' latency and W's way from memory (67 MB at 4999 k up to
+// z = k η₀).  120 ℓ x 4999 k, 3 GFLOP: 187 us with one wavefront per 16 columns over
+// all coefficients, 136 split four ways, 100 with a tile's column groups on one XCD,
+// 88 with four column groups to a wavefront (which is faster from 59 to 2499 ℓ: a
+// call at 499 ℓ takes 0.71 ms against 0.89).
+typedef double dbl4 __attribute__((ext_vector_type(4)));
+template <int NS>
+__global__ void __launch_bounds__(256) k_spline_cl(LosSplArgs A, int tiles, int grid, int first) {
+    constexpr int NOUT = NS == 1 ? 1 : 3, NW = 4, NC = 4;  // NC column groups of 16
+    __shared__ double red[NW][NS][NC][4][WAVE];
+    const int lane = threadIdx.x & (WAVE - 1), wv = threadIdx.x / WAVE;
+    const int col = lane & 15, quarter = lane >> 4;
+    // the column groups of one tile follow each other on one XCD (block b runs on XCD
+    // b % 8), whose L2 then holds the tile's W
+    const int ngroup = (A.nu + 16 * NC - 1) / (16 * NC), idx = blockIdx.x / 8;
+    const int bx = idx / ngroup * 8 + blockIdx.x % 8;
+    if (bx >= grid) return;
+    const int u0 = idx % ngroup * 16 * NC;
+    int uc[NC];
+#pragma unroll
+    for (int n = 0; n < NC; ++n) uc[n] = u0 + 16 * n + col < A.nu ? u0 + 16 * n + col : A.nu - 1;
+    // wavefront n finishes column group n
+    double sum[NOUT] = {};
+    for (int tile = tiles - 1 - bx; tile >= 0; tile -= grid) {
+        const int steps = A.ext[tile] / 16;
+        const double* w = A.W + ((size_t)tile * 16 + col) * BES_LD + 4 * quarter;
+        const double* wp = w + (size_t)tiles * 16 * BES_LD;
+        const double* c = A.c + (size_t)(4 * quarter) * A.nu;
+        dbl4 T[NS][NC];
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+#pragma unroll
+            for (int o = 0; o < NS; ++o) T[o][n] = (dbl4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+        for (int s = wv; s < steps; s += NW) {
+            const dbl4 a = *(const dbl4*)(w + 16 * s);
+            dbl4 e = a;
+            if constexpr (NS == 2) e = *(const dbl4*)(wp + 16 * s);
+            double b[NC][4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int n = 0; n < NC; ++n) b[n][q] = c[(size_t)(16 * s + q) * A.nu + uc[n]];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int n = 0; n < NC; ++n) {
+                    T[0][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q], b[n][q], T[0][n], 0, 0, 0);
+                    if constexpr (NS == 2)
+                        T[1][n] = __builtin_amdgcn_mfma_f64_16x16x4f64(e[q], b[n][q], T[1][n], 0, 0, 0);
+                }
+        }
+#pragma unroll
+        for (int n = 0; n < NC; ++n)
+#pragma unroll
+            for (int o = 0; o < NS; ++o)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) red[wv][o][n][q][lane] = T[o][n][q];
+        __syncthreads();
+        const int l = A.ulist[u0 + 16 * wv + col < A.nu ? u0 + 16 * wv + col : A.nu - 1];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {  // register q of lane l: row 4q + l/16, column l%16
+            double t[NS];
+#pragma unroll
+            for (int o = 0; o < NS; ++o) {
+                t[o] = red[0][o][wv][q][lane];
+#pragma unroll
+                for (int w2 = 1; w2 < NW; ++w2) t[o] += red[w2][o][wv][q][lane];
+            }
+            const double P = A.Pw[tile * 16 + 4 * q + quarter];
+            if constexpr (NS == 1) {
+                const double v = A.spin ? t[0] * spin_factor(l) : t[0];
+                sum[0] += v * v * P;
+            } else {
+                const double ep = t[1] * spin_factor(l);
+                sum[0] += t[0] * t[0] * P;
+                sum[1] += t[0] * ep * P;
+                sum[2] += ep * ep * P;
+            }
+        }
+        __syncthreads();
+    }
+    const int u = u0 + 16 * wv + col;
+#pragma unroll
+    for (int o = 0; o < NOUT; ++o) {
+        sum[o] += __shfl_xor(sum[o], 16);
+        sum[o] += __shfl_xor(sum[o], 32);
+        double* out = A.partial + ((size_t)bx * NOUT + o) * A.nu + u;
+        if (quarter == 0 && u < A.nu) *out = first ? sum[o] : *out + sum[o];
     }
 }
 
@@ -1002,8 +1220,10 @@ __global__ void __launch_bounds__(256) k_los_reduce(const double* partial, int n
     const int u = i < nell ? pmap[i] : 0;
     const int b0 = (int)((long long)wv * nb / 4), b1 = (int)((long long)(wv + 1) * nb / 4);
     double s = 0.0;
-    if (i < nell)
+    if (i < nell) {
+#pragma unroll 16
         for (int b = b0; b < b1; ++b) s += partial[((size_t)b * nout + o) * nu + u];
+    }
     red[wv][lane] = s;
     __syncthreads();
     if (wv == 0 && i < nell && cl) cl[i] = 4.0 * M_PI * (((red[0][lane] + red[1][lane]) + red[2][lane]) + red[3][lane]);
@@ -1203,7 +1423,8 @@ int bolt_ctx_create(int device, bolt_ctx** out) {
                 (void)hipFuncSetAttribute(solver_kernel(sr, layout), hipFuncAttributeMaxDynamicSharedMemorySize,
                                           c->lds_max);
         for (const void* f : {boltsolve_kernel(false), boltsolve_kernel(true),
-                              (const void*)k_rhs, (const void*)k_ics, (const void*)k_rhs_jvp, (const void*)k_ics_jvp})
+                              (const void*)k_rhs, (const void*)k_ics, (const void*)k_rhs_jvp, (const void*)k_ics_jvp,
+                              (const void*)k_spline_weights<1>, (const void*)k_spline_weights<2>})
             (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, c->lds_max);
         (void)hipGetLastError();  // an unsupported opt-in must not surface at the next launch check
     }
@@ -2295,7 +2516,7 @@ static int cl_core(bolt_ctx* ctx, hipStream_t stream, const LosBufs* pre, const 
     for (int e = 0; e < nell; ++e) pmap[e] = lidx[ells[e]];
     const int nout = two ? 3 : 1;
     const int nkm = nkd - 1;
-    const int grid = std::min(LOS_GRID, nkm);
+    int grid = std::min(LOS_GRID, nkm);
     LosBufs lb;
     const size_t npart = (size_t)grid * nout * nu;
     if (pre) {
@@ -2338,27 +2559,49 @@ static int cl_core(bolt_ctx* ctx, hipStream_t stream, const LosBufs* pre, const 
         const double zmax = kmax * host.eta0;
         std::vector<int> ul(nu);
         for (int l = 0; l <= lmax; ++l) if (lidx[l] >= 0) ul[lidx[l]] = l;
-        std::vector<double> cp(BES_N - 2);
-        cp[0] = 0.25;
-        for (int i = 1; i < BES_N - 2; ++i) cp[i] = 1.0 / (4.0 - cp[i - 1]);
-        HIPCHK(ctx->c_btab.ensure(sizeof(double) * ((size_t)(BES_N + 2) * nu + (BES_N - 2)) + sizeof(int) * nu));
-        double* tab = ctx->c_btab.as<double>();
-        double* d_cp = tab + (size_t)(BES_N + 2) * nu;
-        int* d_ul = (int*)(d_cp + (BES_N - 2));
-        HIPCHK(hipMemcpyAsync(d_cp, cp.data(), sizeof(double) * cp.size(), hipMemcpyHostToDevice, stream));
-        HIPCHK(hipMemcpyAsync(d_ul, ul.data(), sizeof(int) * nu, hipMemcpyHostToDevice, stream));
-        hipLaunchKernelGGL(k_bessel_nodes, dim3((BES_N + 127) / 128), dim3(128), 0, stream, zmax, lb.lidx, lmax, nu,
-                           tab);
-        hipLaunchKernelGGL(k_bessel_prefilter, dim3((nu + 63) / 64), dim3(64), 0, stream, nu, (const double*)d_cp,
-                           tab);
-        HIPCHK(hipGetLastError());
+        // one scratch block: W and Pw of up to BES_ROWS midpoints, the two tables, the rest
+        const int nsrc = two ? 2 : 1, batch = std::min(nkm, BES_ROWS);
+        const int tiles = (batch + 15) / 16;
+        const size_t nrow = (size_t)tiles * 16;
+        const size_t nW = nsrc * nrow * BES_LD, nc = (size_t)BES_LD * nu, nraw = (size_t)BES_N * nu;
+        HIPCHK(ctx->c_btab.ensure(sizeof(double) * (nW + 3 * nrow + nc + nraw) + sizeof(BesNode) * BES_N +
+                                  sizeof(int) * (nu + nrow + tiles)));
         LosSplArgs B;
+        B.W = ctx->c_btab.as<double>();
+        B.kt = (double2*)(B.W + nW);
+        B.Pw = (double*)(B.kt + nrow);
+        double* c = B.Pw + nrow;
+        double* raw = c + nc;
+        BesNode* node = (BesNode*)(raw + nraw);
+        int* d_ul = (int*)(node + BES_N);
+        B.ia = d_ul + nu;
+        B.ext = B.ia + nrow;
+        HIPCHK(hipMemcpyAsync(d_ul, ul.data(), sizeof(int) * nu, hipMemcpyHostToDevice, stream));
+        hipLaunchKernelGGL(k_bessel_nodes, dim3((BES_N + WAVE - 1) / WAVE), dim3(WAVE), 0, stream, zmax, d_ul, nu, raw,
+                           node);
+        hipLaunchKernelGGL(k_bessel_prefilter, dim3((nu + WAVE - 1) / WAVE, (BES_N - 2 + BES_PC - 1) / BES_PC), dim3(WAVE),
+                           0, stream, d_ul, nu, raw, node, c);
+        HIPCHK(hipGetLastError());
         B.cosmo = A.cosmo; B.S = A.S; B.SP = A.SP; B.k_src = A.k_src; B.nk_src = A.nk_src; B.kgrid = A.kgrid;
-        B.nkd = A.nkd; B.ulist = d_ul; B.nu = nu; B.tab = tab; B.izd = (BES_N - 1) / zmax; B.etaj = A.etaj;
+        B.nkd = A.nkd; B.ulist = d_ul; B.nu = nu; B.c = c; B.izd = (BES_N - 1) / zmax; B.etaj = A.etaj;
         B.dxj = A.dxj; B.i0 = A.i0; B.nxi = A.nxi; B.spin = A.spin; B.partial = A.partial;
+        grid = std::min(LOS_GRID, tiles);
         HIPCHK(hipEventRecord(e0, stream));
-        if (two) hipLaunchKernelGGL(k_los_spline<2>, dim3(grid), dim3(LOS_SLOTS / 2 * WAVE), 0, stream, B);
-        else hipLaunchKernelGGL(k_los_spline<1>, dim3(grid), dim3(LOS_SLOTS / 2 * WAVE), 0, stream, B);
+        for (int ik0 = 0; ik0 < nkm; ik0 += batch) {
+            B.ik0 = ik0;
+            B.rows = std::min(batch, nkm - ik0);
+            const int nt = (B.rows + 15) / 16;
+            const dim3 gr((nt * 16 + 255) / 256), gw(nt * 16), gc((grid + 7) / 8 * 8 * ((nu + 63) / 64)), b(256);
+            const size_t lds = spline_weights_lds(nsrc, nxi);
+            hipLaunchKernelGGL(k_spline_rows, gr, b, 0, stream, B);
+            if (two) {
+                hipLaunchKernelGGL(k_spline_weights<2>, gw, b, lds, stream, B);
+                hipLaunchKernelGGL(k_spline_cl<2>, gc, b, 0, stream, B, nt, grid, ik0 == 0);
+            } else {
+                hipLaunchKernelGGL(k_spline_weights<1>, gw, b, lds, stream, B);
+                hipLaunchKernelGGL(k_spline_cl<1>, gc, b, 0, stream, B, nt, grid, ik0 == 0);
+            }
+        }
     } else {
         HIPCHK(hipEventRecord(e0, stream));
         const int spw = force_spw ? force_spw : los_shape(ctx, nkd, lmax, two);

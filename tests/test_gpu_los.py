@@ -7,6 +7,7 @@ import pytest
 import boltmi
 import cosmo
 import pyoracle
+from boltmi import _abi
 
 pytestmark = pytest.mark.gpu
 
@@ -55,3 +56,44 @@ def test_last_multipole_does_not_matter():
         for g, r in zip(part, full):
             np.testing.assert_array_equal(g, r[:lmax - 1])
         np.testing.assert_array_equal(boltmi.cltt_on_grid(np.arange(2, lmax + 1), T, dense, par, bg), tt[:lmax - 1])
+
+
+# Both sides sum the same spline terms in 64 bits: 1e-9, as the other comparison with
+# the oracle's spline mode.
+@pytest.mark.parametrize("nxi,nkd,ells", [
+    (9, 2, [2, 3]),                        # one midpoint, fewer columns than a group
+    (63, 17, list(range(2, 18))),          # one full tile, one full column group
+    (65, 18, list(range(2, 19))),          # a midpoint and a column more
+    (320, 65, list(range(0, 34)) + [700]),  # ℓ = 0 and 1, repeated and far ℓ
+    (1024, 520, [2, 15, 16, 900, 1500, 15]),
+    (320, 161, list(range(2, 513))),       # one column short of the wide groups
+    (320, 161, list(range(2, 514))),       # the first wide call
+    (256, 161, list(range(2, 700))),       # a partial wide group
+    (320, 6200, [2, 37, 1100]),            # more midpoints than are kept at once
+])
+def test_spline_sum_against_oracle(nxi, nkd, ells):
+    par, bg, T, P, _ = setting(nxi)
+    dense = boltmi.quadratic_k(0.01 * bg.H0, 1000 * bg.H0, nkd)
+    ells = np.array(ells)
+    o = pyoracle.Oracle(par.as_tuple(), bg.tables_dict())
+    got = boltmi.cl_on_grid(ells, T, P, dense, par, bg, bessel_mode=1)
+    for g, r in zip(got, o.cl(T.grid, P.grid, T.k_grid, dense, ells, 1, nthreads=8)):
+        has = (ells > 0) | np.isfinite(r)  # the oracle's spline mode has no value for ℓ = 0
+        assert np.isfinite(g).all()
+        np.testing.assert_allclose(g[has], r[has], rtol=1e-9, atol=1e-9 * np.max(np.abs(r[has])))
+    np.testing.assert_allclose(boltmi.cltt_on_grid(ells, T, dense, par, bg, bessel_mode=1), got[0], rtol=1e-12)
+
+
+def test_spline_sum_where_eta_does_not_grow():
+    """tables whose η(x) goes back and forth: the x nodes that reach a coefficient are
+    no longer contiguous"""
+    par, bg, T, P, dense = setting(320)
+    x = np.linspace(-20.0, 0.0, bg.nx + 2)
+    bg.coef[_abi.T_ETA] *= 1.0 - 0.05 * np.sin(30.0 * x)**2
+    ells = np.arange(2, 100)
+    o = pyoracle.Oracle(par.as_tuple(), bg.tables_dict())
+    eta = np.array([o.spline(_abi.T_ETA, v) for v in bg.x_grid])
+    assert (np.diff(eta[bg.x_grid > -8.0]) < 0).any()
+    got = boltmi.cl_on_grid(ells, T, P, dense, par, bg, bessel_mode=1)
+    for g, r in zip(got, o.cl(T.grid, P.grid, T.k_grid, dense, ells, 1, nthreads=8)):
+        np.testing.assert_allclose(g, r, rtol=1e-9, atol=1e-9 * np.max(np.abs(r)))
