@@ -4111,8 +4111,11 @@ int bolt_serve_stop(bolt_ctx* ctx) {
 namespace {
 constexpr double MOM_CUT = 40.0;
 constexpr double MOM_SQRT_HALF_PI = 1.2533141373155002512078826424055;
-constexpr int MOM_CHUNK = 128;  // nodes per thread of the prefilter passes
-constexpr int MOM_WARM = 64;    // warm-up nodes: the recurrences contract by ~0.268 a node
+// prefilter: unknowns per lane, lanes per block, warm-up (the recurrences contract by
+// 0.268 an unknown: 4e-28 of the start is left), and the lanes at a block's end whose
+// unknowns only warm the others up
+constexpr int MOM_CHUNK = 32, MOM_LANES = 128, MOM_WARM = 48, MOM_HALO = (MOM_WARM + MOM_CHUNK - 1) / MOM_CHUNK;
+constexpr int MOM_TILE = (MOM_LANES - MOM_HALO) * MOM_CHUNK;  // unknowns a block delivers
 }  // namespace
 
 struct DD {
@@ -4284,82 +4287,95 @@ __host__ __device__ inline double mom_node(const MomTab& T, int i) {
 }
 
 // node values into rows 1..n of each coefficient column
-__global__ void __launch_bounds__(256) k_moment_nodes(MomTab T) {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < T.n; i += gridDim.x * blockDim.x) {
-        const double x = mom_node(T, i);
-        for (int m = 0; m < T.order; ++m) T.coef[(size_t)m * (T.n + 2) + 1 + i] = mom_node_value(x, T.nu, m, T.pref[m]);
-    }
+// a lane per node and moment: the nodes below x = 40 (double-double series, closed
+// forms) take a hundred times as long as the others, and with the three moments one
+// after the other they alone were 101 us at 400 000 nodes; 57 now
+__global__ void __launch_bounds__(256) k_moment_nodes(MomTab T, double* y) {
+    const int m = blockIdx.y;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < T.n; i += gridDim.x * blockDim.x)
+        y[(size_t)m * T.n + i] = mom_node_value(mom_node(T, i), T.nu, m, T.pref[m]);
 }
 
 // Line(OnGrid()) prefilter, the Thomas algorithm of the host tables' prefilter
-// (d_q = (r_q − d_{q−1}) / (4 − cp_{q−1}), cp_q = 1/(4 − cp_{q−1}), cp_0 = 1/4,
-// then c = d − cp·c_next).  The unknowns are c[2..n−1] (q = 0..n−3); c[1] = y_0
-// and c[n] = y_{n−1}.  cp_q is bitwise constant from q ≈ 20 on, and is held at
-// cp_MOM_WARM beyond.  Each thread takes MOM_CHUNK unknowns and starts its
-// recurrence MOM_WARM unknowns early from zero (or at the true start): both
-// recurrences contract by cp ≈ 0.268 per unknown, so the dropped history is
-// ~1e-37 of the values.
-__device__ inline double mom_cp(int q) {
-    double cp = 0.25;
-    const int lim = q < MOM_WARM ? q : MOM_WARM;
-    for (int i = 1; i <= lim; ++i) cp = 1.0 / (4.0 - cp);
-    return cp;
-}
-// forward: d_q = (6 y_{q+1} − [q = 0] y_0 − [q = mm−1] y_{n−1} − d_{q−1}) / (4 − cp_{q−1}), into work
-__global__ void __launch_bounds__(256) k_moment_prefilter_fwd(MomTab T, double* work) {
-    const int mm = T.n - 2;
-    const int nchunk = (mm + MOM_CHUNK - 1) / MOM_CHUNK;
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= nchunk * T.order) return;
-    const int m = g / nchunk, ch = g % nchunk;
-    const double* y = T.coef + (size_t)m * (T.n + 2) + 1;  // node values
-    double* d = work + (size_t)m * mm;
-    const int q0 = ch * MOM_CHUNK, q1 = q0 + MOM_CHUNK < mm ? q0 + MOM_CHUNK : mm;
-    const int qs = q0 - MOM_WARM > 0 ? q0 - MOM_WARM : 0;
-    double dp = 0.0;
-    double cpm = qs > 0 ? mom_cp(qs - 1) : 0.25;  // cp_{q−1}
-    for (int q = qs; q < q1; ++q) {
-        double r = 6.0 * y[q + 1];
-        if (q == 0) r -= y[0];
-        if (q == mm - 1) r -= y[T.n - 1];
-        double v;
-        if (q == 0) {
-            v = r / 4.0;
-        } else {
-            const double den = 4.0 - cpm;
-            v = (r - dp) / den;
-            if (q <= MOM_WARM) cpm = 1.0 / den;
+// (d_q = (r_q − d_{q−1}) cp_q, cp_q = 1/(4 − cp_{q−1}), cp_0 = 1/4, r_q = 6 y_{q+1} −
+// [q = 0] y_0 − [q = mm−1] y_{n−1}, then c_{q+2} = d_q − cp_q c_{q+3}).  The unknowns
+// are c[2..n−1] (q = 0..mm−1 = n−3); c[1] = y_0 and c[n] = y_{n−1}.  cp_q is bitwise
+// constant from q ≈ 20 on.
+// A block brings its node values into LDS in whole lines; a lane takes MOM_CHUNK
+// unknowns and starts its recurrence MOM_WARM of them early from zero (or at the true
+// start), forward in the block's values, backward in its d.  One double of padding
+// after every 32 keeps the lanes' strides off one bank.
+// What bounds it is the chain of 160 steps, 300 blocks at 400 000 nodes x 3.  As two
+// kernels of one lane per 128 unknowns straight from memory, every load and store a
+// line of its own, it was 79 + 198 us; it is 27.
+__global__ void __launch_bounds__(MOM_LANES) k_moment_prefilter(MomTab T, const double* yall) {
+    constexpr int NV = MOM_LANES * MOM_CHUNK;
+    __shared__ double v[(MOM_WARM + NV) / 32 * 33 + 33], cps[MOM_WARM];
+    auto at = [](int i) { return i + (i >> 5); };
+    const int mm = T.n - 2, tid = threadIdx.x, m = blockIdx.y;
+    const int Q0 = blockIdx.x * MOM_TILE;          // the block's first unknown
+    const double* y = yall + (size_t)m * T.n;
+    double* c = T.coef + (size_t)m * (T.n + 2);
+    // v[i]: r of unknown Q0 − MOM_WARM + i
+    for (int i = tid; i < MOM_WARM + NV; i += MOM_LANES) {
+        const int q = Q0 - MOM_WARM + i;
+        double r = 0.0;
+        if (q >= 0 && q < mm) {
+            r = 6.0 * y[q + 1];
+            if (q == 0) r -= y[0];
+            if (q == mm - 1) r -= y[T.n - 1];
         }
-        if (q >= q0) d[q] = v;
-        dp = v;
+        v[at(i)] = r;
     }
-}
-// backward: c_{q+2} = d_q − cp_q c_{q+3}, then the two padding coefficients
-__global__ void __launch_bounds__(256) k_moment_prefilter_bwd(MomTab T, const double* work) {
-    const int mm = T.n - 2;
-    const int nchunk = (mm + MOM_CHUNK - 1) / MOM_CHUNK;
-    const int g = blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= nchunk * T.order) return;
-    const int m = g / nchunk, ch = g % nchunk;
-    double* c = T.coef + (size_t)m * (T.n + 2);
-    const double* d = work + (size_t)m * mm;
-    const int q0 = ch * MOM_CHUNK, q1 = q0 + MOM_CHUNK < mm ? q0 + MOM_CHUNK : mm;
-    const int qe = q1 + MOM_WARM < mm ? q1 + MOM_WARM : mm;
-    double xn = 0.0;  // c_{q+3}
-    const double cpw = mom_cp(MOM_WARM);
-    for (int q = qe - 1; q >= q0; --q) {
-        const double v = q == mm - 1 ? d[q] : d[q] - (q < MOM_WARM ? mom_cp(q) : cpw) * xn;
-        if (q < q1) c[q + 2] = v;
-        xn = v;
+    if (tid == 0) {
+        double cp = 0.25;
+        for (int q = 0; q < MOM_WARM; ++q) {
+            cps[q] = cp;
+            cp = 1.0 / (4.0 - cp);
+        }
     }
-}
-__global__ void k_moment_prefilter_ends(MomTab T) {
-    const int m = threadIdx.x;
-    if (m >= T.order) return;
-    double* c = T.coef + (size_t)m * (T.n + 2);
-    // c[1] = y_0 and c[n] = y_{n−1} are already in place
-    c[0] = 2.0 * c[1] - c[2];
-    c[T.n + 1] = 2.0 * c[T.n] - c[T.n - 1];
+    __syncthreads();
+    auto cp = [&](int q) { return cps[q < MOM_WARM ? (q < 0 ? 0 : q) : MOM_WARM - 1]; };
+    const int q0 = Q0 + tid * MOM_CHUNK;
+    const double cpw = cps[MOM_WARM - 1];
+    const bool head = q0 < 2 * MOM_WARM;  // within reach of the first cp_q
+    double d[MOM_CHUNK], dp = 0.0;
+#pragma unroll 16
+    for (int i = 0; i < MOM_WARM; ++i) {  // before unknown 0 the r are zero and so stays d
+        const int q = q0 - MOM_WARM + i;
+        dp = (v[at(tid * MOM_CHUNK + i)] - dp) * (head ? cp(q) : cpw);
+    }
+#pragma unroll
+    for (int i = 0; i < MOM_CHUNK; ++i)
+        d[i] = dp = (v[at(tid * MOM_CHUNK + MOM_WARM + i)] - dp) * (head ? cp(q0 + i) : cpw);
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MOM_CHUNK; ++i) v[at(tid * MOM_CHUNK + i)] = d[i] = q0 + i < mm ? d[i] : 0.0;
+    __syncthreads();
+    double x = 0.0;  // past the last unknown d is zero and so stays c
+    if (tid < MOM_LANES - MOM_HALO) {
+#pragma unroll 16
+        for (int i = MOM_WARM - 1; i >= 0; --i) {
+            const int q = q0 + MOM_CHUNK + i;
+            x = v[at((tid + 1) * MOM_CHUNK + i)] - (head ? cp(q) : cpw) * x;
+        }
+#pragma unroll
+        for (int i = MOM_CHUNK - 1; i >= 0; --i) d[i] = x = d[i] - (head ? cp(q0 + i) : cpw) * x;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < MOM_CHUNK; ++i) v[at(tid * MOM_CHUNK + i)] = d[i];
+    __syncthreads();
+    const int nq = mm - Q0 < MOM_TILE ? mm - Q0 : MOM_TILE;
+    for (int i = tid; i < nq; i += MOM_LANES) c[Q0 + i + 2] = v[at(i)];
+    if (tid == 0 && Q0 == 0) {
+        c[1] = y[0];
+        c[0] = 2.0 * y[0] - v[at(0)];
+    }
+    if (tid == 0 && Q0 + nq == mm) {
+        c[T.n] = y[T.n - 1];
+        c[T.n + 1] = 2.0 * y[T.n - 1] - v[at(nq - 1)];
+    }
 }
 
 // MomentTable(x) (interpolator.jl:60-68)
@@ -4410,21 +4426,30 @@ __global__ void __launch_bounds__(256) k_filon(MomTab T, const double* f, const 
 }
 
 // Σ_i Filon over (t_i, t_{i+1}) for each k (the loop form, integrator.jl:20-38):
-// one wavefront per k, lane l takes intervals l, l + 64, …, each reusing
+// one block per k, lane l takes intervals l, l + FILON_THREADS, …, each reusing
 // nothing across lanes (I(k t_i) is evaluated at both ends); the lanes' sums
-// are added in a fixed order
-__global__ void __launch_bounds__(WAVE) k_filon_sum(MomTab T, const double* t, const double* f, const double* fp,
-                                                    const double* fpp, int nt, const double* ks, double* out) {
+// are added in a fixed order.  Latency of the table reads: with one wavefront, 16
+// steps of two reads in turn, 1001 t x 700 k were 68 us; with four they are 40.
+constexpr int FILON_THREADS = 256;
+__global__ void __launch_bounds__(FILON_THREADS) k_filon_sum(MomTab T, const double* t, const double* f,
+                                                             const double* fp, const double* fpp, int nt,
+                                                             const double* ks, double* out) {
+    __shared__ double part[FILON_THREADS / WAVE];
     const double k = ks[blockIdx.x];
     double s = 0.0;
-    for (int i = threadIdx.x; i + 1 < nt; i += WAVE) {
+    for (int i = threadIdx.x; i + 1 < nt; i += FILON_THREADS) {
         double Ia[4], Ib[4];
         mom_eval(T, k * t[i + 1], Ib);
         mom_eval(T, k * t[i], Ia);
         s += mom_filon(f[i], fp[i], fpp[i], k, t[i], Ia, Ib);
     }
     s = wave_sum(s);
-    if (threadIdx.x == 0) out[blockIdx.x] = s;
+    if (threadIdx.x % WAVE == 0) part[threadIdx.x / WAVE] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < FILON_THREADS / WAVE; ++w) s += part[w];
+        out[blockIdx.x] = s;
+    }
 }
 
 // the moment functions themselves, per point: method 0 asymptotic, 1 FP64
@@ -4484,18 +4509,16 @@ int bolt_moment_table_create(bolt_ctx* ctx, int nu, int order, double x_min, dou
         return set_error(BOLT_E_NOMEM, "bolt_moment_table_create: coefficients");
     }
     Scratch<double> work;
-    if (work.alloc((size_t)order * (n - 2)) != hipSuccess) {
+    if (work.alloc((size_t)order * n) != hipSuccess) {
         (void)hipFree(T.coef);
         (void)hipStreamDestroy(tab->stream);
         return set_error(BOLT_E_NOMEM, "bolt_moment_table_create: work space");
     }
     hipStream_t st = tab->stream;
     const int nb = std::min((n + 255) / 256, 65536);
-    hipLaunchKernelGGL(k_moment_nodes, dim3(nb), dim3(256), 0, st, T);
-    const int nth = ((n - 2 + MOM_CHUNK - 1) / MOM_CHUNK) * order;
-    hipLaunchKernelGGL(k_moment_prefilter_fwd, dim3((nth + 255) / 256), dim3(256), 0, st, T, work.p);
-    hipLaunchKernelGGL(k_moment_prefilter_bwd, dim3((nth + 255) / 256), dim3(256), 0, st, T, (const double*)work.p);
-    hipLaunchKernelGGL(k_moment_prefilter_ends, dim3(1), dim3(WAVE), 0, st, T);
+    hipLaunchKernelGGL(k_moment_nodes, dim3(nb, order), dim3(256), 0, st, T, work.p);
+    hipLaunchKernelGGL(k_moment_prefilter, dim3((n - 2 + MOM_TILE - 1) / MOM_TILE, order), dim3(MOM_LANES), 0, st, T,
+                       (const double*)work.p);
     const hipError_t e1 = hipGetLastError(), e2 = hipStreamSynchronize(st);
     if (e1 != hipSuccess || e2 != hipSuccess) {
         (void)hipFree(T.coef);
@@ -4575,7 +4598,7 @@ int bolt_filon_sum(bolt_moment_table* tab, const double* t, const double* f, con
     HIPCHK(dt.up(t, nt, st)); HIPCHK(df.up(f, nt, st)); HIPCHK(dfp.up(fp, nt, st)); HIPCHK(dfpp.up(fpp, nt, st));
     HIPCHK(dk.up(k, nk, st));
     HIPCHK(dout.alloc(nk));
-    hipLaunchKernelGGL(k_filon_sum, dim3(nk), dim3(WAVE), 0, st, tab->T, (const double*)dt.p, (const double*)df.p,
+    hipLaunchKernelGGL(k_filon_sum, dim3(nk), dim3(FILON_THREADS), 0, st, tab->T, (const double*)dt.p, (const double*)df.p,
                        (const double*)dfp.p, (const double*)dfpp.p, nt, (const double*)dk.p, dout.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(out, dout.p, sizeof(double) * nk, hipMemcpyDeviceToHost, st));
