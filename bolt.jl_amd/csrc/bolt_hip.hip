@@ -260,7 +260,7 @@ __global__ void k_plin_post(const CosmoDev* cosmos, const CfgDev* cfgs, const Mo
 // recurrence's growing solution has taken over).
 // One block per dense-k midpoint at a time; lanes own x nodes (slots of 64
 // consecutive nodes); ℓ runs in chunks of 16 reduced across the lanes in registers
-// and, every LOS_SPAN multipoles, across the wavefronts through LDS.
+// and, every SPAN multipoles, across the wavefronts through LDS.
 // NS = 1: one source (C_ℓ^TT, or C_ℓ^EE with the spin factor); NS = 2: the
 // temperature and polarization sources share each j_ℓ and give TT, TE, EE.
 #define LOS_SLOTS 16   // x slots of 64 nodes (up to 1024 nodes after x = -8)
@@ -268,8 +268,11 @@ __global__ void k_plin_post(const CosmoDev* cosmos, const CfgDev* cfgs, const Mo
 // b + 2·grid, ... (a spread over k, so blocks cost about the same) and sums
 // their C_ℓ contributions into a row of its own.  Fixed, so that the
 // summation order, and with it every bit of C_ℓ, does not depend on the device
-#define LOS_GRID 512
-#define LOS_SPAN 128       // multipoles between two exchanges of a block's wavefronts
+// Three blocks a CU, which is what k_los<1, 4>'s registers leave room for: the third
+// fills the issue slots in which the wavefronts of the other two wait for each other
+// (512 blocks at two a CU: 1.7 ms at 2500 ℓ x 4999 k against 1.3; TT/TE/EE, which has
+// room for two a CU, the same to 1 %; 1024 blocks: 1.5).
+#define LOS_GRID 768
 #define LOS_SPW_DEFAULT 4  // x slots per wavefront (LOS_SLOTS/SPW wavefronts per block): 1, 2 or 4
 #define LOS_TAU 1e-7
 // lanes with z < LOS_ZS take j_ℓ from its ascending series
@@ -564,29 +567,30 @@ __device__ __attribute__((noinline)) double los_pw(double A_s, double n_s, doubl
 // T_ℓ(k) = Σ_x j_ℓ(k(η₀−η)) S(x, k) Δx for every requested ℓ, and the
 // C_ℓ contributions T_ℓ² P(k) Δk/k summed over the block's midpoints.
 // A block of LOS_SLOTS/SPW wavefronts; wavefront w owns x slots w, w + W, ...
-// (SPW of them).  Each wavefront runs LOS_SPAN multipoles on its own, chunk by
+// (SPW of them).  Each wavefront runs SPAN multipoles on its own, chunk by
 // chunk, its partial T_ℓ kept in LDS; then the block adds its wavefronts' partials
 // and the row entries (entry ℓ is always read and written by the same thread).
 // What bounds it: FP64 issue.  2500 ℓ x 4999 k x 799 x are 5.7e7 wavefront steps, of
 // three instructions where nothing can be cut (los_below, 70 % of them), four up to
 // the turning point and a dozen past it.  With the cut tested in every step (20
 // instructions) and a reduction through LDS with two barriers every 16 ℓ it was
-// 5.9 ms (9.0e8 VALU instructions); it is 1.77 ms (4.7e8, of which the reductions
-// are a fifth), 56 % of the VALU's issue slots; the rest is the wavefronts' unequal
-// shares between two exchanges (13 slots over 4).  TT, TE and EE of 1499 ℓ x 3000 k:
-// 4.0 -> 1.2 ms.
+// 5.9 ms (9.0e8 VALU instructions); it is 1.3 ms (4.7e8, of which the reductions
+// are a fifth), three quarters of the VALU's issue slots; the rest is the wavefronts'
+// unequal shares between two exchanges (13 slots over 4).  TT, TE and EE of 1499 ℓ x
+// 3000 k: 4.0 -> 1.2 ms.
 // SPW: four slots a wavefront share one reduction and four independent chains; two
-// take 25 % more instructions at twice the wavefronts, the same 1.8 ms for NS = 1
-// and 1.3 times as long for NS = 2, so four is the default.
+// take 25 % more instructions, the same time for NS = 1 and 1.2 times as long for
+// NS = 2, so four is the default.
 template <int NS, int SPW>
-__global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 && NS == 1) ? 4 : 2) k_los(LosArgs A) {
+__global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 && NS == 1) ? 4 : NS == 1 ? 3 : 2) k_los(LosArgs A) {
     constexpr int CH = 16;  // ℓ per chunk (NA·CH accumulators per lane)
     constexpr int NW = LOS_SLOTS / SPW;
+    constexpr int SPAN = SPW == 4 ? 256 : 128;  // multipoles between two exchanges of the block's wavefronts
     constexpr int NA = NS == 1 ? 1 : 2;                    // accumulator sets
     constexpr int NOUT = NS == 1 ? 1 : (NS == 2 ? 3 : 2);  // partial-row outputs
     const int lane = threadIdx.x & (WAVE - 1);
     const int wv = threadIdx.x / WAVE;
-    __shared__ double part[2][NW][NA][LOS_SPAN];  // by turns, so that one barrier a span is enough
+    __shared__ double part[2][NW][NA][SPAN];  // by turns, so that one barrier a span is enough
     __shared__ int plive[2][NW];
     int turn = 0;
     __shared__ double nsum[NW];
@@ -693,23 +697,23 @@ __global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 
             }
             return live;
         };
-        // Thread i < len owns ℓ = span + i.  What it adds to is read before the span's
+        // Thread i < SPAN owns ℓ = span + i.  What it adds to is read before the span's
         // recurrences: read after them, 20 spans x 10 midpoints waited for it in turn.
         const int li = threadIdx.x;
         int u = -1;
         double r0 = 0.0, r1 = 0.0, r2 = 0.0;
-        auto fetch = [&](int span, int len) {
+        auto fetch = [&](int span) {
             const int l = span + li;
-            u = li < len && l <= A.lmax ? A.lidx[l] : -1;
+            u = li < SPAN && l <= A.lmax ? A.lidx[l] : -1;
             if (u >= 0 && !first) {
                 r0 = row[u];
                 if (NOUT >= 2) r1 = row[A.nu + u];
                 if (NOUT >= 3) r2 = row[2 * A.nu + u];
             }
         };
-        // the wavefronts' sums of ℓ = span .. span+len-1 to the block's row; false
+        // the wavefronts' sums of ℓ = span .. span+SPAN-1 to the block's row; false
         // when every term was past its cut
-        auto exchange = [&](int span, int len, int live) {
+        auto exchange = [&](int span, int live) {
             if (lane == 0) plive[turn][own] = live;
             __syncthreads();
             int live_block = plive[turn][0];
@@ -740,10 +744,10 @@ __global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 
                 }
             }
             // the remaining T_ℓ are zero, so the block's first midpoint stores
-            // zeros for them (from LOS_LEAN on thread i owns ℓ ≡ LOS_LEAN + i mod
-            // LOS_SPAN) and later midpoints add nothing
-            if (!live_block && first && li < LOS_SPAN)
-                for (int l2 = span + len + li; l2 <= A.lmax; l2 += LOS_SPAN) {
+            // zeros for them (same thread ownership) and later midpoints add
+            // nothing
+            if (!live_block && first && li < SPAN)
+                for (int l2 = span + SPAN + li; l2 <= A.lmax; l2 += SPAN) {
                     const int u2 = A.lidx[l2];
                     if (u2 < 0) continue;
                     for (int o = 0; o < NOUT; ++o) row[o * A.nu + u2] = 0.0;
@@ -751,18 +755,18 @@ __global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 
             turn ^= 1;
             return live_block != 0;
         };
-        fetch(0, LOS_LEAN);
-        int live = chunk(0, 0, std::integral_constant<int, 0>{});
-        for (int L0 = CH; L0 < LOS_LEAN && L0 <= A.lmax; L0 += CH)
-            live |= chunk(L0, L0, std::integral_constant<int, 1>{});
-        if (exchange(0, LOS_LEAN, live))
-            for (int span = LOS_LEAN; span <= A.lmax; span += LOS_SPAN) {
-                live = 0;
-                fetch(span, LOS_SPAN);
-                for (int L0 = span; L0 < span + LOS_SPAN && L0 <= A.lmax; L0 += CH)
-                    live |= chunk(L0, L0 - span, std::integral_constant<int, 2>{});
-                if (!exchange(span, LOS_SPAN, live)) break;
+        for (int span = 0; span <= A.lmax; span += SPAN) {
+            int live = 0, L0 = span;
+            fetch(span);
+            if (span == 0) {
+                live = chunk(0, 0, std::integral_constant<int, 0>{});
+                for (L0 = CH; L0 < LOS_LEAN && L0 <= A.lmax; L0 += CH)
+                    live |= chunk(L0, L0, std::integral_constant<int, 1>{});
             }
+            for (; L0 < span + SPAN && L0 <= A.lmax; L0 += CH)
+                live |= chunk(L0, L0 - span, std::integral_constant<int, 2>{});
+            if (!exchange(span, live)) break;
+        }
         if (A.steps) {
             const double ns = (double)nstep;
             if (lane == 0) nsum[wv] = ns;
