@@ -63,7 +63,7 @@ def measured_traffic(kernel, per_launch=1):
     committed rocprofv3 summary (FETCH_SIZE and WRITE_SIZE, scaled by a plain
     copy of known size), or None where that shape was not measured."""
     import re
-    path = os.path.join(ROOT, "profiles", "k_boltsolve_cmb_full.md")
+    path = os.path.join(ROOT, "profiles", "k_solve_cmb_full.md")
     if not os.path.exists(path):
         return None
     key = kernel if per_launch == 1 else f"{kernel}_x{per_launch}"
@@ -862,8 +862,8 @@ def main():
     los_tf = f_los_nominal / (ms_los * 1e-3) / 1e12
     los_tf_exec = 4.0 * los_exec / (ms_los * 1e-3) / 1e12
     if ms_ode >= ms_los:
-        roof = {"kernel": "k_boltsolve", "bound": "fp64-vector", "achieved": ode_tf, "peak": PEAK_FP64,
-                "unit": "TFLOP/s", "frac": ode_tf / PEAK_FP64, "traffic": measured_traffic("k_boltsolve", B),
+        roof = {"kernel": "k_solve", "bound": "fp64-vector", "achieved": ode_tf, "peak": PEAK_FP64,
+                "unit": "TFLOP/s", "frac": ode_tf / PEAK_FP64, "traffic": measured_traffic("k_solve", B),
                 "chip_level_tflops": f_ode / B / dt / 1e12,
                 "note": "FP64 vector peak (no MFMA instruction is used); algorithmic flops of the structured "
                         "ESDIRK solve per step/RHS/node, from the kernel's own step counters, for one launch "
@@ -886,7 +886,7 @@ def main():
         "per_launch": B,
         "latency_ms": {"mean": float(np.mean(lat)), "max": float(np.max(lat)),
                        "note": "wall time of one batch of per_launch spectra on its lane"},
-        "kernels_ms": {"k_boltsolve": ms_ode, "k_los": ms_los},
+        "kernels_ms": {"k_solve": ms_ode, "k_los": ms_los},
         "ode_steps_total": steps_total,
         "los": {"nominal_tflops": los_tf, "executed_tflops": los_tf_exec, "executed_steps": los_exec,
                 "nominal_steps": f_los_nominal / 4.0},
