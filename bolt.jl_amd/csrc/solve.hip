@@ -992,6 +992,10 @@ __global__ void __launch_bounds__(NTHR) k_solve(SolveArgs A) {
                 en = sqrt(tot / n);
             }
             if (!isfinite(en)) {
+                // the forward scans carried the non-finite values into rows n.. of the
+                // two vectors that wavefront 0 solves in place, where the backward
+                // scans of the next, shorter step begin: zero again
+                for (int c = n + T.tid; c < WS_::ns; c += NTHR) W.w()[c] = W.arg()[c] = 0.0;
                 ++nrej;
                 h *= 0.2;
                 if (h < 1e-14) status = BOLT_MODE_NONFINITE;
