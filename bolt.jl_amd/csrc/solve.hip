@@ -661,8 +661,9 @@ __global__ void __launch_bounds__(NTHR) k_solve(SolveArgs A) {
         for (int c = T.tid; c < n; c += NTHR) W.place()[c] = (unsigned short)chain_to_state(G, c);
         initial_conditions(C, G, W, k, W.u(0), T);
         __syncthreads();
-        // the outputs at the starting point take the initial condition as saved
-        for (int c = T.tid; c < n; c += NTHR) W.u(1)[c] = W.u(0)[c];
+        // the outputs at the starting point take the initial condition as saved (f(1)
+        // with a weight of zero)
+        for (int c = T.tid; c < n; c += NTHR) { W.u(1)[c] = W.u(0)[c]; W.f(1)[c] = 0.0; }
         __syncthreads();
         // owned rows; a row past n is clamped for its loads and never stored
         int rc[NR], rm[NR], rp[NR];
