@@ -678,7 +678,8 @@ __global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 
                         }
                     }
                     if (q.n == 0 || decltype(sl)::value < nb) return;
-                    if (FORM == 2 || los_none(q.iz > 1.0 / LOS_ZL))
+                    // 1/z outside [0, 1/LOS_ZL]; z < 0 (η > η₀) takes the series
+                    if (FORM == 2 || los_none(fabs(q.iz - 0.5 / LOS_ZL) > 0.5 / LOS_ZL))
                         los_slot_turn<NS, CH, I0>(q, L0, acc, accp, nstep);
                     else if (los_any(q.iz != 0.0 && q.z < LOS_ZS))
                         los_slot<NS, CH, I0, true>(q, L0, acc, accp, nstep);

@@ -97,3 +97,23 @@ def test_spline_sum_where_eta_does_not_grow():
     got = boltmi.cl_on_grid(ells, T, P, dense, par, bg, bessel_mode=1)
     for g, r in zip(got, o.cl(T.grid, P.grid, T.k_grid, dense, ells, 1, nthreads=8)):
         np.testing.assert_allclose(g, r, rtol=1e-9, atol=1e-9 * np.max(np.abs(r)))
+
+
+# |z| = k (η − η₀) <= 0.02 at the one node beyond η₀, where the oracle's j₀ and j₁ are exact
+# to rounding; all other nodes at this x have z > 30 from k = 0.004 on
+@pytest.mark.parametrize("spw", ["1", "2", "4"])
+@pytest.mark.parametrize("node", [1201, 1250, 1500])
+def test_exact_sum_where_eta_passes_eta0(node, spw, monkeypatch):
+    """tables in which η(x) exceeds η₀ at a node among others with large z: its
+    argument is negative, and j_ℓ(−z) = (−1)^ℓ j_ℓ(z)"""
+    monkeypatch.setenv("BOLT_LOS_SPW", spw)
+    par, bg, T, P, dense = setting(799)
+    eta = bg.coef[_abi.T_ETA]  # node j has coefficients j, j + 1, j + 2 with weights 1/6, 2/3, 1/6
+    eta[node + 1] += 1.5 * (bg.eta0 + 0.05 - (eta[node] + 4.0 * eta[node + 1] + eta[node + 2]) / 6.0)
+    ells = np.array([2, 3, 10, 30, 47, 48, 63, 64, 100, 300, 700])
+    o = pyoracle.Oracle(par.as_tuple(), bg.tables_dict())
+    assert [i for i, x in enumerate(bg.x_grid) if o.spline(_abi.T_ETA, x) > bg.eta0] == [node]
+    ctx = boltmi.Context(0)
+    got = boltmi.cl_on_grid(ells, T, P, dense, par, bg, ctx=ctx)
+    for g, r in zip(got, o.cl(T.grid, P.grid, T.k_grid, dense, ells, 0, nthreads=8)):
+        np.testing.assert_allclose(g, r, rtol=1e-6, atol=1e-9 * np.max(np.abs(r)))
