@@ -3384,7 +3384,11 @@ constexpr int QS_RCAP = 256;         // requests published and not yet done
 constexpr double QS_IDLE_US = 2e6;    // ~2 s without work before a workgroup leaves on its own
 constexpr double QS_DRAIN_MS = 5.0;    // the launcher drains a launch after this long with no request in the server
 constexpr int QS_XCD = 8;           // MI355X: 8 XCDs, each with its own L2
-constexpr int QS_POLL_SLEEPS = 4;
+// Polls of a workgroup without work, every 3.4 µs x this.  They delay the scratch
+// accesses of the workgroups at work (k_solve's two-pass layouts spill): with 4, 10
+// modes of n = 473 took 104 to 179 ms beside 214 idle workgroups (93 with 16, the same
+// as alone) and of n = 464 with 48 bins 52 to 79 (33.5); 8, 16, 32 and 64 are alike.
+constexpr int QS_POLL_SLEEPS = 16;
 constexpr size_t QS_ALIGN = 256;
 }  // namespace
 

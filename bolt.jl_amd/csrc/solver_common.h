@@ -1576,7 +1576,7 @@ struct SolveArgs {
     int serve = 0;
     int epoch = 0;
     int idle_limit = 0;
-    int poll_sleeps = 4;  // s_sleep 127 (~3.4 µs each) between polls
+    int poll_sleeps = 16;  // s_sleep 127 (~3.4 µs each) between polls
     const int* published = nullptr;
     const int* closed = nullptr;
     const int* drain = nullptr;
