@@ -3390,6 +3390,10 @@ constexpr int QS_XCD = 8;           // MI355X: 8 XCDs, each with its own L2
 // as alone) and of n = 464 with 48 bins 52 to 79 (33.5); 8, 16, 32 and 64 are alike.
 constexpr int QS_POLL_SLEEPS = 16;
 constexpr size_t QS_ALIGN = 256;
+// Layout of a launch (solve_layout.h): up to 512 rows and 16 momentum bins, unless a
+// request needs the one of any size, which is slower for all (10 modes of n = 323: 90
+// against 81 ms, n = 473: 93 against 81, n = 197: 85 against 77).
+constexpr int QS_LAYOUT = 2;
 }  // namespace
 
 struct QArena {
@@ -3476,6 +3480,8 @@ struct QServer {
     int published = 0;
     int epoch = 0;          // launches so far
     bool running = false;   // a solver launch is in flight
+    int launched = QS_LAYOUT;  // its layout
+    int layout = QS_LAYOUT;    // the next launch's
     bool stopping = false;
     long long launches = 0, joined = 0, served = 0;
     std::vector<std::thread> threads;
@@ -3624,6 +3630,18 @@ static void qs_admit_loop(QServer* sv) {
                 sv->cv.wait_for(lk, std::chrono::milliseconds(2));
             }
         }
+        const CfgDev cd = to_cfgdev(&q->rq.cfg);
+        const int layout = wsn_layout(cd.n, cd.nq);
+        {
+            // a running launch whose layout does not hold the request ends first; what it
+            // leaves unclaimed goes to the next one
+            std::unique_lock<std::mutex> lk(sv->mu);
+            sv->layout = std::max(sv->layout, layout);
+            while (sv->running && sv->launched < layout) {
+                __atomic_store_n(&sv->ctl[2], sv->epoch, __ATOMIC_RELEASE);
+                sv->cv.wait_for(lk, std::chrono::milliseconds(1));
+            }
+        }
         const int r = qs_publish(sv, *q);
         std::lock_guard<std::mutex> lk(sv->mu);
         if (r) {  // nothing was published for it: its positions hold no work (status stays 0, done 0)
@@ -3647,7 +3665,7 @@ static void qs_launch_loop(QServer* sv) {
     (void)hipSetDevice(sv->ctx->device);
     int claimed = 0;
     for (;;) {
-        int ep;
+        int ep, layout;
         {
             std::unique_lock<std::mutex> lk(sv->mu);
             for (;;) {
@@ -3661,6 +3679,7 @@ static void qs_launch_loop(QServer* sv) {
                         hipStreamSynchronize(sv->s_solve) == hipSuccess) {
                         __atomic_store_n(&sv->ctl[0], 0, __ATOMIC_RELEASE);
                         sv->published = 0;
+                        sv->layout = QS_LAYOUT;
                         claimed = 0;
                     }
                 }
@@ -3670,6 +3689,8 @@ static void qs_launch_loop(QServer* sv) {
             }
             ep = ++sv->epoch;
             sv->running = true;
+            sv->launched = sv->layout;
+            layout = sv->layout;
             ++sv->launches;
         }
         SolveArgs A;
@@ -3681,7 +3702,7 @@ static void qs_launch_loop(QServer* sv) {
         A.idle_limit = (int)std::max(1000.0, QS_IDLE_US / (3.4 * sv->poll_sleeps + 1.0));
         A.published = sv->ctl; A.closed = sv->ctl + 1; A.drain = sv->ctl + 2; A.leave = sv->d_leave;
         A.done = sv->done;
-        launch_solver(SR_DEFAULT, WSN_LAYOUTS - 1, false, sv->grid, sv->lds, sv->s_solve, A);
+        launch_solver(SR_DEFAULT, layout, false, sv->grid, sv->lds, sv->s_solve, A);
         bool ok = hipGetLastError() == hipSuccess;
         // wait for the launch; drain it once the server has held no request for QS_DRAIN_MS
         double idle_since = -1.0;
