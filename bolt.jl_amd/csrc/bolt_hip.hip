@@ -4456,10 +4456,12 @@ __global__ void __launch_bounds__(256) k_filon(MomTab T, const double* f, const 
 }
 
 // Σ_i Filon over (t_i, t_{i+1}) for each k (the loop form, integrator.jl:20-38):
-// one block per k, lane l takes intervals l, l + FILON_THREADS, …, each reusing
+// one block per k, lane l takes intervals l, l + blockDim.x, …, each reusing
 // nothing across lanes (I(k t_i) is evaluated at both ends); the lanes' sums
 // are added in a fixed order.  Latency of the table reads: with one wavefront, 16
-// steps of two reads in turn, 1001 t x 700 k were 68 us; with four they are 40.
+// steps of two reads in turn, 1001 t x 700 k were 68 us; with four they are 40.  Up to
+// 256 intervals take only the wavefronts that have one (20 t x 5000 k: a call with four
+// is 83 us, with one 73).
 constexpr int FILON_THREADS = 256;
 __global__ void __launch_bounds__(FILON_THREADS) k_filon_sum(MomTab T, const double* t, const double* f,
                                                              const double* fp, const double* fpp, int nt,
@@ -4467,7 +4469,7 @@ __global__ void __launch_bounds__(FILON_THREADS) k_filon_sum(MomTab T, const dou
     __shared__ double part[FILON_THREADS / WAVE];
     const double k = ks[blockIdx.x];
     double s = 0.0;
-    for (int i = threadIdx.x; i + 1 < nt; i += FILON_THREADS) {
+    for (int i = threadIdx.x; i + 1 < nt; i += blockDim.x) {
         double Ia[4], Ib[4];
         mom_eval(T, k * t[i + 1], Ib);
         mom_eval(T, k * t[i], Ia);
@@ -4477,7 +4479,7 @@ __global__ void __launch_bounds__(FILON_THREADS) k_filon_sum(MomTab T, const dou
     if (threadIdx.x % WAVE == 0) part[threadIdx.x / WAVE] = s;
     __syncthreads();
     if (threadIdx.x == 0) {
-        for (int w = 1; w < FILON_THREADS / WAVE; ++w) s += part[w];
+        for (int w = 1; w < (int)blockDim.x / WAVE; ++w) s += part[w];
         out[blockIdx.x] = s;
     }
 }
@@ -4628,7 +4630,8 @@ int bolt_filon_sum(bolt_moment_table* tab, const double* t, const double* f, con
     HIPCHK(dt.up(t, nt, st)); HIPCHK(df.up(f, nt, st)); HIPCHK(dfp.up(fp, nt, st)); HIPCHK(dfpp.up(fpp, nt, st));
     HIPCHK(dk.up(k, nk, st));
     HIPCHK(dout.alloc(nk));
-    hipLaunchKernelGGL(k_filon_sum, dim3(nk), dim3(FILON_THREADS), 0, st, tab->T, (const double*)dt.p, (const double*)df.p,
+    const int nthr = nt > FILON_THREADS ? FILON_THREADS : (nt + WAVE - 2) / WAVE * WAVE;
+    hipLaunchKernelGGL(k_filon_sum, dim3(nk), dim3(nthr), 0, st, tab->T, (const double*)dt.p, (const double*)df.p,
                        (const double*)dfp.p, (const double*)dfpp.p, nt, (const double*)dk.p, dout.p);
     HIPCHK(hipGetLastError());
     HIPCHK(hipMemcpyAsync(out, dout.p, sizeof(double) * nk, hipMemcpyDeviceToHost, st));

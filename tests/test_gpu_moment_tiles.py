@@ -31,3 +31,15 @@ def test_filon_sum_lanes(nt):
     got = boltmi.filon_sum(boltmi.sph_bessel_interpolator(*key), t, f, fp, fpp, ks)
     ref = po.MomentTable(*key).filon_sum(t, f, fp, fpp, ks)
     assert np.max(np.abs(got - ref)) < 1e-13 * max(1.0, np.max(np.abs(ref)))
+
+
+# one to four wavefronts a sum: the same 1e-13
+@pytest.mark.parametrize("nt", [3, 66, 129, 130, 193, 194])
+def test_filon_sum_of_few_intervals(nt):
+    key = (2, 3, 0.0, 300.0, 30001)
+    t = np.linspace(0.05, 12.0, nt)
+    f, fp, fpp = np.cos(0.7 * t) + 0.1 * t, -0.7 * np.sin(0.7 * t) + 0.1, -0.49 * np.cos(0.7 * t)
+    ks = np.geomspace(0.01, 30.0, 300)
+    got = boltmi.filon_sum(boltmi.sph_bessel_interpolator(*key), t, f, fp, fpp, ks)
+    ref = po.MomentTable(*key).filon_sum(t, f, fp, fpp, ks)
+    assert np.max(np.abs(got - ref)) < 1e-13 * max(1.0, np.max(np.abs(ref)))
