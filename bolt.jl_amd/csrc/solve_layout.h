@@ -64,7 +64,7 @@ struct WSN {
     static constexpr int nmax = NS - SR_MAX;  // longest state
 };
 // The layouts: up to 256 rows (one owned row per thread; Bolt's default ℓᵧ = 8 is
-// n = 197), up to 360 (ℓᵧ = ℓ_ν = 50, ℓ_mν = 10 is 323), up to 512 (plin's defaults
+// n = 197), up to 368 (ℓᵧ = ℓ_ν = 50, ℓ_mν = 10 is 323), up to 512 (plin's defaults
 // are 473), and any hierarchy LDS can hold.  The strides spread the LU lanes'
 // rows (stage points 3·NS apart) over the banks.
 using WSN0 = WSN<278, 16>;

@@ -1,6 +1,7 @@
 """The line-of-sight sum at the edges of its splits: x nodes per slot of 64 lanes and
 slots per wavefront, chunks of 16 multipoles, the change to the short recurrence at
-ℓ = 64, and the spans of 128 multipoles between two exchanges of a block."""
+ℓ = 64, and the spans between two exchanges of a block (256 multipoles with 4 slots a
+wavefront, 128 with 1 or 2)."""
 import numpy as np
 import pytest
 
@@ -58,6 +59,29 @@ def test_last_multipole_does_not_matter():
         np.testing.assert_array_equal(boltmi.cltt_on_grid(np.arange(2, lmax + 1), T, dense, par, bg), tt[:lmax - 1])
 
 
+@pytest.mark.parametrize("spw", ["1", "2", "4"])
+def test_last_multipole_at_the_end_of_a_span(spw, monkeypatch):
+    """the same with the last ℓ at the ends of the spans of 128 and 256, and the values
+    there against the oracle (tolerances as above)"""
+    monkeypatch.setenv("BOLT_LOS_SPW", spw)
+    par, bg, T, P, dense = setting(320)
+    ctx = boltmi.Context(0)
+    full = boltmi.cl_on_grid(np.arange(2, 531), T, P, dense, par, bg, ctx=ctx)
+    tt = boltmi.cltt_on_grid(np.arange(2, 531), T, dense, par, bg, ctx=ctx)
+    last = [126, 127, 128, 129, 254, 255, 256, 257, 511, 512, 513]
+    for lmax in last:
+        part = boltmi.cl_on_grid(np.arange(2, lmax + 1), T, P, dense, par, bg, ctx=ctx)
+        for g, r in zip(part, full):
+            np.testing.assert_array_equal(g, r[:lmax - 1])
+        np.testing.assert_array_equal(boltmi.cltt_on_grid(np.arange(2, lmax + 1), T, dense, par, bg, ctx=ctx),
+                                      tt[:lmax - 1])
+    o = pyoracle.Oracle(par.as_tuple(), bg.tables_dict())
+    ells = np.array([2] + last)
+    for g, r in zip(full, o.cl(T.grid, P.grid, T.k_grid, dense, ells, 0, nthreads=8)):
+        np.testing.assert_allclose(g[ells - 2], r, rtol=1e-6, atol=1e-9 * np.max(np.abs(r)))
+    np.testing.assert_allclose(tt, full[0], rtol=1e-13)
+
+
 # Both sides sum the same spline terms in 64 bits: 1e-9, as the other comparison with
 # the oracle's spline mode.
 @pytest.mark.parametrize("nxi,nkd,ells", [
@@ -66,9 +90,9 @@ def test_last_multipole_does_not_matter():
     (65, 18, list(range(2, 19))),          # a midpoint and a column more
     (320, 65, list(range(0, 34)) + [700]),  # ℓ = 0 and 1, repeated and far ℓ
     (1024, 520, [2, 15, 16, 900, 1500, 15]),
-    (320, 161, list(range(2, 513))),       # one column short of the wide groups
-    (320, 161, list(range(2, 514))),       # the first wide call
-    (256, 161, list(range(2, 700))),       # a partial wide group
+    (320, 161, list(range(2, 513))),       # one column short of a block's last 64
+    (320, 161, list(range(2, 514))),       # exactly full
+    (256, 161, list(range(2, 700))),       # a partial last block
     (320, 6200, [2, 37, 1100]),            # more midpoints than are kept at once
 ])
 def test_spline_sum_against_oracle(nxi, nkd, ells):

@@ -1,4 +1,4 @@
-"""The FP64 solver at the edges of its layouts: 256, 360 and 512 rows (one or two
+"""The FP64 solver at the edges of its layouts: 256, 368 and 512 rows (one or two
 owned rows per thread, the vectors' strides), 384 rows (one or two scan passes)
 and 16 momentum bins, each side of the line, and the longest state.  States at
 five x against the oracle at the parity tests' 1e-6, with its step counts; a
@@ -46,3 +46,8 @@ def test_layout_edges_match_oracle(n):
 def test_momentum_bins_at_the_layout_line_match_oracle(nq):
     sizes = (12, 12, 8, nq)
     _check(2 * 12 + 12 + 9 * nq + 8, sizes)
+
+
+@pytest.mark.parametrize("ell_nu", [75, 76])
+def test_second_layouts_last_row_matches_oracle(ell_nu):
+    _check(293 + ell_nu, (60, ell_nu, 10, 15))

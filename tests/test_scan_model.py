@@ -1,5 +1,5 @@
-"""A CPU model of the solver's substitution by wavefront affine scans
-(bolt.jl_amd/csrc/bolt_hip.hip: wave_subst, pass_scan, affine_scan), with the
+"""A CPU model of the FP32 and tangent solves' substitution by wavefront affine scans
+(bolt.jl_amd/csrc/solver_common.h: wave_subst, pass_scan, affine_scan), with the
 kernel's DPP controls and row masks (row_shr 1, 2, 4, 8; row_bcast 15 to rows
 1 and 3; row_bcast 31 to rows 2 and 3; wave_shr 1; invalid sources keep the
 old value, the identity map), its SR rows per lane, its passes of 64·SR rows,
