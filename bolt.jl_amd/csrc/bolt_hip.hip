@@ -615,8 +615,8 @@ __global__ void __launch_bounds__(LOS_SLOTS / SPW * WAVE, SPW == 1 || (SPW == 2 
         const double* Pa = NA == 2 ? A.SP + (size_t)ia * nx + A.i0 : nullptr;
         const double* Pb = NA == 2 ? A.SP + (size_t)(ia + 1) * nx + A.i0 : nullptr;
 
-        // the wavefronts' turns at the longest slots (the earliest x) move on with ik,
-        // differently in the two blocks of a CU
+        // the wavefronts' turns at the longest slots (the earliest x) move on with ik: by
+        // three from one midpoint of a block to its next, which lies LOS_GRID further on
         const int own = (wv + (ik >> 8)) & (NW - 1);
         LosLanes<SPW> Q;
         Q.each([&](LosLane& q, auto sl) {
@@ -1239,7 +1239,7 @@ __global__ void __launch_bounds__(256) k_los_reduce(const double* partial, int n
 // (code under HIP graph capture, serving loops, harnesses that forbid
 // hipMalloc): the LOS partial rows for ℓ <= NOALLOC_MAX_L, η and Δx at the
 // integration nodes, the ℓ -> column table and the column map.  One copy per
-// GPU (a file-scope device array, 12.3 MB), held until the process ends; host
+// GPU (a file-scope device array, 18.5 MB), held until the process ends; host
 // code reaches it only through the address hipGetSymbolAddress returns.
 #define NOALLOC_MAX_L 3000
 #define NOALLOC_MAX_NELL 3001
@@ -5039,7 +5039,7 @@ __device__ inline double xe_saha_early(double z, const RfC& P) {
 
 // dopri_outputs (host_tables.cpp): explicit Dormand–Prince 5(4) with step
 // clipping onto the requested outputs zout(0..nout-1); out(i, y) receives them.
-// Returns false if 500,000 steps ran out (the solves here take ~1e4) or the
+// Returns false if 500,000 steps ran out (a cosmology attempts some 3e4) or the
 // step size fell below 1e-12 of z.
 template <int N, class F, class Z, class O>
 __device__ bool dopri(F&& f, double z0, double* y, int nout, Z&& zout, O&& out, double rtol, double atol) {

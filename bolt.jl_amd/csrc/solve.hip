@@ -25,9 +25,9 @@
 //  - a phase's uniform scalars are one LDS access per wavefront (StageSc), not
 //    one broadcast read each.
 // Measured (one MI355X, against the same solve with its vectors and recipes in LDS
-// and runtime strides): one mode, n = 197, k = 0.2: 59k to 43.7k cycles a step;
-// source_grid of 100 modes, n = 197: 60.9 to 39.1 ms; P(k) of 200 modes, n = 473:
-// 103 to 74.5 ms; 800 modes, n = 323, with C_l: 104.4 to 67.3 ms.
+// and runtime strides; 10 or 200 modes up to k = 0.25 alike, since the largest k's
+// chain is what counts): source grids of n = 197 88.2 to 57.7 ms, of n = 323 87.3 to
+// 65.6; P(k) at n = 473, two scan passes with 96 registers spilled, 95.3 to 80.5.
 
 #include "solve_layout.h"
 

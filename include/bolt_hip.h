@@ -298,7 +298,9 @@ int bolt_source_grid_tp_dev(bolt_ctx* ctx, int cosmo_id, const bolt_hier_cfg* cf
 
 /* cltt(ℓ, sf, kgrid, par, bg) for a list of ℓ (spectra.jl:84-96, 132-150).
  * S: [nk_src][nx] source grid on k_src; kgrid: the dense k grid (nkd nodes, the
- * sum runs over its nkd-1 midpoints); bessel_mode 0 = j_ℓ by recurrence. */
+ * sum runs over its nkd-1 midpoints); bessel_mode 0 = j_ℓ by recurrence, 1 =
+ * Bolt's spline of it, for which the context keeps device memory from the first
+ * such call on: up to 246 MB per source and 80 kB per distinct ℓ. */
 int bolt_cltt(bolt_ctx* ctx, int cosmo_id, const double* S, const double* k_src, int nk_src,
               const double* kgrid, int nkd, const int* ells, int nell, int bessel_mode,
               double* cl);
@@ -313,7 +315,7 @@ int bolt_cltt_dev(bolt_ctx* ctx, int cosmo_id, const double* d_S, const double* 
  * that cannot allocate: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments and results, bit for bit,
  * as bolt_cltt_dev; the LOS work space is a library-owned device array of
- * 12.3 MB per GPU (held until the process ends), so ℓ <= 3000 and at most 3001
+ * 18.5 MB per GPU (held until the process ends), so ℓ <= 3000 and at most 3001
  * entries in ells; larger requests return BOLT_E_ARG.  Calls that overlap on
  * one GPU (from different contexts) share that array and race. */
 int bolt_cltt_dev_noalloc(bolt_ctx* ctx, int cosmo_id, const double* d_S, const double* d_k_src, int nk_src,
